@@ -37,10 +37,10 @@ struct PauliDev {
   void* terms = nullptr;
   void* flat = nullptr;    // DPTermF per term in the caller's order
   void* groups = nullptr;  // DPGroup per flip mask (sparse form only)
-  void* tpasses[2] = {nullptr, nullptr};
   void* tgroups[2] = {nullptr, nullptr};
   void* tterms[2] = {nullptr, nullptr};
   void* truns[2] = {nullptr, nullptr};
+  void* tchunks[2] = {nullptr, nullptr};
   // compiled tile passes (per dtype): modules and one kernel per pass
   std::vector<void*> jmods[2], jfns[2];
 };
@@ -59,6 +59,9 @@ struct PauliTileSched {
   std::vector<DPPass> passes;
   std::vector<DPGroupT> groups;
   std::vector<DPTermT> terms;
+  std::vector<DPChunk> chunks;     // k_pauli_tile's form of the same terms
+  std::vector<DPGroupS> sgroups;
+  std::vector<DPTermS> sterms;
   std::vector<uint32_t> runoff;
   std::vector<int> legacy;         // flip groups wider than a tile
   std::vector<int> legacy_slot0;
@@ -317,11 +320,11 @@ int ensure_pauli(tcm_pauli* H, int dt, PauliDev** out) {
     if (int rc = upload(H->flat, &pd.flat)) return rc;
   }
   const PauliTileSched& S = H->ts[dt];
-  if (S.ok && !pd.tpasses[dt]) {
-    int rc = upload(S.passes, &pd.tpasses[dt]);
-    rc = rc ? rc : upload(S.groups, &pd.tgroups[dt]);
-    rc = rc ? rc : upload(S.terms, &pd.tterms[dt]);
+  if (S.ok && !pd.tchunks[dt]) {
+    int rc = upload(S.sgroups, &pd.tgroups[dt]);
+    rc = rc ? rc : upload(S.sterms, &pd.tterms[dt]);
     rc = rc ? rc : upload(S.runoff, &pd.truns[dt]);
+    rc = rc ? rc : upload(S.chunks, &pd.tchunks[dt]);
     if (rc) return rc;
   }
   if (H->jit[dt].state == 1 && pd.jfns[dt].empty() && !H->jit[dt].chunk.empty())
@@ -338,8 +341,8 @@ int pauli_jit_build(tcm_pauli* H, int dt, double* seconds) {
   if (J.state == 1) return 0;
   if (J.state < 0) return set_error(TCM_E_UNSUPPORTED, "pass compiler failed for this Pauli sum");
   const PauliTileSched& S = H->ts[dt];
-  if (!S.ok) {
-    J.state = 1;  // nothing tiled: the per-group kernels run
+  if (!S.ok || H->n < 10) {
+    J.state = 1;  // tiles of less than a wave: the kernels that are not compiled run
     return 0;
   }
   std::vector<std::string> bodies;
@@ -383,7 +386,8 @@ int pauli_energy_apply(tcm_pauli* H, int dt, const void* psi, void* out, const d
   }
   bool first = true;
   const bool jit = !pd->jfns[dt].empty();
-  for (size_t pi = 0; pi < S.passes.size(); ++pi) {
+  for (size_t pi = 0; pi < S.passes.size();) {
+    int np = 1;
     if (jit) {
       // parameter list of tcm_pauli_k<pi> (passgen.cpp)
       const void* a_psi = psi;
@@ -399,10 +403,14 @@ int pauli_energy_apply(tcm_pauli* H, int dt, const void* psi, void* out, const d
                                                  1u << S.passes[pi].nthr_log, 1, 1, 0, st, args, nullptr);
       if (e != hipSuccess) return set_error((int)e, "hipModuleLaunchKernel(pauli): %s", hipGetErrorString(e));
     } else {
-      launch_pauli_tile<T>(S.passes[pi], (const DPPass*)pd->tpasses[dt], (int)pi, (const DPGroupT*)pd->tgroups[dt],
-                           (const DPTermT*)pd->tterms[dt], (const uint32_t*)pd->truns[dt], psi,
-                           first ? nullptr : out, out, H->n, alpha, epart, estride, batch, energy, apply, st);
+      // passes that apply H accumulate into the same output, one after
+      // another; those that only sum energies share one launch
+      if (!apply) np = std::min<int>((int)(S.passes.size() - pi), kPauliPasses);
+      const PauliTileTables D{pd->tchunks[dt], pd->tgroups[dt], pd->tterms[dt], pd->truns[dt]};
+      launch_pauli_tile<T>(&S.passes[pi], np, D, psi, first ? nullptr : out, out, H->n, alpha, epart, estride, batch,
+                           energy, apply, st);
     }
+    pi += np;
     first = false;
   }
   for (size_t i = 0; i < S.legacy.size(); ++i) {
@@ -422,13 +430,51 @@ uint32_t pext_bits(uint64_t x, const std::vector<int>& pos) {
   return r;
 }
 
+// The pass's terms as k_pauli_tile stages them (DPTermS, DPGroupS, DPChunk).
+void pauli_sort_terms(PauliTileSched& S, DPPass& pp) {
+  pp.c0 = (int)S.chunks.size();
+  DPChunk ch{(int)S.sgroups.size(), 0, (int)S.sterms.size(), 0};
+  auto close = [&]() {
+    if (ch.nt) S.chunks.push_back(ch);
+    ch = DPChunk{(int)S.sgroups.size(), 0, (int)S.sterms.size(), 0};
+  };
+  for (int g = pp.g0; g < pp.g0 + pp.ng; ++g) {
+    const DPGroupT& G = S.groups[g];
+    std::vector<std::pair<int, DPTermS>> ts;  // (imaginary, term)
+    for (int t = G.t0; t < G.t0 + G.nt; ++t) {
+      const DPTermT& tm = S.terms[t];
+      DPTermS s{};
+      const int q = tm.ny & 3;  // (-i)^ny: 1, -i, -1, i
+      s.w = (q == 1 || q == 2) ? -tm.w : tm.w;
+      s.yz_g = tm.yz_g;
+      s.yz_t = tm.yz_t;
+      ts.push_back({q & 1, s});
+    }
+    std::stable_sort(ts.begin(), ts.end(), [](const std::pair<int, DPTermS>& a, const std::pair<int, DPTermS>& b) {
+      return a.first != b.first ? a.first < b.first : a.second.yz_t < b.second.yz_t;
+    });
+    for (size_t i = 0; i < ts.size();) {
+      if (ch.nt == kPauliChunk) close();
+      DPGroupS gs{G.flip_t, 0};
+      for (; i < ts.size() && ch.nt < kPauliChunk; ++i, ++ch.nt) {
+        gs.cnt += ts[i].first ? 0x10000u : 1u;
+        S.sterms.push_back(ts[i].second);
+      }
+      S.sgroups.push_back(gs);
+      ++ch.ng;
+    }
+  }
+  close();
+  pp.nc = (int)S.chunks.size() - pp.c0;
+}
+
 // Pack flip groups into LDS tiles: a tile = the low bits (coalescing) plus
 // the X/Y positions of the groups it evaluates, padded with the lowest free
 // bits; a group wider than a tile keeps the per-group kernel.
 void pauli_tile_sched(tcm_pauli* H, int dt) {
   PauliTileSched& S = H->ts[dt];
   const int n = H->n;
-  if (n < 10) {
+  if (n < 4) {
     S.ok = false;
     return;
   }
@@ -455,11 +501,14 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
   };
   // complex64 tiles of 12 bits (32 KiB of LDS, several blocks per CU), or of
   // 14 bits (128 KiB, one block of 1024 threads per CU) where that saves a
-  // pass: a 24-qubit sum of single X terms then takes 2 passes instead of 3
+  // pass: a 24-qubit sum of single X terms then takes 2 passes instead of 3.
+  // Not for 15 to 19 qubits, where 14-bit tiles are 2 to 32 blocks a state
+  // and leave most CUs idle (200 strings on 4 x 2^18 amplitudes, H psi: 4
+  // passes of 25 us with 14-bit tiles, 6 of 13 us with 12-bit ones).
   int k = std::min(n, dt == 0 ? 12 : 11);
   const int Lw = std::min(dt == 0 ? 4 : 3, k);
   const uint64_t lmask = (1ull << Lw) - 1;
-  if (dt == 0 && n > k) {
+  if (dt == 0 && n > k && (n <= 14 || n >= 20)) {
     const int k14 = std::min(n, 14);
     if (npasses(k14, lmask) < npasses(k, lmask)) k = k14;
   }
@@ -524,6 +573,7 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
       }
       S.groups.push_back(gt);
     }
+    pauli_sort_terms(S, pp);
     S.passes.push_back(pp);
     rem.swap(rest);
   }
@@ -904,7 +954,7 @@ int pauli_expect_prepared(const tcm_pauli* ham, int32_t dtype, const void* state
     std::lock_guard<std::mutex> lk(H->mu);
     if ((int)H->dev.size() > dev) {
       PauliDev& d = H->dev[dev];
-      const bool tables = d.terms && d.groups && (!H->ts[dtype].ok || d.tpasses[dtype]);
+      const bool tables = d.terms && d.groups && (!H->ts[dtype].ok || d.tchunks[dtype]);
       const bool kernels = !(H->jit[dtype].state == 1 && !H->jit[dtype].chunk.empty() && d.jfns[dtype].empty());
       if (tables && kernels) pd = &d;
     }
@@ -1100,7 +1150,7 @@ int tcm_pauli_free(tcm_pauli* ham) {
     if (pd.flat) (void)hipFree(pd.flat);
     if (pd.groups) (void)hipFree(pd.groups);
     for (int dt = 0; dt < 2; ++dt) {
-      void* ps[] = {pd.tpasses[dt], pd.tgroups[dt], pd.tterms[dt], pd.truns[dt]};
+      void* ps[] = {pd.tgroups[dt], pd.tterms[dt], pd.truns[dt], pd.tchunks[dt]};
       for (void* q : ps)
         if (q) (void)hipFree(q);
       for (void* m : pd.jmods[dt])

@@ -44,6 +44,7 @@ struct DPPass {
   int32_t g0, ng;      // groups of this pass
   int32_t nthr_log;    // threads per block (log2)
   int32_t slot0;       // first energy-partial slot
+  int32_t c0, nc;      // chunks of its sorted terms (the kernel that is not compiled)
   int32_t blk_bits[32];
 };
 // one Pauli term in the caller's order (per-term expectations / weighted
@@ -65,6 +66,36 @@ struct DPTermT {
   uint32_t yz_t;       // Y/Z positions inside the tile (tile-local bits)
   int32_t ny;
   double w;
+};
+// the same for k_pauli_tile: w holds the sign of (-i)^ny, `cnt` counts the
+// group's terms with a real (low half) and an imaginary (high half)
+// coefficient; terms are sorted by (group, imaginary, yz_t), so that those
+// with the same high tile bits follow each other for any thread count
+struct DPTermS {
+  double w;
+  uint64_t yz_g;
+  uint32_t yz_t, pad;
+};
+struct DPGroupS {
+  uint32_t flip_t, cnt;
+};
+// what is staged in LDS at a time: at most kPauliChunk terms (and as many
+// groups; a group of more terms is continued in the next chunk)
+struct DPChunk {
+  int32_t g0, ng, t0, nt;
+};
+constexpr int kPauliChunk = 256;
+struct PauliTileArg {
+  int32_t L, runoff0, slot0, c0, nc, pad;
+  uint64_t bmask;      // index bits outside the tile
+};
+constexpr int kPauliPasses = 16;  // passes of one launch
+struct PauliTileArgs {
+  int32_t k, nblk_log;  // the same for all passes of a schedule
+  PauliTileArg p[kPauliPasses];
+};
+struct PauliTileTables {
+  const void *chunks, *groups, *terms, *runoff;
 };
 
 // one program's pass inside a multi-program launch (passed by value)
@@ -139,9 +170,9 @@ template <typename T>
 void launch_pauli(const DPGroup& G, const DPTerm* terms_dev, int n, const void* psi, void* out, int first,
                   const double* alpha, double* epart, int64_t estride, int64_t batch, bool energy, bool apply,
                   hipStream_t st);
+// np > 1 passes (independent tiles of the same states): energies only
 template <typename T>
-void launch_pauli_tile(const DPPass& P, const DPPass* passes_dev, int pi, const DPGroupT* groups_dev,
-                       const DPTermT* terms_dev, const uint32_t* runoff_dev, const void* psi, const void* lam_in,
+void launch_pauli_tile(const DPPass* P, int np, const PauliTileTables& D, const void* psi, const void* lam_in,
                        void* lam_out, int n, const double* alpha, double* epart, int64_t estride, int64_t batch,
                        bool energy, bool apply, hipStream_t st);
 template <typename T>

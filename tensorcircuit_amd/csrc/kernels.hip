@@ -1545,84 +1545,6 @@ __global__ void __launch_bounds__(256) k_pauli(DPGroup G, const DPTerm* __restri
   }
 }
 
-// LDS-tiled Pauli pass.  For every amplitude a of the tile:
-//   h[a] = sum_groups sum_terms w i^ny (-1)^{popcount((y ^ flip) & yz)} psi[y ^ flip]
-// (the index rule of ps2coo_core, quantum.py:1461-1485), with the partner
-// read from LDS; energy += conj(psi[a]) h[a] in fp64 and, when APPLY,
-// lam_out[a] = lam_in[a] (or 0) + alpha * h[a].
-template <typename T, bool ENERGY, bool APPLY>
-__global__ void __launch_bounds__(256) k_pauli_tile(const DPPass* __restrict__ passes, int pi,
-                                                    const DPGroupT* __restrict__ groups,
-                                                    const DPTermT* __restrict__ terms,
-                                                    const uint32_t* __restrict__ runoff,
-                                                    const V2<T>* __restrict__ psi, const V2<T>* lam_in,
-                                                    V2<T>* lam_out, int64_t sstride,
-                                                    const double* __restrict__ alpha,
-                                                    double* __restrict__ epart, int64_t estride) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  V2<T>* tile = reinterpret_cast<V2<T>*>(smem);
-  const DPPass* P = passes + pi;
-  const int k = P->k, L = P->L, nbl = P->nblk_log;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const uint64_t blk = blockIdx.x & ((1ull << nbl) - 1);
-  const uint64_t b = (uint64_t)blockIdx.x >> nbl;
-  uint64_t base = 0;
-  for (int i = 0; i < nbl; ++i)
-    if ((blk >> i) & 1) base |= 1ull << P->blk_bits[i];
-  const V2<T>* s = psi + b * sstride + base;
-  const uint32_t* ro = runoff + P->runoff0;
-  const uint32_t dlo = tile_dep(ro, L, tid);
-  const uint32_t slo = swz(tid);
-  const int per = (1 << k) / nthr;
-  for (int it = 0; it < per; ++it) {
-    const uint32_t ah = it * nthr;
-    tile[swz(ah) ^ slo] = s[tile_dep(ro, L, ah) + dlo];
-  }
-  __syncthreads();
-  const double al = (APPLY && alpha) ? alpha[b] : 1.0;
-  double er = 0.0, ei = 0.0;
-  for (int it = 0; it < per; ++it) {
-    const uint32_t a = it * nthr + tid;
-    const V2<T> p = tile[swz(a)];
-    T hr = 0, hi = 0;
-    for (int g = P->g0; g < P->g0 + P->ng; ++g) {
-      const DPGroupT G = groups[g];
-      const uint32_t src = a ^ G.flip_t;
-      const V2<T> q = G.flip_t ? tile[swz(src)] : p;
-      T cr = 0, ci = 0;
-      for (int t = G.t0; t < G.t0 + G.nt; ++t) {
-        const DPTermT tm = terms[t];
-        const int par = (__popc(src & tm.yz_t) + __popcll(base & tm.yz_g)) & 1;
-        const T w = par ? (T)-tm.w : (T)tm.w;
-        switch (tm.ny & 3) {
-          case 0: cr += w; break;
-          case 1: ci += w; break;
-          case 2: cr -= w; break;
-          default: ci -= w; break;
-        }
-      }
-      hr += cr * q.x - ci * q.y;
-      hi += cr * q.y + ci * q.x;
-    }
-    if constexpr (ENERGY) {
-      er += (double)p.x * hr + (double)p.y * hi;
-      ei += (double)p.x * hi - (double)p.y * hr;
-    }
-    if constexpr (APPLY) {
-      const uint64_t off = b * sstride + base + tile_dep(ro, L, it * nthr) + dlo;
-      V2<T> o = lam_in ? lam_in[off] : mk<T>(0, 0);
-      lam_out[off] = mk<T>((T)(o.x + al * hr), (T)(o.y + al * hi));
-    }
-  }
-  if constexpr (ENERGY) {
-    block_sum2(er, ei);
-    if (threadIdx.x == 0) {
-      epart[b * estride + 2 * (P->slot0 + blk)] = er;
-      epart[b * estride + 2 * (P->slot0 + blk) + 1] = ei;
-    }
-  }
-}
-
 template <typename T>
 __global__ void __launch_bounds__(256) k_inner(const V2<T>* __restrict__ a, const V2<T>* __restrict__ c, int n,
                                                int64_t sstride, double* __restrict__ part, int64_t pstride) {
@@ -1843,34 +1765,6 @@ void launch_pauli(const DPGroup& G, const DPTerm* terms_dev, int n, const void* 
     hipLaunchKernelGGL((k_pauli<T, true, false>), grid, dim3(256), 0, st, G, terms_dev, n, p, ss, o, first, alpha, epart, estride);
   else
     hipLaunchKernelGGL((k_pauli<T, false, true>), grid, dim3(256), 0, st, G, terms_dev, n, p, ss, o, first, alpha, epart, estride);
-}
-
-template <typename T>
-void launch_pauli_tile(const DPPass& P, const DPPass* passes_dev, int pi, const DPGroupT* groups_dev,
-                       const DPTermT* terms_dev, const uint32_t* runoff_dev, const void* psi, const void* lam_in,
-                       void* lam_out, int n, const double* alpha, double* epart, int64_t estride, int64_t batch,
-                       bool energy, bool apply, hipStream_t st) {
-  const int64_t blocks = batch << P.nblk_log;
-  const size_t lds = sizeof(V2<T>) << P.k;
-  // the kernel strides over the tile with blockDim.x threads (at most 256)
-  const dim3 grid((unsigned)blocks), block(1u << std::min(P.nthr_log, 8));
-  const V2<T>* ps = (const V2<T>*)psi;
-  const V2<T>* li = (const V2<T>*)lam_in;
-  V2<T>* lo = (V2<T>*)lam_out;
-  const int64_t ss = 1ll << n;
-  if (energy && apply) {
-    ensure_lds_attr(k_pauli_tile<T, true, true>, lds);
-    hipLaunchKernelGGL((k_pauli_tile<T, true, true>), grid, block, lds, st, passes_dev, pi, groups_dev, terms_dev,
-                       runoff_dev, ps, li, lo, ss, alpha, epart, estride);
-  } else if (energy) {
-    ensure_lds_attr(k_pauli_tile<T, true, false>, lds);
-    hipLaunchKernelGGL((k_pauli_tile<T, true, false>), grid, block, lds, st, passes_dev, pi, groups_dev, terms_dev,
-                       runoff_dev, ps, li, lo, ss, alpha, epart, estride);
-  } else {
-    ensure_lds_attr(k_pauli_tile<T, false, true>, lds);
-    hipLaunchKernelGGL((k_pauli_tile<T, false, true>), grid, block, lds, st, passes_dev, pi, groups_dev, terms_dev,
-                       runoff_dev, ps, li, lo, ss, alpha, epart, estride);
-  }
 }
 
 template <typename T>
@@ -2201,9 +2095,6 @@ void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* v
                                 double*, int64_t, int64_t, bool, bool, hipStream_t);                           \
   template void launch_inner<T>(const void*, const void*, int, int64_t, int, double*, int64_t, hipStream_t); \
   template void launch_fused_fwd_multi<T>(const MultiJobs&, int64_t, int, size_t, hipStream_t);                 \
-  template void launch_pauli_tile<T>(const DPPass&, const DPPass*, int, const DPGroupT*, const DPTermT*,        \
-                                     const uint32_t*, const void*, const void*, void*, int, const double*,       \
-                                     double*, int64_t, int64_t, bool, bool, hipStream_t);                      \
   template void launch_probability<T>(const void*, void*, int64_t, hipStream_t);                               \
   template void launch_sample<T>(const void*, bool, int, int64_t, const double*, int64_t, int64_t*, double*,   \
                                  hipStream_t);                                                                 \
