@@ -29,9 +29,8 @@ HBM_PEAK_GBS = 8000.0
 # (--kernel-only eg, the timed work), FETCH scaled x2.0 and WRITE x1.0 by a
 # 4 GiB copy profiled the same way.  Key: (qubits, layers, batch, ckpt, jit, first-fit
 # scheduling).  Commands and per-counter figures:
-# profiles/tcm_adj_passes_hea24_b32.md (compiled passes, searched schedule)
-# and profiles/k_fused_adj_hea24_b32.md (generic kernels, first-fit schedule).
-MEASURED_ADJ_TRAFFIC = {(24, 20, 32, 5, 0, 1): 17046845037, (24, 20, 32, 5, 1, 0): 16715319666}
+# profiles/tcm_adj_passes_hea24_b32.md (compiled passes, searched schedule).
+MEASURED_ADJ_TRAFFIC = {(24, 20, 32, 5, 1, 0): 16715319666}
 # VALU wave-instructions per launch (rocprofv3 --pmc SQ_INSTS_VALU, mean over
 # the adjoint / forward pass launches of one sweep), same workload and key;
 # profiles/tcm_adj_passes_hea24_b32.md.
@@ -229,7 +228,7 @@ def main():
             key = (n, L, B, args.ckpt, args.jit, args.greedy)
             traffic = MEASURED_ADJ_TRAFFIC.get(key)
             valu = MEASURED_VALU_INSTS.get(key)
-        kname = "tcm_adj_k* (compiled adjoint passes)" if args.jit else "k_fused_adj"
+        kname = "tcm_adj_k* (compiled adjoint passes)" if args.jit else "k_tile_adj"
         out["roofline"] = {"bound": "hbm", "kernel": kname, "achieved": round(adj_gbs, 1),
                            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(adj_gbs / HBM_PEAK_GBS, 4),
                            "traffic": traffic,
@@ -238,7 +237,7 @@ def main():
                            "adjoint pass dispatches (profiles/tcm_adj_passes_hea24_b32.md)",
                            "bytes_per_launch": adj_bytes,
                            "avg_launch_ms": round(adj_launch_ms, 4), "launches_per_step": n_adj}
-        out["roofline_fwd"] = {"kernel": "tcm_fwd_k* (compiled forward passes)" if args.jit else "k_fused_fwd",
+        out["roofline_fwd"] = {"kernel": "tcm_fwd_k* (compiled forward passes)" if args.jit else "k_tile_fwd",
                                "achieved": round(fwd_gbs, 1), "unit": "GB/s",
                                "frac": round(fwd_gbs / HBM_PEAK_GBS, 4), "bytes_per_launch": fwd_bytes,
                                "avg_launch_ms": round(fwd_launch_ms, 4), "launches_per_step": n_fwd}

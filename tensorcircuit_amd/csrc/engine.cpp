@@ -139,7 +139,7 @@ int upload(const std::vector<V>& v, void** out) {
 
 void free_tables(DeviceTables* D) {
   if (!D) return;
-  void* ptrs[] = {D->dpass, D->dgroup, D->dop, D->dmem, D->ukbits, D->runoff, D->recipes, D->factors,
+  void* ptrs[] = {D->dpass, D->dop, D->ukbits, D->runoff, D->blob, D->msrc, D->recipes, D->factors,
                   D->gop_list, D->ctab, D->p_ptr, D->p_gops, D->gfac};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -166,11 +166,11 @@ int ensure_tables(Program& P, int dtype, int mode, DeviceTables** out) {
   DeviceTables* D = new DeviceTables();
   int rc = 0;
   rc = rc ? rc : upload(S.dpass, &D->dpass);
-  rc = rc ? rc : upload(S.dgroup, &D->dgroup);
   rc = rc ? rc : upload(S.dop, &D->dop);
-  rc = rc ? rc : upload(S.dmem, &D->dmem);
   rc = rc ? rc : upload(S.ukbits, &D->ukbits);
   rc = rc ? rc : upload(S.runoff, &D->runoff);
+  rc = rc ? rc : upload(S.blob, &D->blob);
+  rc = rc ? rc : upload(S.msrc, &D->msrc);
   rc = rc ? rc : upload(S.recipes, &D->recipes);
   rc = rc ? rc : upload(S.factors, &D->factors);
   rc = rc ? rc : upload(S.gop_list, &D->gop_list);
@@ -237,8 +237,8 @@ int run_one_pass(Program& P, const Sched& S, const DeviceTables& D, int pi, cons
     if (!S.jit.empty() && S.jit[pi].kernel >= 0) {
       if (int rc = jit_launch_fwd(S, D, pi, sizeof(T) == 8, mtab, D.ctab, state, batch, n, ckout, st, zinit ? 1 : 0))
         return rc;
-    } else if (S.R == 4) {
-      launch_fused_fwd<T, 4>(S, D, pi, mtab, D.ctab, state, batch, n, ckout, st);
+    } else if (S.R == kTileSlots) {
+      launch_tile_fwd<T>(S, D, pi, mtab, D.ctab, state, state, batch, n, ckout, zinit, st);
     } else {
       return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", S.R);
     }
@@ -249,10 +249,15 @@ int run_one_pass(Program& P, const Sched& S, const DeviceTables& D, int pi, cons
   return 0;
 }
 
-// forward passes; init_zero: the state starts as |0..0>, generated by a
-// compiled first pass itself (no separate write and read of the state)
-// unless the first pass is of another kind or the initial state is a
-// checkpoint
+// whether pass 0 of S can generate |0..0> itself (a tile pass, not one on
+// the matrix cores)
+bool tile_first(const Sched& S) {
+  return !S.passes.empty() && S.k > 0 && !S.dpass[0].mfma && S.dpass[0].plain_op < 0;
+}
+
+// forward passes; init_zero: the state starts as |0..0>, generated by the
+// first pass itself (no separate write and read of the state) unless it is
+// no tile pass or the initial state is a checkpoint
 template <typename T>
 int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const void* mtab, void* state,
                        int64_t batch, void* ckpts, hipStream_t st, bool init_zero = false) {
@@ -263,8 +268,7 @@ int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const 
   bool ck0 = false;
   if (ckpts)
     for (int a : S.ckpt_after) ck0 = ck0 || a < 0;
-  const bool zfirst = init_zero && !ck0 && !S.passes.empty() && S.k > 0 && !S.dpass[0].mfma &&
-                      S.dpass[0].plain_op < 0 && !S.jit.empty() && S.jit[0].kernel >= 0;
+  const bool zfirst = init_zero && !ck0 && tile_first(S);
   if (init_zero && !zfirst) launch_init_zero<T>(state, n, batch, st);
   // checkpoints of the initial state (before any pass)
   if (ckpts)
@@ -669,17 +673,16 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
         lin = w.lam;
         continue;
       }
-      // psi after the last pass (p = 0) is not read again; a compiled pass
-      // also skips lambda there unless it is the input gradient
-      const bool jitp = !A.jit.empty() && A.jit[p].kernel >= 0;
+      // psi after the last pass (p = 0) is not read again, nor is lambda
+      // unless it is the input gradient
       void* pout = (c >= 0 || p == 0) ? nullptr : w.psi;
-      void* lout = p > 0 ? w.lam : grad_input ? grad_input : jitp ? nullptr : w.lam;
-      if (jitp) {
+      void* lout = p > 0 ? w.lam : grad_input;
+      if (!A.jit.empty() && A.jit[p].kernel >= 0) {
         if (int rc = jit_launch_adj(A, *D, p, sizeof(T) == 8, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n,
                                     w.part, pstride, st))
           return rc;
-      } else if (A.R == 4) {
-        launch_fused_adj<T, 4>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, w.part, pstride, st);
+      } else if (A.R == kTileSlots) {
+        launch_tile_adj<T>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, w.part, pstride, st);
       } else {
         return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", A.R);
       }
@@ -771,26 +774,25 @@ int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int in
     Program& P = descs[i].prog->p;
     if (int rc = ensure_tables(P, dtype, 0, &D[i])) return rc;
     const Sched& S = P.sched[dtype][0];
-    if (S.k > 0 && S.R != 4)
+    if (S.k > 0 && S.R != kTileSlots)
       return set_error(TCM_E_UNSUPPORTED, "multi-program launches run 4 register slots (program %d has %d)", i, S.R);
     mtab[i] = cv.take(descs[i].batch * (int64_t)std::max(S.mtab_size, 1) * sizeof(T));
     if (descs[i].batch <= 0) continue;
     launch_prep<T>(S, *D[i], D[i]->ctab, descs[i].params, descs[i].param_stride, mtab[i], descs[i].batch, st);
-    if (init_zero) launch_init_zero<T>(descs[i].state, P.n, descs[i].batch, st);
+    if (init_zero && !tile_first(S)) launch_init_zero<T>(descs[i].state, P.n, descs[i].batch, st);
     maxp = std::max(maxp, (int)S.passes.size());
   }
   for (int r = 0; r < maxp; ++r) {
     MultiJobs J{};
     int64_t blocks = 0;
-    int threads = 64;
-    size_t lds = 0;
+    int threads = 64, kmax = 0;
     auto flush = [&]() {
       if (J.njobs == 0) return;
-      launch_fused_fwd_multi<T>(J, blocks, threads, lds, st);
+      launch_tile_fwd_multi<T>(J, blocks, threads, kmax, st);
       J = MultiJobs{};
       blocks = 0;
       threads = 64;
-      lds = 0;
+      kmax = 0;
     };
     for (int i = 0; i < ndesc; ++i) {
       const Program& P = descs[i].prog->p;
@@ -802,13 +804,11 @@ int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int in
                                     descs[i].state, P.n, descs[i].batch, st);
         continue;
       }
-      if (S.R != 4) return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", S.R);
       if (S.dpass[r].mfma) return set_error(TCM_E_UNSUPPORTED, "matrix-core passes are not run in multi launches");
       const DPass& dp = S.dpass[r];
       MultiJob& q = J.job[J.njobs++];
-      q.dpass = D[i]->dpass;
-      q.dgroup = D[i]->dgroup;
-      q.dop = D[i]->dop;
+      q.blob = D[i]->blob;
+      q.msrc = D[i]->msrc;
       q.runoff = D[i]->runoff;
       q.ctab = D[i]->ctab;
       q.mtab = mtab[i];
@@ -816,10 +816,11 @@ int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int in
       q.mstride = S.mtab_size;
       q.sstride = 1ll << P.n;
       q.block0 = blocks;
-      q.pass = r;
+      q.pass = tile_pass_arg(dp);
+      q.zinit = r == 0 && init_zero;
       blocks += descs[i].batch << dp.nblk_log;
       threads = std::max(threads, 1 << dp.tthreads_log);
-      lds = std::max(lds, sizeof(V2<T>) << dp.k);
+      kmax = std::max(kmax, dp.k);
       if (J.njobs == kMaxMultiJobs) flush();
     }
     flush();

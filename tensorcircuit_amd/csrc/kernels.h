@@ -98,13 +98,19 @@ struct PauliTileTables {
   const void *chunks, *groups, *terms, *runoff;
 };
 
+// one table-driven tile pass, by value
+struct TilePassArg {
+  int32_t k, L, nblk_log, runoff0, chunk0, nchunk, full, pad;
+  uint64_t bmask;      // index bits outside the tile
+};
 // one program's pass inside a multi-program launch (passed by value)
 struct MultiJob {
-  const void *dpass, *dgroup, *dop, *runoff, *ctab, *mtab;
+  const void *blob, *msrc, *runoff, *ctab, *mtab;
   void* state;
   int64_t mstride, sstride;
   int64_t block0;   // first block of this job in the launch
-  int32_t pass, pad;
+  TilePassArg pass;
+  int32_t zinit, pad;
 };
 constexpr int kMaxMultiJobs = 24;
 struct MultiJobs {
@@ -115,11 +121,11 @@ struct MultiJobs {
 // device copies of one schedule's descriptors (owned by the program)
 struct DeviceTables {
   void* dpass = nullptr;
-  void* dgroup = nullptr;
   void* dop = nullptr;
-  void* dmem = nullptr;
   void* ukbits = nullptr;
   void* runoff = nullptr;
+  void* blob = nullptr;
+  void* msrc = nullptr;
   void* recipes = nullptr;
   void* factors = nullptr;
   void* gop_list = nullptr;
@@ -152,13 +158,19 @@ void launch_copy(void* dst, const void* src, int64_t total, hipStream_t st);
 template <typename T, bool DAG>
 void launch_plain_gate(const DOp& op, const int32_t* ukbits_dev, const void* mtab, int64_t mstride,
                        const void* ctab, void* state, int n, int64_t batch, hipStream_t st);
-template <typename T, int R>
-void launch_fused_fwd(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                      void* state, int64_t batch, int n, void* ckout, hipStream_t st);
-template <typename T, int R>
-void launch_fused_adj(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                      const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
-                      double* part, int64_t pstride, hipStream_t st);
+// table-driven tile passes (tile_pass.hip); in: the state read, or with zinit
+// nothing (the pass starts from |0..0>)
+TilePassArg tile_pass_arg(const DPass& P);
+template <typename T>
+void launch_tile_fwd(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
+                     const void* in, void* out, int64_t batch, int n, void* ckout, bool zinit, hipStream_t st);
+template <typename T>
+void launch_tile_adj(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
+                     const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
+                     double* part, int64_t pstride, hipStream_t st);
+// k: the largest tile of the jobs
+template <typename T>
+void launch_tile_fwd_multi(const MultiJobs& J, int64_t blocks, int threads, int k, hipStream_t st);
 template <typename T>
 void launch_plain_adj(const DOp& op, const void* mtab, int64_t mstride, const void* ctab, const void* psi_in,
                       void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n, int slots, double* part,
@@ -175,8 +187,6 @@ template <typename T>
 void launch_pauli_tile(const DPPass* P, int np, const PauliTileTables& D, const void* psi, const void* lam_in,
                        void* lam_out, int n, const double* alpha, double* epart, int64_t estride, int64_t batch,
                        bool energy, bool apply, hipStream_t st);
-template <typename T>
-void launch_fused_fwd_multi(const MultiJobs& J, int64_t blocks, int threads, size_t lds, hipStream_t st);
 template <typename T>
 void launch_inner(const void* a, const void* c, int n, int64_t batch, int nblk, double* part, int64_t pstride,
                   hipStream_t st);

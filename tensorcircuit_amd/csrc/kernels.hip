@@ -13,15 +13,13 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "regops.h"
 
 namespace tcm {
 
 // ---------------------------------------------------------------------------
 // small helpers
 // ---------------------------------------------------------------------------
-template <int V>
-using IC = std::integral_constant<int, V>;
-
 template <typename T>
 __device__ __forceinline__ V2<T> mk(T a, T b) {
   V2<T> r;
@@ -29,11 +27,6 @@ __device__ __forceinline__ V2<T> mk(T a, T b) {
   r.y = b;
   return r;
 }
-// Im(conj(a) b), Re(conj(a) b)
-template <typename T>
-__device__ __forceinline__ T imcj(V2<T> a, V2<T> b) { return a.x * b.y - a.y * b.x; }
-template <typename T>
-__device__ __forceinline__ T recj(V2<T> a, V2<T> b) { return a.x * b.x + a.y * b.y; }
 
 __device__ __forceinline__ uint32_t swz(uint32_t t) {
   return t ^ (((t >> 4) ^ (t >> 8) ^ (t >> 12) ^ (t >> 16)) & 0xFu);
@@ -57,67 +50,10 @@ __device__ __forceinline__ P* uniform_ptr(P* p) {
   return reinterpret_cast<P*>(((uint64_t)hi << 32) | lo);
 }
 
-// A block-uniform zero the optimiser cannot see through: addresses rebuilt
-// from it are recomputed (cheap scalar work) instead of held live in
-// registers across the group loop.
-__device__ __forceinline__ uint32_t opaque_zero() {
-  uint32_t z = 0;
-  asm volatile("" : "+v"(z));
-  return __builtin_amdgcn_readfirstlane(z);
-}
-__device__ __forceinline__ void rematerialize(uint32_t& dlo, uint32_t& slo, const uint32_t*& ro) {
-  asm volatile("" : "+v"(dlo), "+v"(slo));
-  ro += opaque_zero();
-}
-
-// tile position of a group's thread bits: the thread index bits moved as
-// runs of consecutive bits to their tile positions
-__device__ __forceinline__ uint32_t group_base(const DGroup* G, uint32_t tid) {
-  uint32_t tb = 0;
-  for (int r = 0; r < G->nrun; ++r) {
-    const uint32_t w = (uint32_t)G->run[r];
-    tb |= ((tid >> (w & 0xFFu)) & ((1u << ((w >> 8) & 0xFFu)) - 1u)) << (w >> 16);
-  }
-  return tb;
-}
-
 // insert a zero bit at position b
 __device__ __forceinline__ uint64_t ins0(uint64_t x, int b) {
   uint64_t lo = x & ((1ull << b) - 1);
   return ((x >> b) << (b + 1)) | lo;
-}
-
-template <typename T>
-__device__ __forceinline__ const T* mptr(int moff, const T* mt, const T* ct) {
-  return moff >= 0 ? mt + moff : ct + (-moff - 1);
-}
-
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
-
-// one DPP row-shift of a double (lanes without a source read 0)
-template <int CTRL>
-__device__ __forceinline__ double dpp_shr(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double read_lane(double x, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
-                          __builtin_amdgcn_readlane(__double2loint(x), lane));
-}
-// fp64 sum over a full 64-lane wave, uniform result: inclusive row prefix
-// sums by DPP row_shr 1/2/4/8 leave each 16-lane row's total in its last
-// lane; the four row totals are read back as scalars.
-__device__ __forceinline__ double wave_sum_dpp(double x) {
-  x += dpp_shr<0x111>(x);
-  x += dpp_shr<0x112>(x);
-  x += dpp_shr<0x114>(x);
-  x += dpp_shr<0x118>(x);
-  return (read_lane(x, 15) + read_lane(x, 31)) + (read_lane(x, 47) + read_lane(x, 63));
 }
 
 // block-wide sum of (a, b) in fp64; result valid in thread 0.  blockDim.x
@@ -143,410 +79,6 @@ __device__ __forceinline__ void block_sum2(double& a, double& b) {
     b = sb;
   }
   __syncthreads();
-}
-
-// ---------------------------------------------------------------------------
-// slot dispatch: runtime register slot -> compile-time template argument.
-// Plain switches (no lambdas capturing the register array) so that the
-// per-thread amplitude array stays in VGPRs.
-// ---------------------------------------------------------------------------
-#define TCM_SW1(R, s, ...)                                          \
-  switch (s) {                                                      \
-    case 0: { constexpr int S_ = 0; __VA_ARGS__; } break;           \
-    case 1: if constexpr (R > 1) { constexpr int S_ = 1; __VA_ARGS__; } break; \
-    case 2: if constexpr (R > 2) { constexpr int S_ = 2; __VA_ARGS__; } break; \
-    case 3: if constexpr (R > 3) { constexpr int S_ = 3; __VA_ARGS__; } break; \
-    case 4: if constexpr (R > 4) { constexpr int S_ = 4; __VA_ARGS__; } break; \
-    default: break;                                                 \
-  }
-
-#define TCM_SW2B(R, A_, s1, ...)                                                         \
-  switch (s1) {                                                                          \
-    case 0: if constexpr (A_ != 0) { constexpr int B_ = 0; __VA_ARGS__; } break;         \
-    case 1: if constexpr (R > 1 && A_ != 1) { constexpr int B_ = 1; __VA_ARGS__; } break; \
-    case 2: if constexpr (R > 2 && A_ != 2) { constexpr int B_ = 2; __VA_ARGS__; } break; \
-    case 3: if constexpr (R > 3 && A_ != 3) { constexpr int B_ = 3; __VA_ARGS__; } break; \
-    case 4: if constexpr (R > 4 && A_ != 4) { constexpr int B_ = 4; __VA_ARGS__; } break; \
-    default: break;                                                                      \
-  }
-
-#define TCM_SW2(R, s0, s1, ...)                                                           \
-  switch (s0) {                                                                           \
-    case 0: { constexpr int A_ = 0; TCM_SW2B(R, A_, s1, __VA_ARGS__) } break;             \
-    case 1: if constexpr (R > 1) { constexpr int A_ = 1; TCM_SW2B(R, A_, s1, __VA_ARGS__) } break; \
-    case 2: if constexpr (R > 2) { constexpr int A_ = 2; TCM_SW2B(R, A_, s1, __VA_ARGS__) } break; \
-    case 3: if constexpr (R > 3) { constexpr int A_ = 3; TCM_SW2B(R, A_, s1, __VA_ARGS__) } break; \
-    case 4: if constexpr (R > 4) { constexpr int A_ = 4; TCM_SW2B(R, A_, s1, __VA_ARGS__) } break; \
-    default: break;                                                                       \
-  }
-
-// ---------------------------------------------------------------------------
-// in-register gate application on v[0 .. 2^R): register index bit S <-> the
-// gate qubit.  DAG applies U^dagger.
-// ---------------------------------------------------------------------------
-template <typename T, int R, int S, bool DAG>
-__device__ __forceinline__ void ap_u1(V2<T>* v, const T* m) {
-  T ar = m[0], ai = m[1], br = m[2], bi = m[3], cr = m[4], ci = m[5], dr = m[6], di = m[7];
-  if constexpr (DAG) {
-    T tr = br, ti = bi;
-    br = cr; bi = -ci;
-    cr = tr; ci = -ti;
-    ai = -ai; di = -di;
-  }
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    V2<T> x = v[j], y = v[j | (1 << S)];
-    v[j] = mk<T>(ar * x.x - ai * x.y + br * y.x - bi * y.y, ar * x.y + ai * x.x + br * y.y + bi * y.x);
-    v[j | (1 << S)] = mk<T>(cr * x.x - ci * x.y + dr * y.x - di * y.y, cr * x.y + ci * x.x + dr * y.y + di * y.x);
-  }
-}
-
-template <typename T, int R, int S, bool DAG>
-__device__ __forceinline__ void ap_r1(V2<T>* v, const T* m) {
-  T a = m[0], b = m[1], c = m[2], d = m[3];
-  if constexpr (DAG) {
-    T t = b; b = c; c = t;
-  }
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    V2<T> x = v[j], y = v[j | (1 << S)];
-    v[j] = mk<T>(a * x.x + b * y.x, a * x.y + b * y.y);
-    v[j | (1 << S)] = mk<T>(c * x.x + d * y.x, c * x.y + d * y.y);
-  }
-}
-
-template <typename T, int R, int S, bool DAG>
-__device__ __forceinline__ void ap_d1(V2<T>* v, const T* m) {
-  T d0r = m[0], d0i = m[1], d1r = m[2], d1i = m[3];
-  if constexpr (DAG) { d0i = -d0i; d1i = -d1i; }
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    V2<T> x = v[j];
-    if (j & (1 << S)) v[j] = mk<T>(d1r * x.x - d1i * x.y, d1r * x.y + d1i * x.x);
-    else v[j] = mk<T>(d0r * x.x - d0i * x.y, d0r * x.y + d0i * x.x);
-  }
-}
-
-template <typename T, int R, int S>
-__device__ __forceinline__ void ap_x1(V2<T>* v) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    V2<T> t = v[j];
-    v[j] = v[j | (1 << S)];
-    v[j | (1 << S)] = t;
-  }
-}
-
-// 2-qubit: matrix index r = (bit S0) << 1 | (bit S1)
-template <typename T, int R, int S0, int S1, bool DAG>
-__device__ __forceinline__ void ap_u2(V2<T>* v, const T* m) {
-  T mr[16], mi[16];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if constexpr (DAG) {
-        mr[r * 4 + c] = m[2 * (c * 4 + r)];
-        mi[r * 4 + c] = -m[2 * (c * 4 + r) + 1];
-      } else {
-        mr[r * 4 + c] = m[2 * (r * 4 + c)];
-        mi[r * 4 + c] = m[2 * (r * 4 + c) + 1];
-      }
-    }
-  constexpr int m0 = 1 << S0, m1 = 1 << S1;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (m0 | m1)) continue;
-    const int idx[4] = {j, j | m1, j | m0, j | m0 | m1};
-    V2<T> x[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) x[c] = v[idx[c]];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      T sr = 0, si = 0;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        sr += mr[r * 4 + c] * x[c].x - mi[r * 4 + c] * x[c].y;
-        si += mr[r * 4 + c] * x[c].y + mi[r * 4 + c] * x[c].x;
-      }
-      v[idx[r]] = mk<T>(sr, si);
-    }
-  }
-}
-
-template <typename T, int R, int S0, int S1, bool DAG>
-__device__ __forceinline__ void ap_d2(V2<T>* v, const T* m) {
-  T dr[4], di[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    dr[r] = m[2 * r];
-    di[r] = DAG ? -m[2 * r + 1] : m[2 * r + 1];
-  }
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    const int r = (((j >> S0) & 1) << 1) | ((j >> S1) & 1);
-    V2<T> x = v[j];
-    v[j] = mk<T>(dr[r] * x.x - di[r] * x.y, dr[r] * x.y + di[r] * x.x);
-  }
-}
-
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ void ap_cx(V2<T>* v) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (!(j & (1 << S0)) || (j & (1 << S1))) continue;
-    V2<T> t = v[j];
-    v[j] = v[j | (1 << S1)];
-    v[j | (1 << S1)] = t;
-  }
-}
-
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ void ap_cz(V2<T>* v) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j)
-    if ((j & (1 << S0)) && (j & (1 << S1))) v[j] = mk<T>(-v[j].x, -v[j].y);
-}
-
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ void ap_swap(V2<T>* v) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (!(j & (1 << S0)) || (j & (1 << S1))) continue;
-    const int jj = (j ^ (1 << S0)) | (1 << S1);
-    V2<T> t = v[j];
-    v[j] = v[jj];
-    v[jj] = t;
-  }
-}
-
-template <typename T, int R, bool DAG>
-__device__ __forceinline__ void ap_dg(V2<T>* v, const T* d) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    T dr = d[2 * j], di = DAG ? -d[2 * j + 1] : d[2 * j + 1];
-    V2<T> x = v[j];
-    v[j] = mk<T>(dr * x.x - di * x.y, dr * x.y + di * x.x);
-  }
-}
-
-// apply one op (kinds with a register form) on v.  FULL = false drops the
-// dense 4x4 kind, whose 32-value matrix dominates register pressure; passes
-// without it run a leaner kernel with higher occupancy.
-template <typename T, int R, bool DAG, bool FULL = true>
-__device__ __forceinline__ void apply_op(V2<T>* v, const DOp& op, const T* mt, const T* ct) {
-  switch (op.kind) {
-    case OK_U1: {
-      const T* m = mptr<T>(op.moff, mt, ct);
-      TCM_SW1(R, op.s0, ap_u1<T, R, S_, DAG>(v, m))
-    } break;
-    case OK_R1: {
-      const T* m = mptr<T>(op.moff, mt, ct);
-      TCM_SW1(R, op.s0, ap_r1<T, R, S_, DAG>(v, m))
-    } break;
-    case OK_D1: {
-      const T* m = mptr<T>(op.moff, mt, ct);
-      TCM_SW1(R, op.s0, ap_d1<T, R, S_, DAG>(v, m))
-    } break;
-    case OK_X1:
-      TCM_SW1(R, op.s0, ap_x1<T, R, S_>(v))
-      break;
-    case OK_U2: {
-      if constexpr (FULL) {
-        const T* m = mptr<T>(op.moff, mt, ct);
-        TCM_SW2(R, op.s0, op.s1, ap_u2<T, R, A_, B_, DAG>(v, m))
-      }
-    } break;
-    case OK_D2: {
-      const T* m = mptr<T>(op.moff, mt, ct);
-      TCM_SW2(R, op.s0, op.s1, ap_d2<T, R, A_, B_, DAG>(v, m))
-    } break;
-    case OK_CX:
-      TCM_SW2(R, op.s0, op.s1, ap_cx<T, R, A_, B_>(v))
-      break;
-    case OK_CZ:
-      TCM_SW2(R, op.s0, op.s1, ap_cz<T, R, A_, B_>(v))
-      break;
-    case OK_SWAP:
-      TCM_SW2(R, op.s0, op.s1, ap_swap<T, R, A_, B_>(v))
-      break;
-    case OK_DG:
-      ap_dg<T, R, DAG>(v, mt + op.moff);
-      break;
-    default:
-      break;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// gradient kernels on registers: Im <l | G | p> summed over the thread's
-// amplitudes (p = psi after the gate, l = lambda after the gate)
-// ---------------------------------------------------------------------------
-template <typename T, int R, int S>
-__device__ __forceinline__ T g_x(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    const int jj = j | (1 << S);
-    a += imcj<T>(l[j], p[jj]) + imcj<T>(l[jj], p[j]);
-  }
-  return a;
-}
-template <typename T, int R, int S>
-__device__ __forceinline__ T g_y(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    const int jj = j | (1 << S);
-    a += recj<T>(l[jj], p[j]) - recj<T>(l[j], p[jj]);
-  }
-  return a;
-}
-template <typename T, int R, int S>
-__device__ __forceinline__ T g_z(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    T t = imcj<T>(l[j], p[j]);
-    a += (j & (1 << S)) ? -t : t;
-  }
-  return a;
-}
-template <typename T, int R, int S>
-__device__ __forceinline__ T g_p1(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j)
-    if (j & (1 << S)) a += imcj<T>(l[j], p[j]);
-  return a;
-}
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ T g_xx(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-  constexpr int m = (1 << S0) | (1 << S1);
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) a += imcj<T>(l[j], p[j ^ m]);
-  return a;
-}
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ T g_yy(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-  constexpr int m = (1 << S0) | (1 << S1);
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    T t = imcj<T>(l[j], p[j ^ m]);
-    const int par = ((j >> S0) ^ (j >> S1)) & 1;
-    a += par ? t : -t;
-  }
-  return a;
-}
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ T g_zz(const V2<T>* p, const V2<T>* l) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    T t = imcj<T>(l[j], p[j]);
-    const int par = ((j >> S0) ^ (j >> S1)) & 1;
-    a += par ? -t : t;
-  }
-  return a;
-}
-// general Hermitian generator, 2x2 (U1 layout) on slot S
-template <typename T, int R, int S>
-__device__ __forceinline__ T g_m1(const V2<T>* p, const V2<T>* l, const T* g) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (1 << S)) continue;
-    const int jj = j | (1 << S);
-    V2<T> x = p[j], y = p[jj];
-    V2<T> u = mk<T>(g[0] * x.x - g[1] * x.y + g[2] * y.x - g[3] * y.y, g[0] * x.y + g[1] * x.x + g[2] * y.y + g[3] * y.x);
-    V2<T> w = mk<T>(g[4] * x.x - g[5] * x.y + g[6] * y.x - g[7] * y.y, g[4] * x.y + g[5] * x.x + g[6] * y.y + g[7] * y.x);
-    a += imcj<T>(l[j], u) + imcj<T>(l[jj], w);
-  }
-  return a;
-}
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ T g_m2(const V2<T>* p, const V2<T>* l, const T* g) {
-  T a = 0;
-  constexpr int m0 = 1 << S0, m1 = 1 << S1;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    if (j & (m0 | m1)) continue;
-    const int idx[4] = {j, j | m1, j | m0, j | m0 | m1};
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      T sr = 0, si = 0;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const T gr = g[2 * (r * 4 + c)], gi = g[2 * (r * 4 + c) + 1];
-        sr += gr * p[idx[c]].x - gi * p[idx[c]].y;
-        si += gr * p[idx[c]].y + gi * p[idx[c]].x;
-      }
-      a += imcj<T>(l[idx[r]], mk<T>(sr, si));
-    }
-  }
-  return a;
-}
-
-template <typename T, int R, bool FULL = true>
-__device__ __forceinline__ T grad_op(const V2<T>* p, const V2<T>* l, int gen, int s0, int s1, const T* ct, int goff) {
-  T a = 0;
-  switch (gen) {
-    case GN_X: TCM_SW1(R, s0, a = (g_x<T, R, S_>(p, l))) break;
-    case GN_Y: TCM_SW1(R, s0, a = (g_y<T, R, S_>(p, l))) break;
-    case GN_Z: TCM_SW1(R, s0, a = (g_z<T, R, S_>(p, l))) break;
-    case GN_P1: TCM_SW1(R, s0, a = (g_p1<T, R, S_>(p, l))) break;
-    case GN_XX: TCM_SW2(R, s0, s1, a = (g_xx<T, R, A_, B_>(p, l))) break;
-    case GN_YY: TCM_SW2(R, s0, s1, a = (g_yy<T, R, A_, B_>(p, l))) break;
-    case GN_ZZ: TCM_SW2(R, s0, s1, a = (g_zz<T, R, A_, B_>(p, l))) break;
-    case GN_M1: TCM_SW1(R, s0, a = (g_m1<T, R, S_>(p, l, ct + goff))) break;
-    case GN_M2:
-      if constexpr (FULL) { TCM_SW2(R, s0, s1, a = (g_m2<T, R, A_, B_>(p, l, ct + goff))) }
-      break;
-    default: break;
-  }
-  return a;
-}
-
-// gradient of a diagonal-generator member from precomputed im[j] = Im(conj(l_j) p_j)
-template <typename T, int R, int S>
-__device__ __forceinline__ T gm_z(const T* im) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) a += ((j >> S) & 1) ? -im[j] : im[j];
-  return a;
-}
-template <typename T, int R, int S>
-__device__ __forceinline__ T gm_p1(const T* im) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j)
-    if ((j >> S) & 1) a += im[j];
-  return a;
-}
-template <typename T, int R, int S0, int S1>
-__device__ __forceinline__ T gm_zz(const T* im) {
-  T a = 0;
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) a += (((j >> S0) ^ (j >> S1)) & 1) ? -im[j] : im[j];
-  return a;
-}
-template <typename T, int R>
-__device__ __forceinline__ T grad_member(const T* im, int gen, int s0, int s1) {
-  T a = 0;
-  switch (gen) {
-    case GN_Z: TCM_SW1(R, s0, a = (gm_z<T, R, S_>(im))) break;
-    case GN_P1: TCM_SW1(R, s0, a = (gm_p1<T, R, S_>(im))) break;
-    case GN_ZZ: TCM_SW2(R, s0, s1, a = (gm_zz<T, R, A_, B_>(im))) break;
-    default: break;
-  }
-  return a;
 }
 
 // ---------------------------------------------------------------------------
@@ -711,7 +243,7 @@ __global__ void k_init_zero(V2<T>* __restrict__ st, int64_t total, int64_t N) {
 // ---------------------------------------------------------------------------
 template <typename T, int KIND, bool DAG>
 __global__ void __launch_bounds__(256) k_plain1(DOp op, const T* __restrict__ mtab, int64_t mstride,
-                                                const T* __restrict__ ct, V2<T>* __restrict__ st,
+                                                const T* __restrict__ ct, A2<T>* __restrict__ st,
                                                 int64_t sstride, int n, int64_t batch) {
   const int64_t items = 1ll << (n - 1);
   const int64_t total = items * batch;
@@ -720,8 +252,8 @@ __global__ void __launch_bounds__(256) k_plain1(DOp op, const T* __restrict__ mt
     const int64_t b = w >> (n - 1);
     const int64_t idx = w & (items - 1);
     const uint64_t i0 = ins0(idx, b0), i1 = i0 | (1ull << b0);
-    V2<T>* s = st + b * sstride;
-    V2<T> v[2] = {s[i0], s[i1]};
+    A2<T>* s = st + b * sstride;
+    A2<T> v[2] = {s[i0], s[i1]};
     const T* mt = mtab + b * mstride;
     DOp o = op;
     o.s0 = 0;
@@ -733,7 +265,7 @@ __global__ void __launch_bounds__(256) k_plain1(DOp op, const T* __restrict__ mt
 
 template <typename T, int KIND, bool DAG>
 __global__ void __launch_bounds__(256) k_plain2(DOp op, const T* __restrict__ mtab, int64_t mstride,
-                                                const T* __restrict__ ct, V2<T>* __restrict__ st,
+                                                const T* __restrict__ ct, A2<T>* __restrict__ st,
                                                 int64_t sstride, int n, int64_t batch) {
   const int64_t items = 1ll << (n - 2);
   const int64_t total = items * batch;
@@ -744,9 +276,9 @@ __global__ void __launch_bounds__(256) k_plain2(DOp op, const T* __restrict__ mt
     const int64_t idx = w & (items - 1);
     const uint64_t i00 = ins0(ins0(idx, lo), hi);
     const uint64_t ma = 1ull << ba, mb = 1ull << bb;
-    V2<T>* s = st + b * sstride;
+    A2<T>* s = st + b * sstride;
     // register index: bit 1 <-> qubit 0 (matrix MSB), bit 0 <-> qubit 1
-    V2<T> v[4] = {s[i00], s[i00 | mb], s[i00 | ma], s[i00 | ma | mb]};
+    A2<T> v[4] = {s[i00], s[i00 | mb], s[i00 | ma], s[i00 | ma | mb]};
     const T* mt = mtab + b * mstride;
     DOp o = op;
     o.s0 = 1;
@@ -809,22 +341,22 @@ __global__ void __launch_bounds__(256) k_plaink(DOp op, const int32_t* __restric
 // grid = (slots, batch); partial[b * pstride + blockIdx.x]
 template <typename T, int NQ>
 __global__ void __launch_bounds__(256) k_plain_adj(DOp op, const T* __restrict__ mtab, int64_t mstride,
-                                                   const T* __restrict__ ct, const V2<T>* psi_in, V2<T>* psi_out,
-                                                   const V2<T>* lam_in, V2<T>* lam_out, int64_t sstride, int n,
+                                                   const T* __restrict__ ct, const A2<T>* psi_in, A2<T>* psi_out,
+                                                   const A2<T>* lam_in, A2<T>* lam_out, int64_t sstride, int n,
                                                    double* __restrict__ part, int64_t pstride) {
   const int64_t items = 1ll << (n - NQ);
   const int64_t b = blockIdx.y;
   const T* mt = mtab + b * mstride;
-  const V2<T>* pi = psi_in + b * sstride;
-  const V2<T>* li = lam_in + b * sstride;
-  V2<T>* po = psi_out ? psi_out + b * sstride : nullptr;
-  V2<T>* lo_ = lam_out + b * sstride;
+  const A2<T>* pi = psi_in + b * sstride;
+  const A2<T>* li = lam_in + b * sstride;
+  A2<T>* po = psi_out ? psi_out + b * sstride : nullptr;
+  A2<T>* lo_ = lam_out + b * sstride;
   double acc = 0.0;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < items; idx += (int64_t)gridDim.x * blockDim.x) {
     if constexpr (NQ == 1) {
       const int b0 = op.s0;
       const uint64_t i0 = ins0(idx, b0), i1 = i0 | (1ull << b0);
-      V2<T> p[2] = {pi[i0], pi[i1]}, l[2] = {li[i0], li[i1]};
+      A2<T> p[2] = {pi[i0], pi[i1]}, l[2] = {li[i0], li[i1]};
       if (op.gen != GN_NONE) acc += (double)grad_op<T, 1>(p, l, op.gen, 0, -1, ct, op.goff);
       DOp o = op;
       o.s0 = 0;
@@ -839,7 +371,7 @@ __global__ void __launch_bounds__(256) k_plain_adj(DOp op, const T* __restrict__
       const uint64_t i00 = ins0(ins0(idx, lo), hi);
       const uint64_t ma = 1ull << ba, mb = 1ull << bb;
       const uint64_t ad[4] = {i00, i00 | mb, i00 | ma, i00 | ma | mb};
-      V2<T> p[4], l[4];
+      A2<T> p[4], l[4];
 #pragma unroll
       for (int c = 0; c < 4; ++c) { p[c] = pi[ad[c]]; l[c] = li[ad[c]]; }
       if (op.gen != GN_NONE) acc += (double)grad_op<T, 2>(p, l, op.gen, 1, 0, ct, op.goff);
@@ -859,223 +391,6 @@ __global__ void __launch_bounds__(256) k_plain_adj(DOp op, const T* __restrict__
     double dummy = 0.0;
     block_sum2(acc, dummy);
     if (threadIdx.x == 0) part[b * pstride + blockIdx.x] = acc;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// fused passes: a tile of 2^k amplitudes (k tile bits) is staged in LDS,
-// register groups of 2^R amplitudes per thread apply runs of gates, and the
-// tile is written back -- one HBM read + write for all gates of the pass.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t block_base(const DPass* P, uint64_t blk) {
-  uint64_t base = 0;
-  for (int i = 0; i < P->nblk_log; ++i)
-    if ((blk >> i) & 1) base |= 1ull << P->blk_bits[i];
-  return base;
-}
-
-// Body of one fused forward pass over tile `blk` of batch item `b`; threads
-// tid >= nthr (a smaller tile than the block) only take part in barriers.
-template <typename T, int R, bool FULL>
-__device__ __forceinline__ void fused_fwd_tile(const DPass* P, const DGroup* __restrict__ groups,
-                                               const DOp* __restrict__ ops, const uint32_t* __restrict__ runoff,
-                                               const T* mt, const T* __restrict__ ct, V2<T>* __restrict__ s,
-                                               V2<T>* __restrict__ c, int nthr, V2<T>* tile) {
-  const int k = P->k, L = P->L;
-  const int tid = threadIdx.x;
-  const bool act = tid < nthr;
-  const uint32_t* ro = runoff + P->runoff0;
-  uint32_t dlo = act ? tile_dep(ro, L, tid) : 0u;
-  uint32_t slo = swz(tid);
-  if (act) {
-    // all loads in flight before the first LDS write
-    V2<T> buf[1 << R];
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) buf[it] = s[tile_dep(ro, L, it * nthr) + dlo];
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) tile[swz(it * nthr) ^ slo] = buf[it];
-  }
-  __syncthreads();
-  for (int g = 0; g < P->ngroups; ++g) {
-    const DGroup* G = groups + P->group0 + g;
-    if (act) {
-      const uint32_t a0 = swz(group_base(G, tid));
-      V2<T> v[1 << R];
-#pragma unroll
-      for (int j = 0; j < (1 << R); ++j) v[j] = tile[a0 ^ (uint32_t)G->S[j]];
-      for (int o = 0; o < G->nops; ++o) apply_op<T, R, false, FULL>(v, ops[G->op0 + o], mt, ct);
-      const DGroup* Gs = G + opaque_zero();
-      uint32_t as = a0;
-      asm volatile("" : "+v"(as));
-#pragma unroll
-      for (int j = 0; j < (1 << R); ++j) tile[as ^ (uint32_t)Gs->S[j]] = v[j];
-    }
-    __syncthreads();
-  }
-  rematerialize(dlo, slo, ro);
-  if (act) {
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) {
-      const uint32_t ah = it * nthr;
-      const V2<T> x = tile[swz(ah) ^ slo];
-      const uint32_t off = tile_dep(ro, L, ah) + dlo;
-      s[off] = x;
-      if (c) c[off] = x;
-    }
-  }
-}
-
-template <typename T, int R, int TB, bool FULL>
-__global__ void __launch_bounds__(TB) k_fused_fwd(const DPass* __restrict__ passes, int pi,
-                                                  const DGroup* __restrict__ groups, const DOp* __restrict__ ops,
-                                                  const uint32_t* __restrict__ runoff, const T* __restrict__ mtab,
-                                                  int64_t mstride, const T* __restrict__ ct,
-                                                  V2<T>* __restrict__ st, int64_t sstride,
-                                                  V2<T>* __restrict__ ckout) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const DPass* P = passes + pi;
-  const int nbl = P->nblk_log;
-  const uint64_t blk = blockIdx.x & ((1ull << nbl) - 1);
-  const uint64_t b = (uint64_t)blockIdx.x >> nbl;
-  const uint64_t base = block_base(P, blk);
-  fused_fwd_tile<T, R, FULL>(P, groups, ops, runoff, mtab + b * mstride, ct, st + b * sstride + base,
-                             ckout ? ckout + b * sstride + base : nullptr, blockDim.x,
-                             reinterpret_cast<V2<T>*>(smem));
-}
-
-// Several programs' passes in one launch (circuits of different qubit
-// counts): block -> job by the prefix of the jobs' block counts.
-template <typename T, int R, int TB>
-__global__ void __launch_bounds__(TB) k_fused_fwd_multi(MultiJobs J) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  int j = 0;
-  while (j + 1 < J.njobs && (int64_t)blockIdx.x >= J.job[j + 1].block0) ++j;
-  j = __builtin_amdgcn_readfirstlane(j);  // block-uniform
-  const MultiJob& Q = J.job[j];
-  // the job's fields are block-uniform: keep them in scalar registers
-  const DPass* P = uniform_ptr((const DPass*)Q.dpass) + __builtin_amdgcn_readfirstlane(Q.pass);
-  const DGroup* groups = uniform_ptr((const DGroup*)Q.dgroup);
-  const DOp* ops = uniform_ptr((const DOp*)Q.dop);
-  const uint32_t* runoff = uniform_ptr((const uint32_t*)Q.runoff);
-  const T* ct = uniform_ptr((const T*)Q.ctab);
-  const int nbl = P->nblk_log;
-  const uint64_t lb = (uint64_t)blockIdx.x - Q.block0;
-  const uint64_t blk = lb & ((1ull << nbl) - 1);
-  const uint64_t b = lb >> nbl;
-  const uint64_t base = block_base(P, blk);
-  const T* mt = uniform_ptr((const T*)Q.mtab + b * Q.mstride);
-  V2<T>* s = uniform_ptr((V2<T>*)Q.state + b * Q.sstride + base);
-  if (P->full)
-    fused_fwd_tile<T, R, true>(P, groups, ops, runoff, mt, ct, s, nullptr, 1 << P->tthreads_log,
-                               reinterpret_cast<V2<T>*>(smem));
-  else
-    fused_fwd_tile<T, R, false>(P, groups, ops, runoff, mt, ct, s, nullptr, 1 << P->tthreads_log,
-                                reinterpret_cast<V2<T>*>(smem));
-}
-
-// Reverse sweep over one fused pass.  psi/lambda tiles are read from
-// psi_in/lam_in, gates are undone in reverse order, gradient partials of the
-// pass's trainable gates are reduced per tile into part[b][gloc][blk], and
-// the tiles are written to psi_out (skipped when NULL: a checkpoint replaces
-// it) and lam_out.
-template <typename T, int R, int TB, bool FULL>
-__global__ void __launch_bounds__(TB) k_fused_adj(const DPass* __restrict__ passes, int pi,
-                                                    const DGroup* __restrict__ groups, const DOp* __restrict__ ops,
-                                                    const DMember* __restrict__ mems,
-                                                    const uint32_t* __restrict__ runoff, const T* __restrict__ mtab,
-                                                    int64_t mstride, const T* __restrict__ ct,
-                                                    const V2<T>* psi_in, V2<T>* psi_out,
-                                                    const V2<T>* lam_in, V2<T>* lam_out, int64_t sstride,
-                                                    double* __restrict__ part, int64_t pstride) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const DPass* P = passes + pi;
-  const int k = P->k, L = P->L, nbl = P->nblk_log;
-  V2<T>* tp = reinterpret_cast<V2<T>*>(smem);
-  V2<T>* tl = tp + (1 << k);
-  // red[gloc][wave]: fp64 wave sums of each trainable gate of the pass
-  double* red = reinterpret_cast<double*>(tl + (1 << k));
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int lane = tid & 63, wv = tid >> 6, nw = nthr >> 6;
-  const uint64_t blk = blockIdx.x & ((1ull << nbl) - 1);
-  const uint64_t b = (uint64_t)blockIdx.x >> nbl;
-  const uint64_t base = block_base(P, blk);
-  const T* mt = mtab + b * mstride;
-  const uint32_t* ro = runoff + P->runoff0;
-  uint32_t dlo = tile_dep(ro, L, tid);
-  uint32_t slo = swz(tid);
-  {
-    const V2<T>* sp = psi_in + b * sstride + base;
-    const V2<T>* sl = lam_in + b * sstride + base;
-    V2<T> bp[1 << R], bl[1 << R];
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) {
-      const uint32_t off = tile_dep(ro, L, it * nthr) + dlo;
-      bp[it] = sp[off];
-      bl[it] = sl[off];
-    }
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) {
-      tp[swz(it * nthr) ^ slo] = bp[it];
-      tl[swz(it * nthr) ^ slo] = bl[it];
-    }
-  }
-  __syncthreads();
-  for (int g = P->ngroups - 1; g >= 0; --g) {
-    const DGroup* G = groups + P->group0 + g;
-    const uint32_t a0 = swz(group_base(G, tid));
-    V2<T> p[1 << R], l[1 << R];
-#pragma unroll
-    for (int j = 0; j < (1 << R); ++j) {
-      p[j] = tp[a0 ^ (uint32_t)G->S[j]];
-      l[j] = tl[a0 ^ (uint32_t)G->S[j]];
-    }
-    for (int o = G->nops - 1; o >= 0; --o) {
-      const DOp& op = ops[G->op0 + o];
-      if (op.kind == OK_DG && op.nmem > 0) {
-        T im[1 << R];
-#pragma unroll
-        for (int j = 0; j < (1 << R); ++j) im[j] = imcj<T>(l[j], p[j]);
-        for (int q = 0; q < op.nmem; ++q) {
-          const DMember& M = mems[op.mem0 + q];
-          const double gs = wave_sum_dpp((double)grad_member<T, R>(im, M.gen, M.s0, M.s1));
-          if (lane == 0) red[M.gloc * nw + wv] = gs;
-        }
-      } else if (op.gen != GN_NONE) {
-        const double gs = wave_sum_dpp((double)grad_op<T, R, FULL>(p, l, op.gen, op.s0, op.s1, ct, op.goff));
-        if (lane == 0) red[op.gloc * nw + wv] = gs;
-      }
-      apply_op<T, R, true, FULL>(p, op, mt, ct);
-      apply_op<T, R, true, FULL>(l, op, mt, ct);
-    }
-    const DGroup* Gs = G + opaque_zero();
-    uint32_t as = a0;
-    asm volatile("" : "+v"(as));
-#pragma unroll
-    for (int j = 0; j < (1 << R); ++j) {
-      tp[as ^ (uint32_t)Gs->S[j]] = p[j];
-      tl[as ^ (uint32_t)Gs->S[j]] = l[j];
-    }
-    __syncthreads();
-  }
-  // recompute the store addresses instead of holding the load addresses in
-  // registers through the group loop
-  rematerialize(dlo, slo, ro);
-  {
-    V2<T>* sp = psi_out ? psi_out + b * sstride + base : nullptr;
-    V2<T>* sl = lam_out + b * sstride + base;
-#pragma unroll
-    for (int it = 0; it < (1 << R); ++it) {
-      const uint32_t ah = it * nthr;
-      const uint32_t off = tile_dep(ro, L, ah) + dlo;
-      if (sp) sp[off] = tp[swz(ah) ^ slo];
-      sl[off] = tl[swz(ah) ^ slo];
-    }
-  }
-  const int ng = P->ngop;
-  for (int q = tid; q < ng; q += nthr) {
-    double s = 0.0;
-    for (int w = 0; w < nw; ++w) s += red[q * nw + w];
-    part[b * pstride + (int64_t)q * (1ll << nbl) + blk] = s;
   }
 }
 
@@ -1617,11 +932,11 @@ void launch_plain_gate(const DOp& op, const int32_t* ukbits_dev, const void* mta
   switch (op.kind) {
     case OK_U1: case OK_R1: case OK_D1: case OK_X1:
       hipLaunchKernelGGL((k_plain1<T, 0, DAG>), dim3(grid_for(batch * (N >> 1))), dim3(256), 0, st, op, mt, mstride,
-                         ct, s, N, n, batch);
+                         ct, (A2<T>*)s, N, n, batch);
       break;
     case OK_U2: case OK_D2: case OK_CX: case OK_CZ: case OK_SWAP:
       hipLaunchKernelGGL((k_plain2<T, 0, DAG>), dim3(grid_for(batch * (N >> 2))), dim3(256), 0, st, op, mt, mstride,
-                         ct, s, N, n, batch);
+                         ct, (A2<T>*)s, N, n, batch);
       break;
     case OK_UK:
       if constexpr (std::is_same<T, float>::value) {
@@ -1643,13 +958,6 @@ void launch_plain_gate(const DOp& op, const int32_t* ukbits_dev, const void* mta
   }
 }
 
-template <typename T>
-static size_t fused_lds_fwd(int k) { return sizeof(V2<T>) << k; }
-template <typename T>
-static size_t fused_lds_adj(int k, int ngop, int nthr) {
-  return (2 * sizeof(V2<T>) << k) + sizeof(double) * (size_t)(ngop > 0 ? ngop : 1) * (nthr / 64);
-}
-
 // kernels that need more than 64 KiB of dynamic LDS must opt in once
 template <typename K>
 static void ensure_lds_attr(K kern, size_t bytes) {
@@ -1663,71 +971,6 @@ static void ensure_lds_attr(K kern, size_t bytes) {
   d = bytes;
 }
 
-template <typename T, int R, int TB, bool FULL>
-static void launch_fused_fwd_tb(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                                void* state, int64_t batch, int n, void* ckout, hipStream_t st) {
-  const DPass& P = S.dpass[pi];
-  const size_t lds = fused_lds_fwd<T>(P.k);
-  ensure_lds_attr(k_fused_fwd<T, R, TB, FULL>, lds);
-  const int64_t blocks = batch << P.nblk_log;
-  hipLaunchKernelGGL((k_fused_fwd<T, R, TB, FULL>), dim3((unsigned)blocks), dim3(1u << P.tthreads_log), lds, st,
-                     (const DPass*)D.dpass, pi, (const DGroup*)D.dgroup, (const DOp*)D.dop,
-                     (const uint32_t*)D.runoff, (const T*)mtab, (int64_t)S.mtab_size, (const T*)ctab,
-                     (V2<T>*)state, (int64_t)1 << n, (V2<T>*)ckout);
-}
-
-template <typename T, int R>
-void launch_fused_fwd(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                      void* state, int64_t batch, int n, void* ckout, hipStream_t st) {
-  const int thr = 1 << S.dpass[pi].tthreads_log;
-  const bool full = S.dpass[pi].full != 0;
-#define TCM_FWD(TB, F) launch_fused_fwd_tb<T, R, TB, F>(S, D, pi, mtab, ctab, state, batch, n, ckout, st)
-  if (thr <= 256) { if (full) TCM_FWD(256, true); else TCM_FWD(256, false); }
-  else if (thr <= 512) { if (full) TCM_FWD(512, true); else TCM_FWD(512, false); }
-  else { if (full) TCM_FWD(1024, true); else TCM_FWD(1024, false); }
-#undef TCM_FWD
-}
-
-template <typename T>
-void launch_fused_fwd_multi(const MultiJobs& J, int64_t blocks, int threads, size_t lds, hipStream_t st) {
-  if (threads <= 256) {
-    ensure_lds_attr(k_fused_fwd_multi<T, 4, 256>, lds);
-    hipLaunchKernelGGL((k_fused_fwd_multi<T, 4, 256>), dim3((unsigned)blocks), dim3(threads), lds, st, J);
-  } else {
-    ensure_lds_attr(k_fused_fwd_multi<T, 4, 512>, lds);
-    hipLaunchKernelGGL((k_fused_fwd_multi<T, 4, 512>), dim3((unsigned)blocks), dim3(threads), lds, st, J);
-  }
-}
-
-template <typename T, int R, int TB, bool FULL>
-static void launch_fused_adj_tb(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                                const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch,
-                                int n, double* part, int64_t pstride, hipStream_t st) {
-  const DPass& P = S.dpass[pi];
-  const size_t lds = fused_lds_adj<T>(P.k, P.ngop, 1 << P.tthreads_log);
-  ensure_lds_attr(k_fused_adj<T, R, TB, FULL>, lds);
-  const int64_t blocks = batch << P.nblk_log;
-  hipLaunchKernelGGL((k_fused_adj<T, R, TB, FULL>), dim3((unsigned)blocks), dim3(1u << P.tthreads_log), lds, st,
-                     (const DPass*)D.dpass, pi, (const DGroup*)D.dgroup, (const DOp*)D.dop,
-                     (const DMember*)D.dmem, (const uint32_t*)D.runoff, (const T*)mtab, (int64_t)S.mtab_size,
-                     (const T*)ctab, (const V2<T>*)psi_in, (V2<T>*)psi_out, (const V2<T>*)lam_in, (V2<T>*)lam_out,
-                     (int64_t)1 << n, part, pstride);
-}
-
-template <typename T, int R>
-void launch_fused_adj(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
-                      const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
-                      double* part, int64_t pstride, hipStream_t st) {
-  const int thr = 1 << S.dpass[pi].tthreads_log;
-  const bool full = S.dpass[pi].full != 0;
-#define TCM_ADJ(TB, F) \
-  launch_fused_adj_tb<T, R, TB, F>(S, D, pi, mtab, ctab, psi_in, psi_out, lam_in, lam_out, batch, n, part, pstride, st)
-  if (thr <= 256) { if (full) TCM_ADJ(256, true); else TCM_ADJ(256, false); }
-  else if (thr <= 512) { if (full) TCM_ADJ(512, true); else TCM_ADJ(512, false); }
-  else { if (full) TCM_ADJ(1024, true); else TCM_ADJ(1024, false); }
-#undef TCM_ADJ
-}
-
 template <typename T>
 void launch_plain_adj(const DOp& op, const void* mtab, int64_t mstride, const void* ctab, const void* psi_in,
                       void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n, int slots, double* part,
@@ -1736,11 +979,11 @@ void launch_plain_adj(const DOp& op, const void* mtab, int64_t mstride, const vo
   const int nq = (op.kind == OK_U1 || op.kind == OK_R1 || op.kind == OK_D1 || op.kind == OK_X1) ? 1 : 2;
   if (nq == 1)
     hipLaunchKernelGGL((k_plain_adj<T, 1>), grid, dim3(256), 0, st, op, (const T*)mtab, mstride, (const T*)ctab,
-                       (const V2<T>*)psi_in, (V2<T>*)psi_out, (const V2<T>*)lam_in, (V2<T>*)lam_out,
+                       (const A2<T>*)psi_in, (A2<T>*)psi_out, (const A2<T>*)lam_in, (A2<T>*)lam_out,
                        (int64_t)1 << n, n, part, pstride);
   else
     hipLaunchKernelGGL((k_plain_adj<T, 2>), grid, dim3(256), 0, st, op, (const T*)mtab, mstride, (const T*)ctab,
-                       (const V2<T>*)psi_in, (V2<T>*)psi_out, (const V2<T>*)lam_in, (V2<T>*)lam_out,
+                       (const A2<T>*)psi_in, (A2<T>*)psi_out, (const A2<T>*)lam_in, (A2<T>*)lam_out,
                        (int64_t)1 << n, n, part, pstride);
 }
 
@@ -2082,11 +1325,6 @@ void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* v
                                             void*, int, int64_t, hipStream_t);                                 \
   template void launch_plain_gate<T, true>(const DOp&, const int32_t*, const void*, int64_t, const void*,     \
                                            void*, int, int64_t, hipStream_t);                                  \
-  template void launch_fused_fwd<T, 4>(const Sched&, const DeviceTables&, int, const void*, const void*,      \
-                                       void*, int64_t, int, void*, hipStream_t);                               \
-  template void launch_fused_adj<T, 4>(const Sched&, const DeviceTables&, int, const void*, const void*,      \
-                                       const void*, void*, const void*, void*, int64_t, int, double*, int64_t, \
-                                       hipStream_t);                                                           \
   template void launch_plain_adj<T>(const DOp&, const void*, int64_t, const void*, const void*, void*,        \
                                     const void*, void*, int64_t, int, int, double*, int64_t, hipStream_t);     \
   template void launch_plain_adj_uk<T>(const DOp&, const int32_t*, const void*, void*, void*, int64_t, int,   \
@@ -2094,7 +1332,6 @@ void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* v
   template void launch_pauli<T>(const DPGroup&, const DPTerm*, int, const void*, void*, int, const double*,   \
                                 double*, int64_t, int64_t, bool, bool, hipStream_t);                           \
   template void launch_inner<T>(const void*, const void*, int, int64_t, int, double*, int64_t, hipStream_t); \
-  template void launch_fused_fwd_multi<T>(const MultiJobs&, int64_t, int, size_t, hipStream_t);                 \
   template void launch_probability<T>(const void*, void*, int64_t, hipStream_t);                               \
   template void launch_sample<T>(const void*, bool, int, int64_t, const double*, int64_t, int64_t*, double*,   \
                                  hipStream_t);                                                                 \

@@ -749,13 +749,16 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
     return -1;
   };
   dg.op0 = (int)S.dop.size();
+  // the table-driven kernels know diagonals only as tables over the group's
+  // slots; compiled passes keep a lone one in its own form
+  const size_t merge = S.R == kTileSlots && !P.opts.jit ? 1 : 2;
   const auto& gl = hg.gates;
   size_t i = 0;
   while (i < gl.size()) {
     // maximal run of mergeable diagonal gates
     size_t j = i;
     while (j < gl.size() && diag_kind(P.gates[gl[j]])) ++j;
-    if (j - i >= 2) {
+    if (j - i >= merge) {
       DRecipe r{};
       r.kind = -1;
       r.out = S.mtab_size;
@@ -800,6 +803,7 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
     op.moff = g.mslot >= 0 ? g.mslot : (g.cslot >= 0 ? -g.cslot - 1 : 0);
     op.gen = g.gen;
     if (g.src == TCM_G_RY && g.okind == OK_R1 && g.mslot >= 0) op.flags |= OP_F_SHEAR;
+    if (g.src == TCM_G_RX && g.mslot >= 0) op.flags |= OP_F_RX;
     op.goff = g.goff;
     op.gop = g.gop;
     op.gloc = g.gop >= 0 ? gloc_of_gop[g.gop] : -1;
@@ -884,6 +888,230 @@ static void tile_run(const Program& P, Sched& S, const std::vector<int>& items, 
   }
 }
 
+// Staged tables (kStage* in tcm_internal.h) of the tile pass dp with register
+// groups hp.groups, for the table-driven kernels; adj: processing order
+// reversed, with gradients.
+static void stage_pass(Sched& S, const HPass& hp, DPass& dp, bool adj) {
+  dp.chunk0 = (int)(S.blob.size() / kStageBlob);
+  uint32_t blob[kStageBlob];
+  int32_t msrc[kStageMat];
+  int nseg = 0, nop = 0, nmat = 0, nmem = 0, ngl = 0;
+  auto reset = [&]() {
+    std::fill(blob, blob + kStageBlob, 0u);
+    std::fill(msrc, msrc + kStageMat, kStageNone);
+    nseg = nop = nmat = nmem = ngl = 0;
+  };
+  auto close = [&]() {
+    if (nseg == 0) return;
+    blob[kStageCount] = (uint32_t)nseg;
+    blob[kStageCount + 1] = (uint32_t)ngl;
+    S.blob.insert(S.blob.end(), blob, blob + kStageBlob);
+    S.msrc.insert(S.msrc.end(), msrc, msrc + kStageMat);
+    reset();
+  };
+  reset();
+  constexpr uint32_t kNoPerm = 0x08421u << 8;
+  // CX control c -> target t: place in the kernels' fixed order
+  auto cx_index = [&](int c, int t) {
+    const int i = 3 * (3 - c) + (3 - (t > c ? t : t + 1));
+    return adj ? 11 - i : i;
+  };
+  // one macro op being filled; stage: the last place taken in its order
+  struct MacroOp {
+    const DOp *ry[4] = {}, *rx[4] = {}, *dg = nullptr, *single = nullptr;
+    uint32_t cx = 0;
+    int m0 = 0, nm = 0, stage = -1;  // members m0 .. m0 + nm - 1
+  };
+  const int ng = (int)hp.groups.size();
+  for (int q = 0; q < ng; ++q) {
+    const int gi = adj ? ng - 1 - q : q;
+    const HGroup& hg = hp.groups[gi];
+    const DGroup& dg = S.dgroup[dp.group0 + gi];
+    std::vector<int> asc(hg.slots.begin(), hg.slots.end());
+    std::sort(asc.begin(), asc.end());
+    uint32_t word = 0;
+    for (int s = 0; s < kTileSlots; ++s) word |= (uint32_t)hg.slots[s] << (4 * s) | (uint32_t)asc[s] << (16 + 4 * s);
+    bool open = false;  // this group has a segment in the current chunk
+    auto segment = [&]() {
+      if (open) return;
+      if (nseg == kStageSegs) close();
+      blob[2 * nseg] = word;
+      blob[2 * nseg + 1] = kNoPerm;
+      ++nseg;
+      open = true;
+    };
+    MacroOp M;
+    // emit M into the chunk (a new one if it does not fit)
+    auto flush = [&]() {
+      if (M.stage < 0) return;
+      auto trains = [&](const DOp* o) { return adj && o && o->gen != GN_NONE; };
+      int mats = 0, grads = M.nm;
+      for (int s = 0; s < kTileSlots; ++s) {
+        mats += (M.ry[s] ? 4 : 0) + (M.rx[s] ? 4 : 0);
+        grads += (trains(M.ry[s]) ? 1 : 0) + (trains(M.rx[s]) ? 1 : 0);
+      }
+      if (M.dg) mats += 2 << kTileSlots;
+      int smat = 0, gmat = 0;
+      bool swapped = false;
+      if (M.single) {
+        const int k = M.single->kind;
+        smat = k == OK_U1 || k == OK_D1 ? 8 : k == OK_R1 ? 4 : k == OK_U2 || k == OK_D2 ? 32 : 0;
+        if (trains(M.single)) {
+          gmat = M.single->gen == GN_M1 ? 8 : M.single->gen == GN_M2 ? 32 : 0;
+          ++grads;
+        }
+        swapped = M.single->s1 >= 0 && M.single->s0 < M.single->s1;
+      }
+      mats += smat + gmat;
+      if (nop == kStageMaxOps || nmat + mats > kStageMat || ngl + grads > kStageGrad || (!open && nseg == kStageSegs)) {
+        close();
+        open = false;
+      }
+      segment();
+      const int m0 = nmat;
+      auto put = [&](int off, int cnt) {  // off >= 0: the item's table, else the constants
+        for (int i = 0; i < cnt; ++i) msrc[nmat++] = off >= 0 ? off + i : off - i;
+      };
+      uint32_t w0 = 0, w1 = 0;
+      auto rotations = [&](const DOp* const* r, int shift) {
+        for (int s = 0; s < kTileSlots; ++s) {
+          if (!r[s]) continue;
+          w0 |= 1u << (shift + s);
+          put(r[s]->moff, 4);
+          if (trains(r[s])) {
+            w1 |= 1u << (shift + s);
+            blob[kStageGl + ngl++] = (uint32_t)r[s]->gloc;
+          }
+        }
+      };
+      auto diagonal = [&]() {
+        if (M.nm) w1 |= (uint32_t)M.nm << 12 | (uint32_t)nmem << 20;
+        for (int i = 0; i < M.nm; ++i) {
+          const DMember& D = S.dmem[M.m0 + i];
+          blob[kStageMems + nmem++] = (uint32_t)D.gen | (uint32_t)(D.s0 & 7) << 4 | (uint32_t)(D.s1 & 7) << 7;
+          blob[kStageGl + ngl++] = (uint32_t)D.gloc;
+        }
+        if (M.dg) {
+          w0 |= 1u << 28;
+          put(M.dg->moff, 2 << kTileSlots);
+        }
+      };
+      w0 |= M.cx << 8;
+      if (adj) {
+        diagonal();
+        rotations(M.rx, 4);
+        rotations(M.ry, 0);
+      } else {
+        rotations(M.ry, 0);
+        rotations(M.rx, 4);
+        diagonal();
+      }
+      int gm = 0;
+      if (M.single) {
+        const DOp& op = *M.single;
+        const int s0 = swapped ? op.s1 : op.s0, s1 = swapped ? op.s0 : op.s1;
+        // a lone diagonal whose generator is a matrix runs as a full one
+        const int kind = op.kind == OK_D1 ? OK_U1 : op.kind == OK_D2 ? OK_U2 : op.kind;
+        w0 |= (uint32_t)(kind + 1) << 20 | (uint32_t)(s0 & 3) << 24 | (uint32_t)(s1 & 3) << 26;
+        // entry e (re / im of a row-major matrix over d basis states; a
+        // two-slot matrix over the slots in descending order)
+        auto full = [&](int off, int d, bool diag) {
+          for (int r = 0; r < d; ++r)
+            for (int c = 0; c < d; ++c)
+              for (int z = 0; z < 2; ++z) {
+                auto basis = [&](int x) { return d == 4 && swapped ? (x >> 1) | (x & 1) << 1 : x; };
+                const int br = basis(r), bc = basis(c);
+                const int e = diag ? 2 * br + z : 2 * (br * d + bc) + z;
+                msrc[nmat++] = diag && r != c ? kStageZero : off >= 0 ? off + e : off - e;
+              }
+        };
+        if (smat == 4) put(op.moff, 4);
+        else if (smat) full(op.moff, smat == 8 ? 2 : 4, op.kind == OK_D1 || op.kind == OK_D2);
+        if (trains(&op)) {
+          w1 |= (uint32_t)op.gen << 8;
+          gm = nmat;
+          if (gmat) full(-op.goff - 1, gmat == 8 ? 2 : 4, false);
+          blob[kStageGl + ngl++] = (uint32_t)op.gloc;
+        }
+      }
+      uint32_t* w = blob + kStageOps + 4 * nop++;
+      w[0] = w0;
+      w[1] = w1;
+      w[2] = (uint32_t)m0 | (uint32_t)gm << 16;
+      ++blob[2 * (nseg - 1) + 1];
+      M = MacroOp();
+    };
+    // places in a macro op's order: forward ry 0, rx 1, diagonal 2, CX 3..14,
+    // single 15; adjoint CX 0..11, members and diagonal 12, rx 13, ry 14,
+    // single 15
+    const int st_ry = adj ? 14 : 0, st_rx = adj ? 13 : 1, st_dg = adj ? 12 : 2, st_cx = adj ? 0 : 3;
+    std::vector<const DOp*> list;
+    for (int oi = 0; oi < dg.nops; ++oi) list.push_back(&S.dop[dg.op0 + (adj ? dg.nops - 1 - oi : oi)]);
+    // permutation gates that end the group: image of each register index
+    size_t nlist = list.size();
+    while (nlist > 0) {
+      const int k = list[nlist - 1]->kind;
+      if (k != OK_X1 && k != OK_CX && k != OK_SWAP) break;
+      --nlist;
+    }
+    auto image = [&](uint32_t i) {
+      for (size_t t = nlist; t < list.size(); ++t) {
+        const DOp& o = *list[t];
+        if (o.kind == OK_X1) i ^= 1u << o.s0;
+        else if (o.kind == OK_CX) i ^= ((i >> o.s0) & 1u) << o.s1;
+        else {
+          const uint32_t d = ((i >> o.s0) ^ (i >> o.s1)) & 1u;
+          i ^= d << o.s0 | d << o.s1;
+        }
+      }
+      return i;
+    };
+    for (size_t t = 0; t < nlist; ++t) {
+      const DOp& op = *list[t];
+      if (op.kind == OK_DG) {
+        int m0 = op.mem0, nm = adj ? op.nmem : 0;
+        for (; nm > 16; m0 += 16, nm -= 16) {  // more members than one op takes: ops of their own first
+          flush();
+          M.m0 = m0;
+          M.nm = 16;
+          M.stage = st_dg;
+          flush();
+        }
+        if (M.stage >= st_dg) flush();
+        M.dg = &op;
+        M.m0 = m0;
+        M.nm = nm;
+        M.stage = st_dg;
+      } else if (op.flags & (OP_F_SHEAR | OP_F_RX)) {
+        const bool ry = op.flags & OP_F_SHEAR;
+        const int st = ry ? st_ry : st_rx;
+        if (M.stage > st || (ry ? M.ry : M.rx)[op.s0]) flush();
+        (ry ? M.ry : M.rx)[op.s0] = &op;
+        M.stage = st;
+      } else if (op.kind == OK_CX) {
+        const int i = cx_index(op.s0, op.s1);
+        if (M.stage >= st_cx + i) flush();
+        M.cx |= 1u << i;
+        M.stage = st_cx + i;
+      } else {
+        if (M.stage >= 15) flush();
+        M.single = &op;
+        M.stage = 15;
+      }
+    }
+    flush();
+    if (nlist < list.size()) {
+      segment();
+      const uint32_t c = image(0);
+      uint32_t perm = c << 24;
+      for (int s = 0; s < kTileSlots; ++s) perm |= (image(1u << s) ^ c) << (8 + 4 * s);
+      blob[2 * (nseg - 1) + 1] = (blob[2 * (nseg - 1) + 1] & 0xffu) | perm;
+    }
+  }
+  close();
+  dp.nchunk = (int)(S.blob.size() / kStageBlob) - dp.chunk0;
+}
+
 // Consecutive dense 5-qubit gates (matrix-core blocks) grouped into tile
 // passes: each pass stages a tile of kM bits (the low Lwant index bits plus
 // the blocks' qubits) and applies its blocks in order from LDS.
@@ -913,7 +1141,7 @@ static void mfma_tile_run(const Program& P, Sched& S, const std::vector<int>& it
   }
 }
 
-static void sched_fused(const Program& P, Sched& S, int k, int R, int Lwant, bool mfma_tiles) {
+static void sched_fused(const Program& P, Sched& S, int k, int R, int Lwant, bool mfma_tiles, bool adj) {
   const int n = P.n;
   k = std::min(k, n);
   S.k = k;
@@ -1084,9 +1312,10 @@ static void sched_fused(const Program& P, Sched& S, int k, int R, int Lwant, boo
       }
       build_group_ops(P, S, hg, local_of_bit, gloc_of_gop, dg);
       for (int o = dg.op0; o < dg.op0 + dg.nops; ++o)
-        if (S.dop[o].kind == OK_U2 || S.dop[o].gen == GN_M2) dp.full = 1;
+        if (S.dop[o].kind == OK_U2 || (R == kTileSlots && S.dop[o].kind == OK_D2) || S.dop[o].gen == GN_M2) dp.full = 1;
       S.dgroup.push_back(dg);
     }
+    if (R == kTileSlots) stage_pass(S, hp, dp, adj);
     S.dpass.push_back(dp);
   }
 }
@@ -1144,26 +1373,29 @@ int build_program(const tcm_gate* gates, int32_t ngates, int32_t n, int32_t npar
     // 4 otherwise (1024 x 16-qubit batch: 4.80 ms with 4, 5.59 ms with 5)
     const int R = o.reg_slots ? o.reg_slots : ((o.jit && dt == 0 && n >= 20) ? 5 : 4);
     const int Lw = dt == 0 ? 4 : 3;
-    // defaults measured on MI355X: 32 KiB forward tiles (several blocks per
-    // CU overlap HBM and compute); the generic adjoint holds two tiles.
-    // Compiled passes (jit) hold fewer registers and take 64 KiB tiles, and
-    // their adjoint stages psi and lambda through one tile: fewer passes at
-    // about the same per-pass bandwidth (24-qubit HEA: 44 + 44 passes
-    // instead of 56 + 68)
-    int kf = o.tile_bits > 0 ? o.tile_bits : (dt == 0 ? 12 : 11) + (o.jit ? 1 : 0);
-    int ka = o.adj_tile_bits > 0 ? o.adj_tile_bits : (o.jit ? (dt == 0 ? 13 : 12) : (dt == 0 ? 11 : 10));
+    // 32 KiB tiles in the table-driven passes (several blocks per CU overlap
+    // HBM and compute), both ways: the adjoint stages psi and lambda through
+    // one tile.  Compiled passes hold fewer registers and take 64 KiB tiles:
+    // fewer passes at about the same per-pass bandwidth (24-qubit HEA: 44 +
+    // 44 passes instead of 56 + 68)
+    const int kd = (dt == 0 ? 12 : 11) + (o.jit ? 1 : 0);
+    int kf = o.tile_bits > 0 ? o.tile_bits : kd;
+    int ka = o.adj_tile_bits > 0 ? o.adj_tile_bits : kd;
     // a tile must fit one CU's 160 KiB of LDS with room for the adjoint's
     // partial sums: 2^14 complex64 or 2^13 complex128 amplitudes (128 KiB)
     const int kmax = dt == 0 ? 14 : 13;
     kf = std::min(kf, kmax);
     ka = std::min(ka, kmax);
-    // fused passes need at least one full wave (64 threads) per tile
+    // tile passes need a full wave (64 threads) per tile, but states of 4 to
+    // 9 qubits are one tile of the table-driven kernels, with idle lanes: one
+    // launch instead of one per gate
     bool fused = o.fuse != 0 && n >= R + 6;
+    const bool small = o.fuse != 0 && R == kTileSlots && n >= kTileSlots && n < R + 6;
     for (int mode = 0; mode < 2; ++mode) {
       Sched& S = P->sched[dt][mode];
       int k = mode == 0 ? kf : ka;
-      if (fused && std::min(k, n) >= R + 6 && k >= std::min(n, Lw + 5)) {
-        sched_fused(*P, S, k, R, Lw, dt == 0 && mode == 0 && o.mfma == 2);
+      if (small || (fused && std::min(k, n) >= R + 6 && k >= std::min(n, Lw + 5))) {
+        sched_fused(*P, S, small ? n : k, R, Lw, dt == 0 && mode == 0 && o.mfma == 2, mode == 1);
       } else {
         sched_plain(*P, S);
       }

@@ -29,7 +29,7 @@ enum OpKind : int32_t {
   OK_CZ = 7,    // no matrix
   OK_SWAP = 8,  // no matrix
   OK_DG = 9,    // fused diagonal over a register group
-  OK_UK = 10,   // dense k-qubit, k = 3..5 (applied directly on the LDS tile)
+  OK_UK = 10,   // dense k-qubit, k = 3..5
   OK_NKINDS
 };
 
@@ -67,7 +67,8 @@ struct DOp {
 // DOp flags
 // OP_F_SHEAR: an ry rotation whose table entry also holds the three-shear
 // form of its reduced angle (see k_prep): entries 4, 5, 6 = t, s, sigma
-enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2 };
+// OP_F_RX: an rx rotation
+enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2, OP_F_RX = 4 };
 
 // Gradient member of an OK_DG op (diagonal generator on slots of the group).
 struct DMember {
@@ -93,6 +94,35 @@ struct DGroup {
 // LDS with the tile: 8 KiB each)
 constexpr int kMfmaTileMaxOps = 8;
 
+// Staged tables of the table-driven tile passes (tile_pass.hip): a pass's
+// segments in processing order (reversed for the adjoint), cut into chunks of
+// a fixed size that one block copies into LDS at a time.
+//   blob words per chunk: [segments, 2 words each][ops, 2 words each]
+//     [members][gradient indices][segment count, gradient count]
+//   segment: tile bit of slot s at bits 4s, the same four ascending at bits
+//     16 + 4i; then its number of ops, at bits 8 + 4s the slots that register
+//     bit s is written to and at bits 24..27 a constant added to them (the
+//     permutation gates that end the segment)
+//   op: a macro op, up to one op of each kind below, run in this order (the
+//   adjoint: CX, members, diagonal, rx, ry, single)
+//     word 0: ry slots (4 bits) | rx slots << 4 | CX mask << 8 | (OpKind of
+//       the single op + 1) << 20 | s0 << 24 | s1 << 26 | diagonal << 28
+//     word 1: ry slots with a gradient | rx ones << 4 | single's GenKind << 8
+//       | members << 12 | first member << 20
+//     word 2: first matrix entry | single's generator matrix << 16
+//     matrices follow each other in the order they are used: 4 entries per
+//     rotation (the first of its matrix), 32 for the diagonal, then the single op's
+//   member: gen | s0 << 4 | s1 << 7
+// msrc: for each staged matrix entry its offset in the item's table, or
+// -1 - offset in the constant table, or kStageNone / kStageZero.
+// 24 ops, 304 entries and 32 gradients keep a 32 KiB tile, its tables and
+// the adjoint's reduction buffers within a quarter of a CU's 160 KiB.
+constexpr int kTileSlots = 4;
+constexpr int kStageSegs = 32, kStageMaxOps = 24, kStageGrad = 32, kStageMat = 304;
+constexpr int kStageOps = 2 * kStageSegs, kStageMems = kStageOps + 4 * kStageMaxOps,
+              kStageGl = kStageMems + kStageGrad, kStageCount = kStageGl + kStageGrad, kStageBlob = kStageCount + 2;
+constexpr int32_t kStageNone = INT32_MIN, kStageZero = INT32_MIN + 1;
+
 struct DPass {
   int32_t k;          // tile bits
   int32_t L;          // contiguous low bits inside the tile (run length 2^L)
@@ -107,6 +137,7 @@ struct DPass {
   int32_t blk_bits[32];  // global bit positions of the block bits (ascending)
   int32_t mfma;       // 1: a tile pass of dense 5-qubit blocks on FP32 matrix cores
   int32_t mop0, nmop; // its blocks: Sched::dop entries (OK_UK, tile-local bits)
+  int32_t chunk0, nchunk;  // staged tables (4 register slots)
   int32_t pad;
 };
 
@@ -197,6 +228,8 @@ struct Sched {
   std::vector<DMember> dmem;
   std::vector<int32_t> ukbits;  // bit tables of OK_UK ops
   std::vector<uint32_t> runoff;
+  std::vector<uint32_t> blob;   // staged tables, kStageBlob words per chunk
+  std::vector<int32_t> msrc;    // staged tables, kStageMat entries per chunk
   std::vector<DRecipe> recipes; // base recipes + DG recipes of this schedule
   std::vector<DFactor> factors;
   int32_t mtab_size = 0;        // per-batch matrix table size (T units)

@@ -54,3 +54,95 @@ def test_pauli_tile(gpu, n, T, letters):
             assert abs(e[b] - sv.pauli_sum_expectation(sd[b], n, terms)) <= tol
             ref = alpha[b] * sv.pauli_sum_apply(sd[b], n, terms)
             assert np.abs(hs[b] - ref).max() <= 2.0 * tol
+
+
+def _long_runs(n):
+    """Runs that overflow one staged chunk or one staged op: 45 merged
+    diagonals (27 trainable) on four qubits, 40 rotations of one qubit,
+    every CX order, and permutation gates before, between and after them."""
+    ops = []
+    for i in range(27):
+        ops.append(("rz" if i % 3 else "rzz", (i % 4,) if i % 3 else (i % 4, (i + 1) % 4), 0.1 + 0.05 * i))
+    ops += [("cz", (0, 1), 0.0), ("s", (2,), 0.0), ("t", (3,), 0.0)] * 6
+    ops += [(("ry", "rx")[i % 2], (i % 2,), 0.3 - 0.02 * i) for i in range(40)]
+    ops += [("cnot", (a, b), 0.0) for a in range(4) for b in range(4) if a != b]
+    ops += [("ry", (q,), 0.2 * (q + 1)) for q in range(n)]
+    ops += [("swap", (0, n - 1), 0.0), ("x", (1,), 0.0), ("cnot", (n - 1, 0), 0.0), ("swap", (3, 1), 0.0)]
+    return ops
+
+
+# states smaller than a wave of threads, one tile, a tile and more; few gates
+# and enough to fill several chunks of staged tables
+@pytest.mark.parametrize("n,gates", [(4, 12), (4, 0), (5, 30), (7, 60), (9, 25), (10, 0), (11, 90), (12, 400), (13, 0),
+                                     (14, 120)])
+def test_tile_pass(gpu, n, gates):
+    import tensorcircuit_amd as tc
+    from tensorcircuit_amd import engine
+    from test_gpu_jit import _circuit, _random_ops, _terms
+
+    rng = np.random.default_rng(31 * n + gates)
+    ops = _random_ops(rng, n, gates) if gates else _long_runs(n)
+    c, oops = _circuit(tc, n, ops)
+    specs, thetas = c._lower()
+    terms = _terms(rng, n, 5)
+    wsum = sum(abs(t[0]) for t in terms)
+    ham = engine.PauliSum(n, [t[1] for t in terms], [t[0] for t in terms], jit=0)
+    prog = engine.Program(n, specs, len(thetas), fuse=1, jit=0)
+    B = 3
+    params = np.array([float(np.real(t)) for t in thetas])[None, :] + rng.normal(0, 0.3, size=(B, len(thetas)))
+    inputs = random_states(rng, B, n)
+    for dt in DTYPES:
+        name = str(dt).split(".")[1]
+        p = torch.as_tensor(params).to(torch.float32 if dt == torch.complex64 else torch.float64).cuda()
+        pd = np_of(p).astype(np.float64)
+        # each gate turns a unit state with a few roundings
+        tol = 8 * (len(ops) + 4) * UNIT[dt]
+        st, _ = prog.forward(p, B, name)
+        e, g = prog.energy_grad(p, ham, B, name)
+        si = torch.as_tensor(inputs).to(dt).cuda()
+        gs = torch.as_tensor(inputs[::-1].copy()).to(dt).cuda()
+        out, _ = prog.forward(p, B, name, inputs=si)
+        gp, gi = prog.vjp(p, None, out, gs, B, name, True)
+        for b in range(B):
+            assert np.abs(np_of(st)[b] - sv.run_ops(n, oops, pd[b])).max() <= tol
+            e_ref, g_ref = sv.adjoint_value_and_grad(n, oops, pd[b], terms)
+            assert abs(float(e[b]) - e_ref) <= 2 * tol * wsum
+            assert np.abs(np_of(g)[b] - g_ref).max() <= 4 * tol * wsum
+            # U^dagger of the output's cotangent, and of the output itself
+            ref = sv.run_ops(n, oops, pd[b], inputs[b])
+            assert np.abs(np_of(out)[b] - ref).max() <= 2 * tol
+            lhs = np.vdot(np_of(gs)[b].astype(np.complex128), ref)
+            rhs = np.vdot(np_of(gi)[b].astype(np.complex128), inputs[b])
+            assert abs(lhs - rhs) <= 4 * tol
+        assert torch.isfinite(gp).all()
+
+
+def test_tile_pass_multi(gpu):
+    """Programs of 3 (per-gate), 4, 7, 9, 12 and 13 qubits in shared launches
+    against single runs, from |0..0> and from given states."""
+    import tensorcircuit_amd as tc
+    from tensorcircuit_amd import engine
+    from test_gpu_jit import _circuit, _random_ops
+
+    rng = np.random.default_rng(77)
+    for dt in DTYPES:
+        name = str(dt).split(".")[1]
+        rdt = torch.float32 if dt == torch.complex64 else torch.float64
+        items, ref = [], []
+        start = []
+        for n, B in ((3, 2), (4, 5), (7, 1), (9, 70), (12, 3), (13, 2)):
+            ops = _random_ops(rng, n, 10 * n)
+            c, oops = _circuit(tc, n, ops)
+            specs, thetas = c._lower()
+            prog = engine.Program(n, specs, len(thetas), fuse=1, jit=0)
+            p = torch.as_tensor(rng.uniform(0, 6, size=(B, len(thetas)))).to(rdt).cuda()
+            start.append(torch.as_tensor(random_states(rng, B, n)).to(dt).cuda())
+            items.append((prog, p, torch.empty(B, 1 << n, dtype=dt, device="cuda")))
+        for zero in (True, False):
+            if not zero:
+                for it, s in zip(items, start):
+                    it[2].copy_(s)
+            engine.forward_multi(items, name, init_zero=zero)
+            for (prog, p, st), s in zip(items, start):
+                one, _ = prog.forward(p, p.shape[0], name, inputs=None if zero else s)
+                assert torch.equal(st, one)
