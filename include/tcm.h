@@ -267,6 +267,16 @@ int tcm_csr_expect(int32_t nqubits, int32_t dtype, const int64_t* rowptr,
 int tcm_csr_matvec(int32_t nqubits, int32_t dtype, const int64_t* rowptr,
                    const int64_t* cols, const void* vals, const void* x,
                    void* y, int64_t batch, void* stream);
+/* y_b = conj(g_b) A x_b + g_b A^dagger x_b, the vector-Jacobian product of
+ * x -> <x|A|x> (g in the state's complex type, one per state, on the
+ * device).  dag_*: the CSR form of A^dagger, all three, or all null where
+ * A = A^dagger (then y_b = 2 Re(g_b) A x_b). */
+int tcm_csr_expect_vjp(int32_t nqubits, int32_t dtype, const int64_t* rowptr,
+                       const int64_t* cols, const void* vals,
+                       const int64_t* dag_rowptr, const int64_t* dag_cols,
+                       const void* dag_vals, const void* x, const void* g,
+                       void* y, int64_t batch, void* stream);
+
 
 /* out[b] = <a_b|b_b> (complex fp64) -- expectation of general operators after
  * they were applied to a copy of the state (circuit.py:914-990). */

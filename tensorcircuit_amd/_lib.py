@@ -100,6 +100,7 @@ SIGNATURES = {
     "tcm_expect_pauli_terms": (C.c_int, [_vp, _i32, _vp, _i64, _vp, _vp, _i64, _vp]),
     "tcm_apply_pauli_terms": (C.c_int, [_vp, _i32, _vp, _vp, _i64, _vp, _vp]),
     "tcm_csr_matvec": (C.c_int, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "tcm_csr_expect_vjp": (C.c_int, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "tcm_inner_workspace_bytes": (C.c_int, [_i32, _i64, C.POINTER(_i64)]),
     "tcm_inner": (C.c_int, [_i32, _i32, _vp, _vp, _i64, _vp, _vp, _i64, _vp]),
     "tcm_probability": (C.c_int, [_i32, _i32, _vp, _i64, _vp, _vp]),

@@ -1337,10 +1337,6 @@ int tcm_pauli_coo(const tcm_pauli* ham, int32_t dtype, int64_t* rows, int64_t* c
   return 0;
 }
 
-namespace {
-constexpr int kCsrBlocks = 1024;
-}
-
 int tcm_csr_expect_workspace_bytes(int32_t n, int64_t* bytes) {
   if (!bytes || n < 1 || n > 40) return set_error(TCM_E_ARG, "bad arguments to tcm_csr_expect_workspace_bytes");
   *bytes = 2 * kCsrBlocks * (int64_t)sizeof(double);
@@ -1354,11 +1350,10 @@ int tcm_csr_expect(int32_t n, int32_t dtype, const int64_t* rowptr, const int64_
   if (ws_bytes < 2 * kCsrBlocks * (int64_t)sizeof(double)) return set_error(TCM_E_WORKSPACE, "workspace too small");
   hipStream_t st = (hipStream_t)stream;
   const int64_t nrows = (int64_t)1 << n;
-  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(kCsrBlocks, nrows / 256));
   if (dtype == TCM_C64)
-    launch_csr_expect<float>(rowptr, cols, vals, state, nrows, nblk, (double*)workspace, out, st);
+    launch_csr_expect<float>(rowptr, cols, vals, state, nrows, (double*)workspace, out, st);
   else
-    launch_csr_expect<double>(rowptr, cols, vals, state, nrows, nblk, (double*)workspace, out, st);
+    launch_csr_expect<double>(rowptr, cols, vals, state, nrows, (double*)workspace, out, st);
   HIP_TRY(hipGetLastError(), "csr_expect launch");
   return 0;
 }
@@ -1447,6 +1442,24 @@ int tcm_csr_matvec(int32_t n, int32_t dtype, const int64_t* rowptr, const int64_
   else
     launch_csr_matvec<double>(rowptr, cols, vals, x, y, nrows, batch, st);
   HIP_TRY(hipGetLastError(), "csr_matvec launch");
+  return 0;
+}
+
+int tcm_csr_expect_vjp(int32_t n, int32_t dtype, const int64_t* rowptr, const int64_t* cols, const void* vals,
+                       const int64_t* dag_rowptr, const int64_t* dag_cols, const void* dag_vals, const void* x,
+                       const void* g, void* y, int64_t batch, void* stream) {
+  if (n < 1 || n > 40 || !valid_dtype(dtype) || batch < 0 ||
+      (batch > 0 && (!rowptr || !cols || !vals || !x || !g || !y)) || x == y ||
+      (dag_rowptr != nullptr) != (dag_cols != nullptr) || (dag_rowptr != nullptr) != (dag_vals != nullptr))
+    return set_error(TCM_E_ARG, "bad arguments to tcm_csr_expect_vjp");
+  if (batch == 0) return 0;
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t nrows = (int64_t)1 << n;
+  if (dtype == TCM_C64)
+    launch_csr_vjp<float>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, nrows, batch, st);
+  else
+    launch_csr_vjp<double>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, nrows, batch, st);
+  HIP_TRY(hipGetLastError(), "csr_expect_vjp launch");
   return 0;
 }
 

@@ -211,7 +211,7 @@ void launch_probability(const void* psi, void* out, int64_t total, hipStream_t s
 template <typename T>
 void launch_pauli_coo(const DPGroup* groups, int ngroups, const DPTerm* terms, int n, int64_t nterms, int64_t* rows,
                       int64_t* cols, void* vals, hipStream_t st);
-// per-term Pauli expectations and weighted applications, CSR mat-vec
+// per-term Pauli expectations and weighted applications
 // (kernels_aux.hip)
 template <typename T>
 void launch_pauli_terms(const DPTermF* terms_dev, int nterms, int n, const void* psi, int64_t batch, int nblk,
@@ -219,12 +219,18 @@ void launch_pauli_terms(const DPTermF* terms_dev, int nterms, int n, const void*
 template <typename T>
 void launch_pauli_terms_apply(const DPTermF* terms_dev, int nterms, int n, const void* psi, void* out,
                               const double* weights, int64_t batch, hipStream_t st);
+// CSR matrices (csr.hip); drowptr null: A = A^dagger
+constexpr int kCsrBlocks = 2048;  // most blocks, and partial sums, of a launch
 template <typename T>
 void launch_csr_matvec(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* x, void* y,
                        int64_t nrows, int64_t batch, hipStream_t st);
 template <typename T>
+void launch_csr_vjp(const int64_t* rowptr, const int64_t* cols, const void* vals, const int64_t* drowptr,
+                    const int64_t* dcols, const void* dvals, const void* x, const void* g, void* y, int64_t nrows,
+                    int64_t batch, hipStream_t st);
+template <typename T>
 void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* psi, int64_t nrows,
-                       int nblk, double* part, double* out, hipStream_t st);
+                       double* part, double* out, hipStream_t st);
 // src: states [batch][2^n] (prob false) or probability vectors (prob true)
 template <typename T>
 void launch_sample(const void* src, bool prob, int n, int64_t batch, const double* u, int64_t shots, int64_t* out,

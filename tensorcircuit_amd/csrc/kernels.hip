@@ -1243,8 +1243,7 @@ void launch_measure_step(const void* psi, int n, int64_t batch, const MeasureSte
 
 // ---------------------------------------------------------------------------
 // Sparse form of a Pauli sum (PauliStringSum2COO / ps2coo_core,
-// quantum.py:1304-1485) and <psi|H|psi> over a CSR matrix
-// (sparse_expectation, templates/measurements.py:177-191).
+// quantum.py:1304-1485).
 // ---------------------------------------------------------------------------
 // entry t * N + y of term t (group g): row y, column y ^ flip,
 // value w (-i)^ny (-1)^popc(y & yz); grid-stride over nterms * N
@@ -1273,46 +1272,12 @@ __global__ void k_pauli_coo(const DPGroup* __restrict__ groups, int ngroups, con
   }
 }
 
-// part[blk] = sum over rows r of this block's grid-stride share of
-// conj(psi_r) * sum_k vals_k psi_{cols_k} (fp64); one thread per row
-template <typename T>
-__global__ void __launch_bounds__(256) k_csr_expect(const int64_t* __restrict__ rowptr, const int64_t* __restrict__ cols,
-                                                    const V2<T>* __restrict__ vals, const V2<T>* __restrict__ psi,
-                                                    int64_t nrows, double* __restrict__ part) {
-  double er = 0.0, ei = 0.0;
-  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * blockDim.x) {
-    double hr = 0.0, hi = 0.0;
-    for (int64_t k = rowptr[r]; k < rowptr[r + 1]; ++k) {
-      const V2<T> v = vals[k], x = psi[cols[k]];
-      hr += (double)v.x * x.x - (double)v.y * x.y;
-      hi += (double)v.x * x.y + (double)v.y * x.x;
-    }
-    const V2<T> p = psi[r];
-    er += (double)p.x * hr + (double)p.y * hi;
-    ei += (double)p.x * hi - (double)p.y * hr;
-  }
-  block_sum2(er, ei);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = er;
-    part[2 * blockIdx.x + 1] = ei;
-  }
-}
-
 template <typename T>
 void launch_pauli_coo(const DPGroup* groups, int ngroups, const DPTerm* terms, int n, int64_t nterms, int64_t* rows,
                       int64_t* cols, void* vals, hipStream_t st) {
   const int64_t total = nterms << n;
   hipLaunchKernelGGL(k_pauli_coo<T>, dim3(grid_for(total)), dim3(256), 0, st, groups, ngroups, terms, n, rows, cols,
                      (V2<T>*)vals, total);
-}
-
-template <typename T>
-void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* psi, int64_t nrows,
-                       int nblk, double* part, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_csr_expect<T>, dim3((unsigned)nblk), dim3(256), 0, st, rowptr, cols, (const V2<T>*)vals,
-                     (const V2<T>*)psi, nrows, part);
-  hipLaunchKernelGGL(k_sum_slots, dim3(1), dim3(256), 0, st, (const double*)part, (int64_t)2 * nblk, (int64_t)nblk, 2,
-                     out);
 }
 
 // explicit instantiations used by engine.cpp
@@ -1338,9 +1303,7 @@ void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* v
   template void launch_measure_step<T>(const void*, int, int64_t, const MeasureStep&, int, int, const double*,  \
                                        uint64_t*, double*, double*, double*, int, hipStream_t);                \
   template void launch_pauli_coo<T>(const DPGroup*, int, const DPTerm*, int, int64_t, int64_t*, int64_t*, void*,  \
-                                    hipStream_t);                                                              \
-  template void launch_csr_expect<T>(const int64_t*, const int64_t*, const void*, const void*, int64_t, int,      \
-                                     double*, double*, hipStream_t);
+                                    hipStream_t);
 
 TCM_INST(float)
 TCM_INST(double)

@@ -3,9 +3,7 @@
 //    behind any_measurements / parameterized_local_measurements over many
 //    structures at once (templates/measurements.py:18-153);
 //  - weighted Pauli applications  out_b = sum_t a[b][t] w_t P_t psi_b, the
-//    vector-Jacobian product of those expectations;
-//  - CSR mat-vec  y_b = A x_b, the vector-Jacobian product of
-//    sparse_expectation (templates/measurements.py:177-191).
+//    vector-Jacobian product of those expectations.
 //
 // Pauli action (index rule of ps2coo_core, quantum.py:1461-1485):
 //   (P psi)[a] = (-i)^ny (-1)^popcount(a & yz) psi[a ^ flip].
@@ -139,26 +137,6 @@ __global__ void __launch_bounds__(256) k_pauli_terms_apply(const DPTermF* __rest
   }
 }
 
-// y_b[r] = sum_k vals[k] x_b[cols[k]] over row r of a CSR matrix (fp64
-// accumulation); one thread per (b, r)
-template <typename T>
-__global__ void __launch_bounds__(256) k_csr_matvec(const int64_t* __restrict__ rowptr,
-                                                    const int64_t* __restrict__ cols, const V2<T>* __restrict__ vals,
-                                                    const V2<T>* __restrict__ x, V2<T>* __restrict__ y,
-                                                    int64_t nrows, int64_t total) {
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t b = i / nrows, r = i - b * nrows;
-    const V2<T>* xb = x + b * nrows;
-    double hr = 0.0, hi = 0.0;
-    for (int64_t k = rowptr[r]; k < rowptr[r + 1]; ++k) {
-      const V2<T> v = vals[k], q = xb[cols[k]];
-      hr += (double)v.x * q.x - (double)v.y * q.y;
-      hi += (double)v.x * q.y + (double)v.y * q.x;
-    }
-    y[i] = make2<T>((T)hr, (T)hi);
-  }
-}
-
 namespace {
 unsigned grid_of(int64_t total) {
   int64_t g = (total + 255) / 256;
@@ -184,21 +162,11 @@ void launch_pauli_terms_apply(const DPTermF* terms_dev, int nterms, int n, const
                      (const V2<T>*)psi, (V2<T>*)out, weights, total);
 }
 
-template <typename T>
-void launch_csr_matvec(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* x, void* y,
-                       int64_t nrows, int64_t batch, hipStream_t st) {
-  const int64_t total = batch * nrows;
-  hipLaunchKernelGGL(k_csr_matvec<T>, dim3(grid_of(total)), dim3(256), 0, st, rowptr, cols, (const V2<T>*)vals,
-                     (const V2<T>*)x, (V2<T>*)y, nrows, total);
-}
-
 #define TCM_AUX_INST(T)                                                                                       \
   template void launch_pauli_terms<T>(const DPTermF*, int, int, const void*, int64_t, int, double*, double*,  \
                                       hipStream_t);                                                           \
   template void launch_pauli_terms_apply<T>(const DPTermF*, int, int, const void*, void*, const double*,      \
-                                            int64_t, hipStream_t);                                            \
-  template void launch_csr_matvec<T>(const int64_t*, const int64_t*, const void*, const void*, void*, int64_t, \
-                                     int64_t, hipStream_t);
+                                            int64_t, hipStream_t);
 
 TCM_AUX_INST(float)
 TCM_AUX_INST(double)

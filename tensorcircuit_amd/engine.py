@@ -672,6 +672,10 @@ class CsrMatrix:
         dag = torch.sparse_coo_tensor(torch.stack([idx[1], idx[0]]), torch.conj(coo.values()).resolve_conj(),
                                       (N, N)).coalesce()
         self.dag = self._csr(dag)
+        # A = A^dagger entry for entry: one copy serves both
+        self.hermitian = all(a.shape == b.shape and bool(torch.equal(a, b)) for a, b in zip(self.fwd, self.dag))
+        if self.hermitian:
+            self.dag = self.fwd
 
     @staticmethod
     def _csr(h: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -690,7 +694,7 @@ class CsrMatrix:
         ws = _workspace(nb.value, s.device)
         check(lib.tcm_csr_expect(self.n, code, rowptr.data_ptr(), cols.data_ptr(), vals.data_ptr(), s.data_ptr(),
                                  out.data_ptr(), ws.data_ptr(), ws.numel(), _stream()), "tcm_csr_expect")
-        return torch.complex(out[0], out[1])
+        return torch.view_as_complex(out)
 
     def matvec(self, x: torch.Tensor, dagger: bool = False) -> torch.Tensor:
         """A x_b (or A^dagger x_b) for x [batch, 2^n] (tcm_csr_matvec)."""
@@ -700,6 +704,20 @@ class CsrMatrix:
         out = torch.empty_like(s)
         check(lib.tcm_csr_matvec(self.n, code, rowptr.data_ptr(), cols.data_ptr(), vals.data_ptr(), s.data_ptr(),
                                  out.data_ptr(), s.shape[0], _stream()), "tcm_csr_matvec")
+        return out
+
+    def vjp(self, x: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
+        """conj(g_b) A x_b + g_b A^dagger x_b for x [batch, 2^n], g [batch] in
+        x's dtype, from one launch (tcm_csr_expect_vjp)."""
+        _hold(self)
+        s, code = _states(x, self.n)
+        gg = g.to(device=s.device, dtype=s.dtype).reshape(s.shape[0]).resolve_conj().contiguous()
+        rowptr, cols, vals = self.fwd
+        dag = (None, None, None) if self.hermitian else self.dag
+        out = torch.empty_like(s)
+        check(lib.tcm_csr_expect_vjp(self.n, code, rowptr.data_ptr(), cols.data_ptr(), vals.data_ptr(),
+                                     _ptr(dag[0]), _ptr(dag[1]), _ptr(dag[2]), s.data_ptr(), gg.data_ptr(),
+                                     out.data_ptr(), s.shape[0], _stream()), "tcm_csr_expect_vjp")
         return out
 
 
@@ -974,7 +992,7 @@ class OpExpFn(torch.autograd.Function):
 class CsrExpFn(torch.autograd.Function):
     """psi [N] -> <psi|A|psi> for a sparse A (complex, the state dtype);
     dL/dpsi = conj(g) A psi + g A^dagger psi (the same convention as
-    OpExpFn), both products by the CSR mat-vec kernel."""
+    OpExpFn), both products by one CSR launch."""
 
     @staticmethod
     def forward(st, m):
@@ -1001,9 +1019,7 @@ class CsrExpFn(torch.autograd.Function):
 class CsrVJPFn(torch.autograd.Function):
     @staticmethod
     def forward(st, g, m):
-        s = st.reshape(1, -1)
-        gg = g.to(st.dtype).reshape(())
-        return (torch.conj(gg) * m.matvec(s) + gg * m.matvec(s, dagger=True)).reshape(st.shape)
+        return m.vjp(st.reshape(1, -1), g).reshape(st.shape)
 
     @staticmethod
     def setup_context(ctx, inputs, output):
@@ -1018,8 +1034,7 @@ class CsrVJPFn(torch.autograd.Function):
         B = info.batch_size
         N = 1 << m.n
         s = _to_batch(st, in_dims[0], B, (N,))
-        gg = _to_batch(g, in_dims[1], B, ()).to(s.dtype).reshape(B, 1)
-        return torch.conj(gg) * m.matvec(s) + gg * m.matvec(s, dagger=True), 0
+        return m.vjp(s, _to_batch(g, in_dims[1], B, ())), 0
 
 
 class PauliTermsFn(torch.autograd.Function):

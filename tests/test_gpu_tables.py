@@ -146,3 +146,38 @@ def test_tile_pass_multi(gpu):
             for (prog, p, st), s in zip(items, start):
                 one, _ = prog.forward(p, p.shape[0], name, inputs=None if zero else s)
                 assert torch.equal(st, one)
+
+
+# rows of no entry, one, a few and many (a group of lanes per row from 1 to
+# 64); Hermitian or not
+@pytest.mark.parametrize("n,mean,hermitian", [(1, 1, True), (3, 2, False), (6, 0.3, False), (7, 30, True),
+                                              (9, 5, False), (9, 200, False), (11, 12, True)])
+def test_csr(gpu, n, mean, hermitian):
+    from tensorcircuit_amd import engine
+
+    rng = np.random.default_rng(int(100 * n + mean))
+    N = 1 << n
+    m = (rng.standard_normal((N, N)) + 1j * rng.standard_normal((N, N))) * (rng.random((N, N)) < mean / N)
+    m[N // 2] = 0
+    if N > 2:
+        m[1] = rng.standard_normal(N)  # a full row
+    if hermitian:
+        m = m + m.conj().T
+    x = random_states(rng, 3, n)
+    g = rng.standard_normal(3) + 1j * rng.standard_normal(3)
+    for dt in DTYPES:
+        c = engine.CsrMatrix(torch.as_tensor(m).to(dt).cuda().to_sparse_csr(), n, dt)
+        assert c.hermitian == hermitian
+        xd, gd = torch.as_tensor(x).to(dt).cuda(), torch.as_tensor(g).to(dt).cuda()
+        mr, xr, gr = (np_of(torch.as_tensor(v).to(dt)).astype(np.complex128) for v in (m, x, g))
+        # sums in fp64; the result is rounded once
+        tol = 4 * UNIT[dt] * np.abs(mr).sum(axis=1).max()
+        ax, dx = xr @ mr.T, xr @ mr.conj()
+        assert np.abs(np_of(c.matvec(xd)) - ax).max() <= tol
+        assert np.abs(np_of(c.matvec(xd, dagger=True)) - dx).max() <= tol
+        ref = gr.conj()[:, None] * ax + gr[:, None] * dx
+        assert np.abs(np_of(c.vjp(xd, gd)) - ref).max() <= 8 * tol
+        # a lazily conjugated cotangent
+        assert np.abs(np_of(c.vjp(xd, torch.conj(gd))) - (gr[:, None] * ax + gr.conj()[:, None] * dx)).max() <= 8 * tol
+        for b in range(3):
+            assert abs(complex(c.expect(xd[b])) - np.vdot(xr[b], ax[b])) <= max(tol, 1e-12) * np.sqrt(N)
