@@ -1195,10 +1195,11 @@ int tcm_expect_pauli_sum(const tcm_pauli* ham, int32_t dtype, const void* state,
 
 // ---- measurement ----------------------------------------------------------
 namespace {
-// chunk prefix sums of the sampler: batch x (2^(n - min(n, 10)) + 1) doubles
+// the sampler's chunk prefix sums (2^(n - min(n, 10)) + 1 doubles per item)
+// and stretch sums (2^(n - min(n, 6)))
 int64_t sample_ws(int n, int64_t batch) {
-  const int cl = n < 10 ? n : 10;
-  return batch * (((int64_t)1 << (n - cl)) + 1) * (int64_t)sizeof(double);
+  const int cl = std::min(n, kSampleChunkLog), sl = std::min(n, kSampleSubLog);
+  return batch * (((int64_t)1 << (n - cl)) + 1 + ((int64_t)1 << (n - sl))) * (int64_t)sizeof(double);
 }
 // blocks of the measurement partial sums and workspace: fixval (u64 per
 // batch item), then part[batch][kMeasBlocks][2]
@@ -1234,7 +1235,7 @@ int sample_impl(const char* what, bool prob, int32_t n, int32_t dtype, const voi
       (batch > 0 && shots > 0 && (!state || !uniforms || !out || !workspace)))
     return set_error(TCM_E_ARG, "bad arguments to %s", what);
   if (batch == 0 || shots == 0) return 0;
-  if (batch > 65535 || (shots + 3) / 4 > 0x7fffffffll || ((int64_t)1 << (n - (n < 10 ? n : 10))) > 0x7fffffffll)
+  if (batch > 65535 || (shots + 15) / 16 > 0x7fffffffll || ((int64_t)1 << (n - std::min(n, kSampleChunkLog))) > 0x7fffffffll)
     return set_error(TCM_E_ARG, "%s: batch, shots or state too large for one launch", what);
   if (ws_bytes < sample_ws(n, batch)) return set_error(TCM_E_WORKSPACE, "workspace too small");
   hipStream_t st = (hipStream_t)stream;

@@ -231,7 +231,9 @@ void launch_csr_vjp(const int64_t* rowptr, const int64_t* cols, const void* vals
 template <typename T>
 void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* psi, int64_t nrows,
                        double* part, double* out, hipStream_t st);
-// src: states [batch][2^n] (prob false) or probability vectors (prob true)
+// src: states [batch][2^n] (prob false) or probability vectors (prob true);
+// cum: scratch of sample_ws (sample.hip)
+constexpr int kSampleChunkLog = 10, kSampleSubLog = 6;
 template <typename T>
 void launch_sample(const void* src, bool prob, int n, int64_t batch, const double* u, int64_t shots, int64_t* out,
                    double* cum, hipStream_t st);

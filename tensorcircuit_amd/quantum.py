@@ -117,16 +117,13 @@ def count_tuple2dict(count: Tuple[Any, Any], n: int, key: str = "bin") -> Dict[A
 def sample2all(sample: Any, n: int, format: str = "count_vector", jittable: bool = False) -> Any:
     """sample_int or sample_bin -> the requested format (quantum.py:2325-2373)."""
     s = torch.as_tensor(sample)
-    if s.dim() == 1:
-        sample_int, sample_bin = s, sample_int2bin(s, n)
-    elif s.dim() == 2:
-        sample_int, sample_bin = sample_bin2int(s, n), s
-    else:
+    if s.dim() not in (1, 2):
         raise ValueError("unrecognized tensor shape for sample")
+    if format == "sample_bin":
+        return s if s.dim() == 2 else sample_int2bin(s, n)
+    sample_int = s if s.dim() == 1 else sample_bin2int(s, n)
     if format == "sample_int":
         return sample_int
-    if format == "sample_bin":
-        return sample_bin
     count_tuple = sample2count(sample_int, n, jittable)
     if format == "count_tuple":
         return count_tuple

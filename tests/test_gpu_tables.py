@@ -181,3 +181,33 @@ def test_csr(gpu, n, mean, hermitian):
         assert np.abs(np_of(c.vjp(xd, torch.conj(gd))) - (gr[:, None] * ax + gr.conj()[:, None] * dx)).max() <= 8 * tol
         for b in range(3):
             assert abs(complex(c.expect(xd[b])) - np.vdot(xr[b], ax[b])) <= max(tol, 1e-12) * np.sqrt(N)
+
+
+# one stretch, several, one chunk, 16 chunks (one search level), more than
+# 4096 chunks (two tiles of the scan); sparse weights, and draws at both ends
+@pytest.mark.parametrize("n,shots", [(1, 5), (3, 40), (6, 17), (8, 100), (10, 1), (11, 333), (14, 2000), (15, 64),
+                                     (23, 500)])
+def test_sample_levels(gpu, n, shots):
+    from tensorcircuit_amd import engine
+
+    rng = np.random.default_rng(500 + n)
+    N = 1 << n
+    for dt in (torch.float32, torch.float64):
+        p = torch.as_tensor(rng.random((2, N)) * (rng.random((2, N)) < (0.3 if n > 3 else 1.0))).to(dt)
+        p[:, 0] = 0.0
+        p[:, -1] = 0.0
+        u = rng.random((2, shots))
+        u[0, 0] = 0.0  # r = total
+        got = engine.sample_prob_indices(p.cuda(), n, torch.as_tensor(u)).cpu().numpy()
+        pd = p.to(torch.float64).numpy()
+        for b in range(2):
+            cdf = np.cumsum(pd[b])
+            r = cdf[-1] * (1.0 - u[b])
+            if cdf[-1] == 0:  # no weight (n = 1 here): the first index
+                assert (got[b] == 0).all()
+                continue
+            assert (pd[b][got[b]] > 0).all()
+            # the running sums agree to about N units in the last place
+            slack = N * 2.0**-52 * cdf[-1]
+            assert (cdf[got[b]] >= r - slack).all()
+            assert (cdf[got[b]] - pd[b][got[b]] <= r + slack).all()
