@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libtcm.so")
 
-SOURCES = ["kernels.hip", "program.cpp", "engine.cpp", "passgen.cpp", "jit.cpp", "kernels_aux.hip", "csr.hip",
+SOURCES = ["kernels.hip", "program.cpp", "engine.cpp", "passgen.cpp", "jit.cpp", "pauli_terms.hip", "csr.hip",
            "sample.hip", "pauli_tile.hip", "tile_pass.hip", "noalloc.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -35,7 +35,7 @@ struct tcm_multi_plan {
 
 struct PauliDev {
   void* terms = nullptr;
-  void* flat = nullptr;    // DPTermF per term in the caller's order
+  void *xterms = nullptr, *xgroups = nullptr, *xchunks = nullptr;  // strings kept apart
   void* groups = nullptr;  // DPGroup per flip mask (sparse form only)
   void* tgroups[2] = {nullptr, nullptr};
   void* tterms[2] = {nullptr, nullptr};
@@ -72,7 +72,9 @@ struct tcm_pauli {
   int n = 0;
   std::vector<DPGroup> groups;     // by flip mask, diagonal first
   std::vector<DPTerm> terms;
-  std::vector<DPTermF> flat;       // every term in the caller's order
+  std::vector<DPTermX> xterms;     // the strings kept apart (pauli_terms.hip)
+  std::vector<DPGroupX> xgroups;
+  std::vector<DPChunk> xchunks;
   int nslots = 0;                  // slots of the per-group kernels
   PauliTileSched ts[2];
   PauliJit jit[2];
@@ -320,8 +322,14 @@ int ensure_pauli(tcm_pauli* H, int dt, PauliDev** out) {
   if (!pd.groups) {
     if (int rc = upload(H->groups, &pd.groups)) return rc;
   }
-  if (!pd.flat) {
-    if (int rc = upload(H->flat, &pd.flat)) return rc;
+  if (!pd.xterms) {
+    if (int rc = upload(H->xterms, &pd.xterms)) return rc;
+  }
+  if (!pd.xgroups) {
+    if (int rc = upload(H->xgroups, &pd.xgroups)) return rc;
+  }
+  if (!pd.xchunks) {
+    if (int rc = upload(H->xchunks, &pd.xchunks)) return rc;
   }
   const PauliTileSched& S = H->ts[dt];
   if (S.ok && !pd.tchunks[dt]) {
@@ -470,6 +478,36 @@ void pauli_sort_terms(PauliTileSched& S, DPPass& pp) {
   }
   close();
   pp.nc = (int)S.chunks.size() - pp.c0;
+}
+
+// The strings as k_pauli_terms stages them (DPTermX, DPGroupX, DPChunk).
+void pauli_sort_strings(tcm_pauli* H, std::map<uint64_t, std::vector<std::pair<int, DPTermX>>>& by_flip) {
+  DPChunk ch{0, 0, 0, 0};
+  auto close = [&]() {
+    if (ch.nt) H->xchunks.push_back(ch);
+    ch = DPChunk{(int)H->xgroups.size(), 0, (int)H->xterms.size(), 0};
+  };
+  for (auto& kv : by_flip) {
+    auto& ts = kv.second;
+    std::stable_sort(ts.begin(), ts.end(), [](const std::pair<int, DPTermX>& a, const std::pair<int, DPTermX>& b) {
+      if (a.first != b.first) return a.first < b.first;
+      // the tile's bits first: strings that differ only outside it share an
+      // element pattern
+      return (a.second.yz & 0xfffu) != (b.second.yz & 0xfffu) ? (a.second.yz & 0xfffu) < (b.second.yz & 0xfffu)
+                                                              : a.second.yz < b.second.yz;
+    });
+    for (size_t i = 0; i < ts.size();) {
+      if (ch.nt == kTermsChunk) close();
+      DPGroupX g{(uint32_t)kv.first, 0};
+      for (; i < ts.size() && ch.nt < kTermsChunk; ++i, ++ch.nt) {
+        g.cnt += ts[i].first ? 0x10000u : 1u;
+        H->xterms.push_back(ts[i].second);
+      }
+      H->xgroups.push_back(g);
+      ++ch.ng;
+    }
+  }
+  close();
 }
 
 // Pack flip groups into LDS tiles: a tile = the low bits (coalescing) plus
@@ -1093,7 +1131,7 @@ int tcm_pauli_build(const int8_t* codes, const double* coeffs, int32_t nterms, i
   if (nqubits < 1 || nqubits > 32) return set_error(TCM_E_ARG, "nqubits=%d out of range", nqubits);
   if (nterms < 1 || !codes || !coeffs) return set_error(TCM_E_ARG, "need at least one term");
   std::map<uint64_t, std::vector<DPTerm>> by_flip;
-  std::vector<DPTermF> flat;
+  std::map<uint64_t, std::vector<std::pair<int, DPTermX>>> strings;  // by flip: (odd Y, string)
   for (int t = 0; t < nterms; ++t) {
     if (!std::isfinite(coeffs[t])) return set_error(TCM_E_NONFINITE, "term %d: non-finite coefficient", t);
     uint64_t flip = 0, yz = 0;
@@ -1111,16 +1149,16 @@ int tcm_pauli_build(const int8_t* codes, const double* coeffs, int32_t nterms, i
     tm.ny = ny;
     tm.w = coeffs[t];
     by_flip[flip].push_back(tm);
-    DPTermF tf{};
-    tf.flip = flip;
-    tf.yz = yz;
-    tf.ny = ny;
-    tf.w = coeffs[t];
-    flat.push_back(tf);
+    DPTermX tx{};
+    const int q = ny & 3;  // (-i)^ny: 1, -i, -1, i
+    tx.w = (q == 1 || q == 2) ? -coeffs[t] : coeffs[t];
+    tx.yz = (uint32_t)yz;
+    tx.idx = (uint32_t)t;
+    strings[flip].push_back({q & 1, tx});
   }
   tcm_pauli* H = new tcm_pauli();
   H->n = nqubits;
-  H->flat = std::move(flat);
+  pauli_sort_strings(H, strings);
   int slot = 0;
   for (auto& kv : by_flip) {  // std::map: flip 0 (diagonal) first
     DPGroup g{};
@@ -1148,7 +1186,8 @@ int tcm_pauli_free(tcm_pauli* ham) {
     PauliDev& pd = ham->dev[d];
     (void)hipSetDevice((int)d);
     if (pd.terms) (void)hipFree(pd.terms);
-    if (pd.flat) (void)hipFree(pd.flat);
+    for (void* q : {pd.xterms, pd.xgroups, pd.xchunks})
+      if (q) (void)hipFree(q);
     if (pd.groups) (void)hipFree(pd.groups);
     for (int dt = 0; dt < 2; ++dt) {
       void* ps[] = {pd.tgroups[dt], pd.tterms[dt], pd.truns[dt], pd.tchunks[dt]};
@@ -1375,9 +1414,9 @@ int tcm_apply_pauli_sum(const tcm_pauli* ham, int32_t dtype, const void* state, 
 
 // ---- per-term Pauli expectations / weighted applications ------------------
 namespace {
-int pauli_terms_blocks(int n) { return pauli_blocks(n, false); }
 int64_t pauli_terms_ws(const tcm_pauli* H, int64_t batch) {
-  return align_up(batch * (int64_t)H->flat.size() * pauli_terms_blocks(H->n) * 2 * (int64_t)sizeof(double));
+  // the complex128 count: the larger
+  return align_up(batch * (int64_t)H->xterms.size() * pauli_terms_blocks(H->n, false) * (int64_t)sizeof(double));
 }
 }  // namespace
 
@@ -1392,7 +1431,7 @@ int tcm_expect_pauli_terms(const tcm_pauli* ham, int32_t dtype, const void* stat
   if (!ham || !valid_dtype(dtype) || batch < 0 || (batch > 0 && (!state || !out)))
     return set_error(TCM_E_ARG, "bad arguments to tcm_expect_pauli_terms");
   if (batch == 0) return 0;
-  const int64_t nt = (int64_t)ham->flat.size();
+  const int64_t nt = (int64_t)ham->xterms.size();
   if (nt > 65535 || batch > 65535)
     return set_error(TCM_E_ARG, "tcm_expect_pauli_terms: %lld terms x %lld states exceeds 65535 per axis",
                      (long long)nt, (long long)batch);
@@ -1401,12 +1440,12 @@ int tcm_expect_pauli_terms(const tcm_pauli* ham, int32_t dtype, const void* stat
   PauliDev* pd = nullptr;
   if (int rc = ensure_pauli(H, dtype, &pd)) return rc;
   hipStream_t st = (hipStream_t)stream;
-  const int nblk = pauli_terms_blocks(H->n);
+  const PauliTermTables D{pd->xchunks, pd->xgroups, pd->xterms};
+  const int nch = (int)H->xchunks.size();
   if (dtype == TCM_C64)
-    launch_pauli_terms<float>((const DPTermF*)pd->flat, (int)nt, H->n, state, batch, nblk, (double*)workspace, out, st);
+    launch_pauli_terms<float>(D, nch, (int)nt, H->n, state, batch, (double*)workspace, out, st);
   else
-    launch_pauli_terms<double>((const DPTermF*)pd->flat, (int)nt, H->n, state, batch, nblk, (double*)workspace, out,
-                               st);
+    launch_pauli_terms<double>(D, nch, (int)nt, H->n, state, batch, (double*)workspace, out, st);
   HIP_TRY(hipGetLastError(), "pauli_terms launch");
   return 0;
 }
@@ -1421,11 +1460,12 @@ int tcm_apply_pauli_terms(const tcm_pauli* ham, int32_t dtype, const void* state
   PauliDev* pd = nullptr;
   if (int rc = ensure_pauli(H, dtype, &pd)) return rc;
   hipStream_t st = (hipStream_t)stream;
-  const int nt = (int)H->flat.size();
+  const PauliTermTables D{pd->xchunks, pd->xgroups, pd->xterms};
+  const int nt = (int)H->xterms.size(), nch = (int)H->xchunks.size();
   if (dtype == TCM_C64)
-    launch_pauli_terms_apply<float>((const DPTermF*)pd->flat, nt, H->n, state, out_state, weights, batch, st);
+    launch_pauli_terms_apply<float>(D, nch, nt, H->n, state, out_state, weights, batch, st);
   else
-    launch_pauli_terms_apply<double>((const DPTermF*)pd->flat, nt, H->n, state, out_state, weights, batch, st);
+    launch_pauli_terms_apply<double>(D, nch, nt, H->n, state, out_state, weights, batch, st);
   HIP_TRY(hipGetLastError(), "pauli_terms_apply launch");
   return 0;
 }

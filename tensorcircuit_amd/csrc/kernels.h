@@ -47,14 +47,22 @@ struct DPPass {
   int32_t c0, nc;      // chunks of its sorted terms (the kernel that is not compiled)
   int32_t blk_bits[32];
 };
-// one Pauli term in the caller's order (per-term expectations / weighted
-// applications): P = w (-i)^ny X^flip with the sign (-1)^popcount(row & yz)
-struct DPTermF {
-  uint64_t flip;   // X/Y positions (index bits)
-  uint64_t yz;     // Y/Z positions (index bits)
-  int32_t ny;      // number of Y factors
-  int32_t pad;
-  double w;        // weight
+// Pauli strings kept apart (pauli_terms.hip), sorted by (flip mask, odd
+// number of Y, yz): `idx` is the string's place in the caller's order, w holds
+// the sign of (-i)^ny, `cnt` counts the group's strings with an even (low
+// half) and an odd (high half) number of Y
+struct DPTermX {
+  double w;
+  uint32_t yz, idx;
+};
+struct DPGroupX {
+  uint32_t flip, cnt;
+};
+// strings a block of k_pauli_terms takes (DPChunk): 32 and not 128, so that a
+// state of few tiles has blocks enough (59 strings, 20 qubits: 24 us, not 28)
+constexpr int kTermsChunk = 32;
+struct PauliTermTables {
+  const void *chunks, *groups, *terms;
 };
 
 struct DPGroupT {
@@ -211,13 +219,14 @@ void launch_probability(const void* psi, void* out, int64_t total, hipStream_t s
 template <typename T>
 void launch_pauli_coo(const DPGroup* groups, int ngroups, const DPTerm* terms, int n, int64_t nterms, int64_t* rows,
                       int64_t* cols, void* vals, hipStream_t st);
-// per-term Pauli expectations and weighted applications
-// (kernels_aux.hip)
+// per-term Pauli expectations and weighted applications (pauli_terms.hip);
+// part: pauli_terms_blocks partial sums per (state, string)
+int pauli_terms_blocks(int n, bool c64);
 template <typename T>
-void launch_pauli_terms(const DPTermF* terms_dev, int nterms, int n, const void* psi, int64_t batch, int nblk,
+void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n, const void* psi, int64_t batch,
                         double* part, double* out, hipStream_t st);
 template <typename T>
-void launch_pauli_terms_apply(const DPTermF* terms_dev, int nterms, int n, const void* psi, void* out,
+void launch_pauli_terms_apply(const PauliTermTables& D, int nchunks, int nterms, int n, const void* psi, void* out,
                               const double* weights, int64_t batch, hipStream_t st);
 // CSR matrices (csr.hip); drowptr null: A = A^dagger
 constexpr int kCsrBlocks = 2048;  // most blocks, and partial sums, of a launch

@@ -211,3 +211,37 @@ def test_sample_levels(gpu, n, shots):
             slack = N * 2.0**-52 * cdf[-1]
             assert (cdf[got[b]] >= r - slack).all()
             assert (cdf[got[b]] - pd[b][got[b]] <= r + slack).all()
+
+
+# (qubits, strings, letters): less than a wave, the last size with one
+# amplitude per thread and the first with eight, one tile (2^11 or 2^12
+# amplitudes) and several, the second chunk of 32 staged strings, flips that
+# stay in the tile and flips that leave it
+@pytest.mark.parametrize("n,T,letters", [(1, 4, 4), (2, 9, 4), (5, 32, 4), (6, 33, 4), (8, 40, 4), (9, 128, 4),
+                                         (11, 33, 4), (12, 257, 4), (13, 90, "z"), (14, 131, "xz")])
+def test_pauli_strings(gpu, n, T, letters):
+    from tensorcircuit_amd import engine
+
+    rng = np.random.default_rng(77 * n + T)
+    alphabet = {4: [0, 1, 2, 3], "z": [0, 3], "xz": [0, 0, 0, 0, 0, 0, 1, 3]}[letters]
+    codes = rng.choice(alphabet, size=(T, n)).astype(np.int8)
+    w = rng.standard_normal(T)
+    a = rng.standard_normal((3, T))
+    a[:, rng.integers(0, T, T // 3)] = 0.0
+    ham = engine.PauliSum(n, codes, w)
+    s = random_states(rng, 3, n)
+    for dt in DTYPES:
+        st = torch.as_tensor(s).to(dt).cuda()
+        sd = np_of(st).astype(np.complex128)
+        e = np_of(ham.expect_terms(st))
+        out = np_of(ham.apply_terms(st, torch.as_tensor(a).cuda()))
+        for b in range(3):
+            ref = np.zeros(2**n, dtype=np.complex128)
+            for t in range(T):
+                p = sv.pauli_sum_apply(sd[b], n, [(1.0, list(codes[t]))])
+                # 2^n products summed in 64 bits; their magnitudes sum to 1
+                assert abs(e[b, t] - w[t] * np.vdot(sd[b], p)) <= 1.01 * (2**n + 8) * 2.0**-53 * abs(w[t])
+                ref += a[b, t] * w[t] * p
+            # T products summed in 64 bits, then one rounding to the state's type
+            tol = (2 * T + 8) * 2.0**-53 * np.abs(a[b] * w).sum() + 2 * UNIT[dt] * np.abs(ref).max()
+            assert np.abs(out[b] - ref).max() <= tol
