@@ -142,7 +142,7 @@ int upload(const std::vector<V>& v, void** out) {
 void free_tables(DeviceTables* D) {
   if (!D) return;
   void* ptrs[] = {D->dpass, D->dop, D->ukbits, D->runoff, D->blob, D->msrc, D->recipes, D->factors,
-                  D->gop_list, D->ctab, D->p_ptr, D->p_gops, D->gfac};
+                  D->gop_list, D->gop_sum, D->ctab, D->p_ptr, D->p_gops, D->gfac};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (void* m : D->jit_mod)
@@ -176,6 +176,7 @@ int ensure_tables(Program& P, int dtype, int mode, DeviceTables** out) {
   rc = rc ? rc : upload(S.recipes, &D->recipes);
   rc = rc ? rc : upload(S.factors, &D->factors);
   rc = rc ? rc : upload(S.gop_list, &D->gop_list);
+  rc = rc ? rc : upload(S.gop_sum, &D->gop_sum);
   if (!rc) {
     if (dtype == TCM_C64) {
       std::vector<float> cf(P.ctab.begin(), P.ctab.end());
@@ -303,7 +304,9 @@ int forward_impl(Program& P, int dtype, const void* params, int64_t pstride, voi
   Carve cv(ws);
   void* mtab = cv.take(batch * (int64_t)std::max(S.mtab_size, 1) * sizeof(T));
   if (cv.off > ws_bytes) return set_error(TCM_E_WORKSPACE, "workspace %lld < %lld bytes", (long long)ws_bytes, (long long)cv.off);
-  launch_prep<T>(S, *D, D->ctab, params, pstride, mtab, batch, st);
+  PrepJobs J;
+  add_prep<T>(J, S, *D, D->ctab, params, pstride, mtab, batch, st);
+  launch_prep<T>(J, st);
   if (int rc = run_forward_passes<T>(P, S, *D, mtab, state, batch, ckpts, st, init_zero != 0)) return rc;
   HIP_TRY(hipGetLastError(), "forward launch");
   return 0;
@@ -629,7 +632,8 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
 // ---- adjoint ---------------------------------------------------------------
 struct AdjWs {
   void *mtab_f, *mtab_a, *psi, *lam, *ckpt;
-  double *part, *gsum, *epart, *e2;
+  double *part, *gsum, *epart;
+  bool all;  // `part` holds every pass (Sched::part_base)
   int64_t bytes;
 };
 
@@ -646,13 +650,15 @@ AdjWs carve_adj(const Program& P, const tcm_pauli* H, int dtype, int64_t batch, 
   w.lam = cv.take(batch * N * 2 * ts);
   w.ckpt = mode == 0 ? cv.take((int64_t)P.ckpt_gate.size() * batch * N * 2 * ts) : nullptr;
   const int64_t ngp = std::max(A.max_ngop_pass, 1);
-  w.part = (double*)cv.take(batch * ngp * (int64_t)A.max_slots * sizeof(double));
+  // gradient partials of all passes, summed by one launch at the end, unless
+  // they are many (deep circuits): then of one pass at a time
+  w.all = A.part_total * batch * (int64_t)sizeof(double) <= std::max<int64_t>(64 << 20, batch * N * 2 * ts / 4);
+  w.part = (double*)cv.take(batch * (w.all ? A.part_total : ngp * (int64_t)A.max_slots) * (int64_t)sizeof(double));
   w.gsum = (double*)cv.take(batch * (int64_t)std::max(P.ngop, 1) * sizeof(double));
   if (mode == 0 && H) {
     w.epart = (double*)cv.take(batch * (int64_t)pauli_slots(H, dtype) * 2 * sizeof(double));
-    w.e2 = (double*)cv.take(batch * 2 * sizeof(double));
   } else {
-    w.epart = w.e2 = nullptr;
+    w.epart = nullptr;
   }
   w.bytes = cv.off;
   return w;
@@ -670,6 +676,7 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
   auto ckpt_ptr = [&](size_t c) { return (const void*)((const char*)ckpts + (int64_t)c * tot * 2 * sizeof(T)); };
   const int64_t ngp = std::max(A.max_ngop_pass, 1);
   const int64_t pstride = ngp * (int64_t)A.max_slots;
+  auto part_of = [&](int p) { return w.all ? w.part + batch * A.part_base[p] : w.part; };
   const int np = (int)A.passes.size();
   // checkpoint restoring psi before pass p: the one taken after pass p-1
   auto ckpt_before = [&](int p) -> int {
@@ -687,9 +694,9 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
         launch_plain_adj_uk<T>(op, (const int32_t*)D->ukbits, D->ctab, w.psi, w.lam, batch, n, st);
       } else {
         const int slots = op.gop >= 0 ? A.gop_slots[op.gop] : std::min<int64_t>(512, std::max<int64_t>(1, (N >> 2) / 256));
-        launch_plain_adj<T>(op, w.mtab_a, A.mtab_size, D->ctab, w.psi, w.psi, w.lam, w.lam, batch, n, slots, w.part,
-                            pstride, st);
-        if (op.gop >= 0) launch_reduce_gop(w.part, pstride, slots, nullptr, op.gop, 1, w.gsum, P.ngop, batch, st);
+        launch_plain_adj<T>(op, w.mtab_a, A.mtab_size, D->ctab, w.psi, w.psi, w.lam, w.lam, batch, n, slots,
+                            part_of(p), w.all ? slots : pstride, st);
+        if (op.gop >= 0 && !w.all) launch_reduce_gop(w.part, pstride, slots, nullptr, op.gop, 1, w.gsum, P.ngop, batch, st);
       }
       int c = ckpt_before(p);
       if (c >= 0 && ckpts) launch_copy<T>(w.psi, ckpt_ptr(c), tot, st);
@@ -715,16 +722,17 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
       // unless it is the input gradient
       void* pout = (c >= 0 || p == 0) ? nullptr : w.psi;
       void* lout = p > 0 ? w.lam : grad_input;
+      const int64_t ps = w.all ? (int64_t)dp.ngop << dp.nblk_log : pstride;
       if (!A.jit.empty() && A.jit[p].kernel >= 0) {
         if (int rc = jit_launch_adj(A, *D, p, sizeof(T) == 8, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n,
-                                    w.part, pstride, st))
+                                    part_of(p), ps, st))
           return rc;
       } else if (A.R == kTileSlots) {
-        launch_tile_adj<T>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, w.part, pstride, st);
+        launch_tile_adj<T>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, part_of(p), ps, st);
       } else {
         return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", A.R);
       }
-      if (dp.ngop > 0)
+      if (dp.ngop > 0 && !w.all)
         launch_reduce_gop(w.part, pstride, 1ll << dp.nblk_log, (const int32_t*)D->gop_list + dp.gop_list0, 0,
                           dp.ngop, w.gsum, P.ngop, batch, st);
       pin = c >= 0 ? ckpt_ptr(c) : w.psi;
@@ -733,6 +741,13 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
     if (np == 0 && grad_input) launch_copy<T>(grad_input, lam_src, tot, st);
   }
   return 0;
+}
+
+void finish_sweep(const Program& P, const Sched& A, const DeviceTables& D, const AdjWs& w, const double* epart,
+                  int64_t nslots, double* energy, double mult, double* grad, int64_t batch, hipStream_t st) {
+  launch_finish(epart, nslots, energy, w.all ? w.part : w.gsum, w.all ? (const DGopSum*)D.gop_sum : nullptr, P.ngop,
+                (const int32_t*)D.p_ptr, (const int32_t*)D.p_gops, (const double*)D.gfac, mult, grad, P.nparams,
+                A.max_slots, batch, st);
 }
 
 template <typename T>
@@ -751,22 +766,18 @@ int energy_grad_impl(Program& P, int dtype, const void* params, int64_t pstride,
   const Sched& F = P.sched[dtype][0];
   const Sched& A = P.sched[dtype][1];
   const int64_t N = 1ll << P.n;
+  PrepJobs J;
+  add_prep<T>(J, F, *DF, DF->ctab, params, pstride, w.mtab_f, batch, st);
+  add_prep<T>(J, A, *DA, DA->ctab, params, pstride, w.mtab_a, batch, st);
+  launch_prep<T>(J, st);
   // forward with checkpoints
-  launch_prep<T>(F, *DF, DF->ctab, params, pstride, w.mtab_f, batch, st);
   if (inputs) launch_copy<T>(w.psi, inputs, batch * N, st);
   if (int rc = run_forward_passes<T>(P, F, *DF, w.mtab_f, w.psi, batch, w.ckpt, st, inputs == nullptr)) return rc;
   // energy and lambda = H psi
   if (int rc = pauli_energy_apply<T>(H, dtype, w.psi, w.lam, nullptr, batch, w.epart, true, true, st)) return rc;
-  launch_sum_slots(w.epart, (int64_t)pauli_slots(H, dtype) * 2, pauli_slots(H, dtype), 2, w.e2, batch, st);
-  // reverse sweep
-  launch_prep<T>(A, *DA, DA->ctab, params, pstride, w.mtab_a, batch, st);
+  // reverse sweep, then energies and gradients from the partial sums
   if (int rc = reverse_sweep<T>(P, dtype, w, w.psi, w.lam, w.ckpt, nullptr, batch, st)) return rc;
-  launch_grad_assemble(w.gsum, P.ngop, (const int32_t*)DA->p_ptr, (const int32_t*)DA->p_gops,
-                       (const double*)DA->gfac, 1.0, grad, P.nparams, batch, st);
-  // energy real parts
-  HIP_TRY(hipMemcpy2DAsync(energy, sizeof(double), w.e2, 2 * sizeof(double), sizeof(double), batch,
-                           hipMemcpyDeviceToDevice, st),
-          "energy copy");
+  finish_sweep(P, A, *DA, w, w.epart, pauli_slots(H, dtype), energy, 1.0, grad, batch, st);
   HIP_TRY(hipGetLastError(), "adjoint launch");
   return 0;
 }
@@ -782,11 +793,11 @@ int vjp_impl(Program& P, int dtype, const void* params, int64_t pstride, const v
   DeviceTables* DA = nullptr;
   if (int rc = ensure_tables(P, dtype, 1, &DA)) return rc;
   const Sched& A = P.sched[dtype][1];
-  launch_prep<T>(A, *DA, DA->ctab, params, pstride, w.mtab_a, batch, st);
+  PrepJobs J;
+  add_prep<T>(J, A, *DA, DA->ctab, params, pstride, w.mtab_a, batch, st);
+  launch_prep<T>(J, st);
   if (int rc = reverse_sweep<T>(P, dtype, w, state, grad_state, ckpts, grad_input, batch, st)) return rc;
-  if (grad_params)
-    launch_grad_assemble(w.gsum, P.ngop, (const int32_t*)DA->p_ptr, (const int32_t*)DA->p_gops,
-                         (const double*)DA->gfac, 0.5, grad_params, P.nparams, batch, st);
+  if (grad_params) finish_sweep(P, A, *DA, w, nullptr, 0, nullptr, 0.5, grad_params, batch, st);
   HIP_TRY(hipGetLastError(), "vjp launch");
   return 0;
 }
@@ -806,6 +817,7 @@ template <typename T>
 int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int init_zero, void* ws, hipStream_t st) {
   std::vector<DeviceTables*> D(ndesc);
   std::vector<void*> mtab(ndesc);
+  PrepJobs prep;
   Carve cv(ws);
   int maxp = 0;
   for (int i = 0; i < ndesc; ++i) {
@@ -816,10 +828,11 @@ int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int in
       return set_error(TCM_E_UNSUPPORTED, "multi-program launches run 4 register slots (program %d has %d)", i, S.R);
     mtab[i] = cv.take(descs[i].batch * (int64_t)std::max(S.mtab_size, 1) * sizeof(T));
     if (descs[i].batch <= 0) continue;
-    launch_prep<T>(S, *D[i], D[i]->ctab, descs[i].params, descs[i].param_stride, mtab[i], descs[i].batch, st);
+    add_prep<T>(prep, S, *D[i], D[i]->ctab, descs[i].params, descs[i].param_stride, mtab[i], descs[i].batch, st);
     if (init_zero && !tile_first(S)) launch_init_zero<T>(descs[i].state, P.n, descs[i].batch, st);
     maxp = std::max(maxp, (int)S.passes.size());
   }
+  launch_prep<T>(prep, st);
   for (int r = 0; r < maxp; ++r) {
     MultiJobs J{};
     int64_t blocks = 0;
@@ -899,6 +912,7 @@ int forward_plan_impl(tcm_multi_plan* M, const tcm_multi_desc* descs, int ndesc,
   if (int rc = plan_load(M, &fns)) return rc;
   std::vector<DeviceTables*> D(ndesc);
   std::vector<void*> mtab(ndesc);
+  PrepJobs prep;
   Carve cv(ws);
   for (int i = 0; i < ndesc; ++i) {
     Program& P = descs[i].prog->p;
@@ -906,9 +920,10 @@ int forward_plan_impl(tcm_multi_plan* M, const tcm_multi_desc* descs, int ndesc,
     const Sched& S = P.sched[dtype][0];
     mtab[i] = cv.take(descs[i].batch * (int64_t)std::max(S.mtab_size, 1) * sizeof(T));
     if (descs[i].batch <= 0) continue;
-    launch_prep<T>(S, *D[i], D[i]->ctab, descs[i].params, descs[i].param_stride, mtab[i], descs[i].batch, st);
+    add_prep<T>(prep, S, *D[i], D[i]->ctab, descs[i].params, descs[i].param_stride, mtab[i], descs[i].batch, st);
     if (init_zero) launch_init_zero<T>(descs[i].state, P.n, descs[i].batch, st);
   }
+  launch_prep<T>(prep, st);
   for (int r = 0; r < M->maxp; ++r) {
     std::vector<char> in_kernel(ndesc, 0);
     if (M->kid[r] >= 0) {
@@ -1004,12 +1019,13 @@ int pauli_expect_prepared(const tcm_pauli* ham, int32_t dtype, const void* state
                      "tcm_expect_pauli_sum call with it for this dtype first)",
                      dev);
   hipStream_t st = (hipStream_t)stream;
-  double* epart = (double*)scratch;
+  // a single partial per state is the energy itself
+  const int ns = pauli_slots(H, dtype);
+  double* epart = ns > 1 ? (double*)scratch : out;
   int rc = dtype == TCM_C64 ? pauli_energy_apply<float>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st, pd)
                             : pauli_energy_apply<double>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st, pd);
   if (rc) return rc;
-  const int ns = pauli_slots(H, dtype);
-  launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, out, batch, st);
+  if (ns > 1) launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, out, batch, st);
   HIP_TRY(hipGetLastError(), "expect launch");
   return 0;
 }
@@ -1222,12 +1238,13 @@ int tcm_expect_pauli_sum(const tcm_pauli* ham, int32_t dtype, const void* state,
   if (pauli_ws(ham, dtype, batch) > ws_bytes) return set_error(TCM_E_WORKSPACE, "workspace too small");
   hipStream_t st = (hipStream_t)stream;
   tcm_pauli* H = const_cast<tcm_pauli*>(ham);
-  double* epart = (double*)workspace;
+  // a single partial per state is the energy itself
+  const int ns = pauli_slots(H, dtype);
+  double* epart = ns > 1 ? (double*)workspace : out;
   int rc = dtype == TCM_C64 ? pauli_energy_apply<float>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st)
                             : pauli_energy_apply<double>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st);
   if (rc) return rc;
-  const int ns = pauli_slots(H, dtype);
-  launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, out, batch, st);
+  if (ns > 1) launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, out, batch, st);
   HIP_TRY(hipGetLastError(), "expect launch");
   return 0;
 }

@@ -137,6 +137,7 @@ struct DeviceTables {
   void* recipes = nullptr;
   void* factors = nullptr;
   void* gop_list = nullptr;
+  void* gop_sum = nullptr;
   // program-wide (shared by both schedules of a dtype, owned by mode 0)
   void* ctab = nullptr;    // constant matrices in T
   void* p_ptr = nullptr;
@@ -156,9 +157,25 @@ int jit_launch_adj(const Sched& S, const DeviceTables& D, int pi, int dt, const 
                    const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
                    double* part, int64_t pstride, hipStream_t st);
 
+// matrix tables of up to kMaxPrepJobs schedules in one launch
+constexpr int kMaxPrepJobs = 16;
+struct PrepJob {
+  const void *rec, *fac, *params, *ctab;
+  void* mtab;
+  int64_t pstride, mstride, block0;
+  int32_t nrec, first_dg, dg_log, pad;
+};
+struct PrepJobs {
+  int32_t njobs = 0, widest = 0;
+  int64_t blocks = 0;
+  PrepJob job[kMaxPrepJobs];
+};
+// adds a job; launches the jobs when they are kMaxPrepJobs
 template <typename T>
-void launch_prep(const Sched& S, const DeviceTables& D, const void* ctab, const void* params, int64_t pstride,
-                 void* mtab, int64_t batch, hipStream_t st);
+void add_prep(PrepJobs& J, const Sched& S, const DeviceTables& D, const void* ctab, const void* params,
+              int64_t pstride, void* mtab, int64_t batch, hipStream_t st);
+template <typename T>
+void launch_prep(PrepJobs& J, hipStream_t st);
 template <typename T>
 void launch_init_zero(void* state, int n, int64_t batch, hipStream_t st);
 template <typename T>
@@ -252,8 +269,10 @@ void launch_measure_step(const void* psi, int n, int64_t batch, const MeasureSte
                          int nblk, hipStream_t st);
 void launch_reduce_gop(const double* part, int64_t pstride, int64_t nslots, const int32_t* gop_list, int gop_single,
                        int ngop_pass, double* gsum, int ngop, int64_t batch, hipStream_t st);
-void launch_grad_assemble(const double* gsum, int ngop, const int32_t* p_ptr, const int32_t* p_gops,
-                          const double* gfac, double mult, double* grad, int nparams, int64_t batch,
-                          hipStream_t st);
+// energies (epart non-null: nslots (re, im) partials per state) and parameter
+// gradients from the gop partials (gs) or, gs null, from gsum[b][gop] = part
+void launch_finish(const double* epart, int64_t nslots, double* energy, const double* part, const DGopSum* gs, int ngop,
+                   const int32_t* p_ptr, const int32_t* p_gops, const double* gfac, double mult, double* grad,
+                   int nparams, int max_slots, int64_t batch, hipStream_t st);
 
 }  // namespace tcm

@@ -82,15 +82,27 @@ __device__ __forceinline__ void block_sum2(double& a, double& b) {
 }
 
 // ---------------------------------------------------------------------------
-// matrix preparation: per batch item, evaluate every recipe from params
+// matrix preparation: a block evaluates every recipe of one batch item of one
+// schedule from its parameters.  A chain of a few loads and 64-bit sines, so
+// the schedules of a call (forward and reverse, or the programs of an uneven
+// batch) share a launch: 2 of 5 us became one of 6 us at 12 qubits x 4
+// layers, 9 of 9 us one of 9 us for 9 programs.  Blocks are 1024 threads
+// where a batch item has more than 512 entries
+// and its block would be alone on its CU (2 of 63 us with 256 threads,
+// one of 27 us, for 1420 gates and 4 parameter sets), else 256.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void k_prep(const DRecipe* __restrict__ rec, int nrec, int first_dg, int dg_log,
-                       const DFactor* __restrict__ fac, const T* __restrict__ params, int64_t pstride,
-                       const T* __restrict__ ct, T* __restrict__ mtab, int64_t mstride) {
-  const int64_t b = blockIdx.x;
-  T* mt = mtab + b * mstride;
-  const T* pr = params ? params + b * pstride : nullptr;
+__global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
+  int q = 0;
+  while (q + 1 < J.njobs && (int64_t)blockIdx.x >= J.job[q + 1].block0) ++q;
+  const DRecipe* __restrict__ rec = (const DRecipe*)J.job[q].rec;
+  const DFactor* __restrict__ fac = (const DFactor*)J.job[q].fac;
+  const T* __restrict__ ct = (const T*)J.job[q].ctab;
+  const int nrec = J.job[q].nrec, first_dg = J.job[q].first_dg, dg_log = J.job[q].dg_log;
+  const int64_t b = blockIdx.x - J.job[q].block0;
+  T* mt = (T*)J.job[q].mtab + b * J.job[q].mstride;
+  const T* __restrict__ pr = (const T*)J.job[q].params;
+  if (pr) pr += b * J.job[q].pstride;
   for (int i = threadIdx.x; i < first_dg; i += blockDim.x) {
     const DRecipe r = rec[i];
     if (r.kind < 0) continue;
@@ -728,15 +740,28 @@ bool launch_mfma_tile(const DPass& P, const DPass* passes_dev, int pi, const DOp
 // ---------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------
-// out[b * ncomp + c] = sum_s part[b * bstride + s * ncomp + c]
-__global__ void k_sum_slots(const double* __restrict__ part, int64_t bstride, int64_t nslots, int ncomp,
-                            double* __restrict__ out) {
-  const int64_t b = blockIdx.x;
-  double a = 0.0, c = 0.0;
-  for (int64_t s = threadIdx.x; s < nslots; s += blockDim.x) {
-    a += part[b * bstride + s * ncomp];
-    if (ncomp > 1) c += part[b * bstride + s * ncomp + 1];
+// sum of part[s * step], s = tid, tid + nthr, ... < n: four loads in flight
+__device__ __forceinline__ double strided_sum(const double* __restrict__ part, int64_t n, int step, int tid, int nthr) {
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  int64_t s = tid;
+  for (; s + 3 * (int64_t)nthr < n; s += 4 * (int64_t)nthr) {
+    a0 += part[s * step];
+    a1 += part[(s + nthr) * step];
+    a2 += part[(s + 2 * (int64_t)nthr) * step];
+    a3 += part[(s + 3 * (int64_t)nthr) * step];
   }
+  for (; s < n; s += nthr) a0 += part[s * step];
+  return (a0 + a1) + (a2 + a3);
+}
+
+// out[b * ncomp + c] = sum_s part[b * bstride + s * ncomp + c]; one block per
+// b, bound by the loads that it keeps in flight (49k pairs: 86 us with 256
+// threads and one load each, 20 us with 1024 and four)
+__global__ void __launch_bounds__(1024) k_sum_slots(const double* __restrict__ part, int64_t bstride, int64_t nslots,
+                                                    int ncomp, double* __restrict__ out) {
+  const int64_t b = blockIdx.x;
+  double a = strided_sum(part + b * bstride, nslots, ncomp, threadIdx.x, blockDim.x), c = 0.0;
+  if (ncomp > 1) c = strided_sum(part + b * bstride + 1, nslots, ncomp, threadIdx.x, blockDim.x);
   block_sum2(a, c);
   if (threadIdx.x == 0) {
     out[b * ncomp] = a;
@@ -759,17 +784,50 @@ __global__ void k_reduce_gop(const double* __restrict__ part, int64_t pstride, i
   }
 }
 
-// grad[b][p] = mult * sum_{gop of p} gfac[gop] * gsum[b][gop]
-__global__ void k_grad_assemble(const double* __restrict__ gsum, int ngop, const int32_t* __restrict__ p_ptr,
-                                const int32_t* __restrict__ p_gops, const double* __restrict__ gfac, double mult,
-                                double* __restrict__ grad, int nparams, int64_t batch) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= (int64_t)nparams * batch) return;
-  const int64_t b = i / nparams;
-  const int p = (int)(i % nparams);
-  double a = 0.0;
-  for (int q = p_ptr[p]; q < p_ptr[p + 1]; ++q) a += gfac[p_gops[q]] * gsum[b * ngop + p_gops[q]];
-  grad[i] = mult * a;
+// The end of a reverse sweep in one launch (after a launch per pass for its
+// partials, then sums, a copy and the chain rule, it was npasses + 3):
+//   energy[b]  = sum_s epart[b][s].re            blocks 0 .. nenergy - 1
+//   grad[b][p] = mult * sum_{gop of p} gfac[gop] * (sum of the gop's partials)
+// 16 passes of a 24-qubit circuit with 4 parameter sets: 16 launches and 105 us
+// before, 15 us here; a circuit of one tile: 4 launches, 14 us, before, 5 us here.
+// LP threads share a (b, p): a wave, or one thread where a gop has a single
+// partial (states of one tile).
+template <int LP>
+__global__ void __launch_bounds__(256) k_finish(const double* __restrict__ epart, int64_t nslots, int64_t nenergy,
+                                                double* __restrict__ energy, const double* __restrict__ part,
+                                                const DGopSum* __restrict__ gs, int ngop,
+                                                const int32_t* __restrict__ p_ptr, const int32_t* __restrict__ p_gops,
+                                                const double* __restrict__ gfac, double mult,
+                                                double* __restrict__ grad, int nparams, int64_t batch) {
+  if ((int64_t)blockIdx.x < nenergy) {
+    for (int64_t b = blockIdx.x; b < batch; b += nenergy) {
+      double a = strided_sum(epart + b * nslots * 2, nslots, 2, threadIdx.x, 256), c = 0.0;
+      block_sum2(a, c);
+      if (threadIdx.x == 0) energy[b] = a;
+    }
+    return;
+  }
+  const int64_t total = (int64_t)nparams * batch, step = (int64_t)(gridDim.x - nenergy) * (256 / LP);
+  const int lane = threadIdx.x & (LP - 1);
+  for (int64_t i = ((int64_t)blockIdx.x - nenergy) * (256 / LP) + threadIdx.x / LP; i < total; i += step) {
+    const int64_t b = i / nparams;
+    const int p = (int)(i - b * nparams);
+    double a = 0.0;
+    for (int q = p_ptr[p]; q < p_ptr[p + 1]; ++q) {
+      const int gop = p_gops[q];
+      double x;
+      if (gs) {
+        const DGopSum g = gs[gop];
+        x = strided_sum(part + batch * g.base + (b * g.ngop + g.row) * (int64_t)g.slots, g.slots, 1, lane, LP);
+      } else {
+        x = lane == 0 ? part[b * ngop + gop] : 0.0;
+      }
+      a += gfac[gop] * x;
+    }
+    if (LP > 1)
+      for (int off = LP / 2; off > 0; off >>= 1) a += __shfl_xor(a, off, LP);
+    if (lane == 0) grad[i] = mult * a;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -895,8 +953,8 @@ static inline int grid_for(int64_t work, int64_t cap = 1 << 20) {
 }
 
 template <typename T>
-void launch_prep(const Sched& S, const DeviceTables& D, const void* ctab, const void* params, int64_t pstride,
-                 void* mtab, int64_t batch, hipStream_t st) {
+void add_prep(PrepJobs& J, const Sched& S, const DeviceTables& D, const void* ctab, const void* params,
+              int64_t pstride, void* mtab, int64_t batch, hipStream_t st) {
   if (S.recipes.empty() || batch <= 0) return;
   // merged-diagonal (DG) recipes follow the base recipes; their widest group
   const int nrec = (int)S.recipes.size();
@@ -906,9 +964,19 @@ void launch_prep(const Sched& S, const DeviceTables& D, const void* ctab, const 
       if (first_dg == nrec) first_dg = i;
       dg_log = std::max(dg_log, (int)S.recipes[i].R);
     }
-  hipLaunchKernelGGL(k_prep<T>, dim3((unsigned)batch), dim3(256), 0, st, (const DRecipe*)D.recipes, nrec, first_dg,
-                     dg_log, (const DFactor*)D.factors, (const T*)params, pstride, (const T*)ctab, (T*)mtab,
-                     (int64_t)S.mtab_size);
+  J.job[J.njobs++] = PrepJob{D.recipes, D.factors, params, ctab, mtab, pstride, (int64_t)S.mtab_size, J.blocks,
+                             nrec, first_dg, dg_log, 0};
+  J.blocks += batch;
+  J.widest = std::max({J.widest, first_dg, (nrec - first_dg) << dg_log});
+  if (J.njobs == kMaxPrepJobs) launch_prep<T>(J, st);
+}
+
+template <typename T>
+void launch_prep(PrepJobs& J, hipStream_t st) {
+  if (J.njobs)
+    hipLaunchKernelGGL(k_prep<T>, dim3((unsigned)J.blocks), dim3(J.widest > 512 && J.blocks <= 1024 ? 1024 : 256), 0,
+                       st, J);
+  J = PrepJobs();
 }
 
 template <typename T>
@@ -1019,7 +1087,7 @@ void launch_inner(const void* a, const void* c, int n, int64_t batch, int nblk, 
 
 void launch_sum_slots(const double* part, int64_t bstride, int64_t nslots, int ncomp, double* out, int64_t batch,
                       hipStream_t st) {
-  hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)batch), dim3(256), 0, st, part, bstride, nslots, ncomp, out);
+  hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)batch), dim3(nslots > 1024 ? 1024 : 256), 0, st, part, bstride, nslots, ncomp, out);
 }
 
 void launch_reduce_gop(const double* part, int64_t pstride, int64_t nslots, const int32_t* gop_list, int gop_single,
@@ -1028,13 +1096,19 @@ void launch_reduce_gop(const double* part, int64_t pstride, int64_t nslots, cons
                      nslots, gop_list, gop_single, gsum, ngop);
 }
 
-void launch_grad_assemble(const double* gsum, int ngop, const int32_t* p_ptr, const int32_t* p_gops,
-                          const double* gfac, double mult, double* grad, int nparams, int64_t batch,
-                          hipStream_t st) {
-  const int64_t total = (int64_t)nparams * batch;
-  if (total <= 0) return;
-  hipLaunchKernelGGL(k_grad_assemble, dim3(grid_for(total, 1 << 24)), dim3(256), 0, st, gsum, ngop, p_ptr, p_gops,
-                     gfac, mult, grad, nparams, batch);
+void launch_finish(const double* epart, int64_t nslots, double* energy, const double* part, const DGopSum* gs, int ngop,
+                   const int32_t* p_ptr, const int32_t* p_gops, const double* gfac, double mult, double* grad,
+                   int nparams, int max_slots, int64_t batch, hipStream_t st) {
+  const int64_t total = grad ? (int64_t)nparams * batch : 0, nen = epart ? std::min<int64_t>(batch, 1 << 16) : 0;
+  if (total + nen == 0) return;
+  const bool one = !gs || max_slots == 1;
+  const int64_t blocks = std::min<int64_t>((total + (one ? 255 : 3)) / (one ? 256 : 4), 1 << 20);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(nen + blocks)), dim3(256), 0, st, epart, nslots, nen, energy, part, gs,
+                       ngop, p_ptr, p_gops, gfac, mult, grad, nparams, batch);
+  };
+  if (one) go(k_finish<1>);
+  else go(k_finish<64>);
 }
 
 // ---------------------------------------------------------------------------
@@ -1160,8 +1234,9 @@ void launch_pauli_coo(const DPGroup* groups, int ngroups, const DPTerm* terms, i
 
 // explicit instantiations used by engine.cpp
 #define TCM_INST(T)                                                                                            \
-  template void launch_prep<T>(const Sched&, const DeviceTables&, const void*, const void*, int64_t, void*,   \
-                               int64_t, hipStream_t);                                                          \
+  template void add_prep<T>(PrepJobs&, const Sched&, const DeviceTables&, const void*, const void*, int64_t,     \
+                            void*, int64_t, hipStream_t);                                                        \
+  template void launch_prep<T>(PrepJobs&, hipStream_t);                                                           \
   template void launch_init_zero<T>(void*, int, int64_t, hipStream_t);                                         \
   template void launch_copy<T>(void*, const void*, int64_t, hipStream_t);                                      \
   template void launch_plain_gate<T, false>(const DOp&, const int32_t*, const void*, int64_t, const void*,    \

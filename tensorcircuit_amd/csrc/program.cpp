@@ -1339,6 +1339,25 @@ static void finish_sched(const Program& P, Sched& S) {
     for (int g = 0; g < P.ngop; ++g) S.gop_slots[g] = slots;
     S.max_slots = slots;
   }
+  S.gop_sum.assign(P.ngop, DGopSum{0, 0, 1, 0, 0});
+  S.part_base.clear();
+  S.part_total = 0;
+  auto place = [&](int gop, int row, int ngop, int slots) { S.gop_sum[gop] = DGopSum{S.part_total, row, ngop, slots, 0}; };
+  if (S.k == 0) {
+    for (const DOp& op : S.dop) {
+      S.part_base.push_back(S.part_total);
+      if (op.gop < 0) continue;
+      place(op.gop, 0, 1, S.gop_slots[op.gop]);
+      S.part_total += S.gop_slots[op.gop];
+    }
+  } else {
+    for (const DPass& dp : S.dpass) {
+      S.part_base.push_back(S.part_total);
+      const int slots = 1 << dp.nblk_log;
+      for (int i = 0; i < dp.ngop; ++i) place(S.gop_list[dp.gop_list0 + i], i, dp.ngop, slots);
+      S.part_total += (int64_t)dp.ngop * slots;
+    }
+  }
 }
 
 int build_program(const tcm_gate* gates, int32_t ngates, int32_t n, int32_t nparams,

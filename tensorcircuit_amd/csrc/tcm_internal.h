@@ -154,6 +154,13 @@ struct DRecipe {
   double theta, scale;
 };
 
+// Where a gop's gradient partials are (Sched::part_base): for batch item b,
+// `slots` values at batch * base + (b * ngop + row) * slots
+struct DGopSum {
+  int64_t base;
+  int32_t row, ngop, slots, pad;
+};
+
 // Table entries of an ry recipe: [c, -s, s, c] of the exact rotation by
 // phi = angle / 2, then [t, s', sigma, 0]: phi reduced to phi' in
 // [-pi/2, pi/2] with R(phi) = sigma R(phi'), t = tan(phi' / 2), s' = sin phi'
@@ -239,6 +246,11 @@ struct Sched {
   int32_t max_slots = 0;        // largest number of gradient partial slots per gop
   std::vector<int32_t> gop_slots;  // per gop: number of partial slots (blocks)
   std::vector<int32_t> gop_list;   // per pass (from DPass::gop_list0): gops by gloc
+  // gradient partials of all passes side by side: pass p's [batch][gop][slot]
+  // at batch * part_base[p], part_total values per batch item
+  std::vector<int64_t> part_base;
+  int64_t part_total = 0;
+  std::vector<DGopSum> gop_sum;    // per gop: where its partials are
   std::vector<DeviceTables*> dev;  // per device
   // pass compiler output (opts.jit): 0 not built, 1 built, -1 failed
   int32_t jit_state = 0;

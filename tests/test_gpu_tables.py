@@ -245,3 +245,67 @@ def test_pauli_strings(gpu, n, T, letters):
             # T products summed in 64 bits, then one rounding to the state's type
             tol = (2 * T + 8) * 2.0**-53 * np.abs(a[b] * w).sum() + 2 * UNIT[dt] * np.abs(ref).max()
             assert np.abs(out[b] - ref).max() <= tol
+
+
+# (qubits, gates, batch, type of pass): partial sums of all passes side by
+# side, one or many per gate, and (the last two: more than 64 MiB of them) of
+# one pass at a time; also the per-gate kernels
+@pytest.mark.parametrize("n,gates,batch,fuse", [(3, 20, 5, 1), (6, 90, 3, 1), (13, 60, 2, 1), (14, 70, 3, 0),
+                                                (4, 310, 30000, 1), (3, 150, 60000, 0)])
+def test_gradient_sums(gpu, n, gates, batch, fuse):
+    from tensorcircuit_amd import _lib, engine
+
+    rng = np.random.default_rng(gates + batch)
+    specs, ops = [], []
+    kinds = [("x", _lib.G_RX), ("y", _lib.G_RY), ("z", _lib.G_RZ)]
+    for i in range(gates):
+        name, kind = kinds[i % 3]
+        q = int(rng.integers(n))
+        # every third gate shares its parameter with the one before
+        p = i - 1 if i % 3 == 2 else i
+        specs.append(engine.GateSpec(kind, (q,), p, 0.0, 1.0, None))
+        ops.append((name, q, p))
+        if i % 7 == 0:
+            cx = np.eye(4)[[0, 1, 3, 2]].astype(np.complex128)
+            a, b = (int(x) for x in rng.choice(n, 2, replace=False))
+            specs.append(engine.GateSpec(_lib.G_MAT, (a, b), -1, 0.0, 1.0, cx))
+            ops.append(("cx", a, b))
+    prog = engine.Program(n, specs, gates, fuse=fuse)
+    codes, w = rng.integers(0, 4, size=(4, n)).astype(np.int8), rng.standard_normal(4)
+    ham = engine.PauliSum(n, codes, w, jit=0)
+    terms = [(float(w[k]), list(codes[k])) for k in range(4)]
+    params = torch.as_tensor(rng.uniform(-2, 2, (batch, gates)))
+    e, g = prog.energy_grad(params.cuda(), ham, batch, "complex128")
+    e, g = np_of(e), np_of(g)
+    pauli = {"x": np.array([[0, 1], [1, 0]]), "y": np.array([[0, -1j], [1j, 0]]), "z": np.diag([1, -1])}
+
+    def turn(s, m, q):
+        return np.einsum("ij,ajb->aib", m, s.reshape(2**q, 2, -1)).reshape(-1)
+
+    for b in (0, batch // 2, batch - 1):
+        th = params[b].numpy()
+        s = np.zeros(2**n, dtype=np.complex128)
+        s[0] = 1.0
+        for name, q, p in ops:
+            if name == "cx":
+                idx = np.arange(2**n)
+                s = s[np.where(idx >> (n - 1 - q) & 1, idx ^ (1 << (n - 1 - p)), idx)]
+            else:
+                s = turn(s, np.cos(th[p] / 2) * np.eye(2) - 1j * np.sin(th[p] / 2) * pauli[name], q)
+        lam = sv.pauli_sum_apply(s, n, terms)
+        ref_e, ref = np.vdot(s, lam).real, np.zeros(gates)
+        for name, q, p in reversed(ops):
+            if name == "cx":
+                idx = np.arange(2**n)
+                src = np.where(idx >> (n - 1 - q) & 1, idx ^ (1 << (n - 1 - p)), idx)
+                s, lam = s[src], lam[src]
+            else:
+                ref[p] += np.imag(np.vdot(lam, turn(s, pauli[name], q)))
+                m = np.cos(th[p] / 2) * np.eye(2) + 1j * np.sin(th[p] / 2) * pauli[name]
+                s, lam = turn(s, m, q), turn(lam, m, q)
+        # each gate is off by a few units of rounding of the state it acts on,
+        # there and back, for state and adjoint (of norm <= sum |w|); two
+        # gates at most share a parameter
+        tol = 2 * (16 * gates + 2**n) * 2.0**-53 * np.abs(w).sum()
+        assert abs(e[b] - ref_e) <= tol
+        assert np.abs(g[b] - ref).max() <= tol
