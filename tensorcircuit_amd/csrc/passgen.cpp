@@ -259,12 +259,30 @@ struct Gen {
                x.c_str(), P, r, P, r, P, r, P, r));
     }
   }
-  void op_dg(const char* a, const std::string& pre) {
+  // for every entry of a merged diagonal the first one that equals it, or -1
+  // where it is one: one coefficient per distinct entry (2 of them for two
+  // rz's are 3 of 32), no work for ones
+  std::vector<int> dg_reps(const DOp& op) const {
+    const DRecipe* r = nullptr;
+    for (const DRecipe& q : S.recipes)
+      if (q.kind < 0 && q.out == op.moff) r = &q;
+    std::vector<int> rep(nreg, -1);
+    std::vector<uint64_t> key(nreg, 0);
+    for (int j = 0; j < nreg; ++j) {
+      key[j] = dg_class(S, *r, j);
+      if (key[j] == 0 && !(op.flags & OP_F_ALL)) continue;
+      for (int q = 0; q <= j && rep[j] < 0; ++q)
+        if (key[q] == key[j]) rep[j] = q;
+    }
+    return rep;
+  }
+  void op_dg(const char* a, const std::vector<int>& rep, const std::string& pre) {
     const char* P = pre.c_str();
     for (int j = 0; j < nreg; ++j) {
+      if (rep[j] < 0) continue;
       const std::string x = var(a, j);
       line(fmt("{ const cT x = %s; %s = cT{%sg%dr * x.x - %sg%di * x.y, %sg%dr * x.y + %sg%di * x.x}; }", x.c_str(),
-               x.c_str(), P, j, P, j, P, j, P, j));
+               x.c_str(), P, rep[j], P, rep[j], P, rep[j], P, rep[j]));
     }
   }
   void op_u2(const char* a, int S0, int S1, const std::string& pre) {
@@ -329,11 +347,13 @@ struct Gen {
           line(fmt("const T %sd%dr = %s, %sd%di = %s%s;", P, r, mel(op.moff, 2 * r).c_str(), P, r, dag ? "-" : "",
                    mel(op.moff, 2 * r + 1).c_str()));
         break;
-      case OK_DG:
+      case OK_DG: {
+        const std::vector<int> rep = dg_reps(op);
         for (int j = 0; j < nreg; ++j)
-          line(fmt("const T %sg%dr = %s, %sg%di = %s%s;", P, j, mel(op.moff, 2 * j).c_str(), P, j, dag ? "-" : "",
-                   mel(op.moff, 2 * j + 1).c_str()));
-        break;
+          if (rep[j] == j)
+            line(fmt("const T %sg%dr = %s, %sg%di = %s%s;", P, j, mel(op.moff, 2 * j).c_str(), P, j, dag ? "-" : "",
+                     mel(op.moff, 2 * j + 1).c_str()));
+      } break;
       case OK_U2:
         for (int r = 0; r < 4; ++r)
           for (int c = 0; c < 4; ++c) {
@@ -363,7 +383,9 @@ struct Gen {
         break;
       case OK_D1: for (auto a : arrs) op_d1(a, op.s0, pre); break;
       case OK_D2: for (auto a : arrs) op_d2(a, op.s0, op.s1, pre); break;
-      case OK_DG: for (auto a : arrs) op_dg(a, pre); break;
+      case OK_DG:
+        for (auto a : arrs) op_dg(a, dg_reps(op), pre);
+        break;
       case OK_U2: for (auto a : arrs) op_u2(a, op.s0, op.s1, pre); break;
       case OK_CZ: for (auto a : arrs) op_cz(a, op.s0, op.s1); break;
       case OK_X1: {
@@ -613,7 +635,13 @@ std::string pass_body(const Program& P, const Sched& S, int pi, bool adj, int dt
   auto emit_adj_ops = [&](const DGroup& dg) -> bool {
       for (int o = dg.op0 + dg.nops - 1; o >= dg.op0; --o) {
         const DOp& op = S.dop[o];
-        if (op.kind == OK_DG && op.nmem > 0) {
+        if (op.kind == OK_DG && op.nmem == 1) {
+          const DMember& M = S.dmem[op.mem0];
+          G.line("{");
+          G.grad(M.gen, M.s0, M.s1, 0);
+          emit_grad("ga", M.gloc);
+          G.line("}");
+        } else if (op.kind == OK_DG && op.nmem > 0) {
           G.line("{");
           for (int j = 0; j < nreg; ++j) G.line(fmt("const T im%d = imcj(%s, %s);", j, G.lv(j).c_str(), G.pv(j).c_str()));
           // Z-generator sums sum_j (-1)^{bit b of j} im_j for every needed

@@ -489,6 +489,14 @@ bool diag_kind(const LGate& g) {
          (g.gen == GN_NONE || g.gen == GN_Z || g.gen == GN_ZZ || g.gen == GN_P1);
 }
 
+// table entries of a gate's recipe
+int recipe_slot(const Program& P, const LGate& g) {
+  if (g.src == TCM_G_RY) return kRySlot;
+  if (P.opts.jit && g.src == TCM_G_RZ) return kRzSlot;
+  if (P.opts.jit && g.src == TCM_G_RZZ) return kRzzSlot;
+  return layout_size(g.okind);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -640,7 +648,7 @@ static int lower(Program& P, const tcm_gate* gates, int32_t ngates) {
     }
     if (g.kind != TCM_G_MAT) {
       L.mslot = mslot;
-      mslot += L.src == TCM_G_RY ? kRySlot : layout_size(L.okind);
+      mslot += recipe_slot(P, L);
       if (L.param >= 0) {
         L.gop = P.ngop++;
         L.gfac = 2.0 * c * L.scale;
@@ -692,8 +700,9 @@ static void base_recipes(const Program& P, std::vector<DRecipe>& out, int* size)
     r.goff = g.goff;
     r.theta = g.theta;
     r.scale = g.scale;
+    r.extra = P.opts.jit && (g.src == TCM_G_RY || g.src == TCM_G_RZ || g.src == TCM_G_RZZ);
     out.push_back(r);
-    sz = std::max(sz, g.mslot + (g.src == TCM_G_RY ? kRySlot : layout_size(g.okind)));
+    sz = std::max(sz, g.mslot + recipe_slot(P, g));
   }
   *size = sz;
 }
@@ -738,9 +747,31 @@ static void sched_plain(const Program& P, Sched& S) {
   }
 }
 
+// DFactor::cls of a diagonal gate
+static int32_t factor_classes(const Program& P, const LGate& g) {
+  if (g.okind == OK_CZ) return 0x1000;
+  if (g.mslot >= 0 && g.src == TCM_G_RZ && P.opts.jit) return 0x10;
+  if (g.mslot >= 0 && g.src == TCM_G_RZZ && P.opts.jit) return 0x0110;
+  if (g.mslot >= 0 && g.src == TCM_G_PHASE) return 0x10;
+  const int d = g.okind == OK_D1 ? 2 : 4;
+  int32_t c = 0;
+  for (int r = 0; r < d; ++r) {
+    int k = r + 1;
+    if (g.mslot < 0 && g.cslot >= 0) {  // constant: entries that are one, or equal an earlier one
+      const double* e = &P.ctab[g.cslot];
+      if (e[2 * r] == 1.0 && e[2 * r + 1] == 0.0) k = 0;
+      for (int q = r - 1; q >= 0 && k; --q)
+        if (e[2 * q] == e[2 * r] && e[2 * q + 1] == e[2 * r + 1]) k = q + 1;
+    }
+    c |= k << 4 * r;
+  }
+  return c;
+}
+
+// `scalars` collects the first entries that the rz and rzz factors leave out
 static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
                             const std::vector<int>& local_of_bit,
-                            const std::vector<int>& gloc_of_gop, DGroup& dg) {
+                            const std::vector<int>& gloc_of_gop, DGroup& dg, std::vector<DFactor>& scalars) {
   // slot of a tile-local bit inside this group
   auto slot_of = [&](int global_bit) {
     int lb = local_of_bit[global_bit];
@@ -749,16 +780,14 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
     return -1;
   };
   dg.op0 = (int)S.dop.size();
-  // the table-driven kernels know diagonals only as tables over the group's
-  // slots; compiled passes keep a lone one in its own form
-  const size_t merge = S.R == kTileSlots && !P.opts.jit ? 1 : 2;
   const auto& gl = hg.gates;
   size_t i = 0;
   while (i < gl.size()) {
     // maximal run of mergeable diagonal gates
     size_t j = i;
     while (j < gl.size() && diag_kind(P.gates[gl[j]])) ++j;
-    if (j - i >= merge) {
+    // a lone CZ of a compiled pass is a few sign changes
+    if (j - i >= 2 || (j > i && !(P.opts.jit && P.gates[gl[i]].okind == OK_CZ))) {
       DRecipe r{};
       r.kind = -1;
       r.out = S.mtab_size;
@@ -780,6 +809,13 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
         f.layout = g.okind;
         f.s0 = slot_of(g.bits[0]);
         f.s1 = g.nq > 1 ? slot_of(g.bits[1]) : -1;
+        f.cls = factor_classes(P, g);
+        if (P.opts.jit && g.mslot >= 0 && (g.src == TCM_G_RZ || g.src == TCM_G_RZZ)) {
+          const bool rz = g.src == TCM_G_RZ;
+          scalars.push_back(DFactor{f.src, DF_SCALAR, -1, -1, rz ? kRzFirst : kRzzFirst, 0});
+          f.src += rz ? kRzOne : kRzzOne;
+          f.low = rz ? kRzLow - kRzOne : kRzzLow - kRzzOne;
+        }
         S.factors.push_back(f);
         if (g.gop >= 0) {
           DMember m{};
@@ -818,6 +854,52 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
     ++i;
   }
   dg.nops = (int)S.dop.size() - dg.op0;
+}
+
+// class of entry j of a merged diagonal: the classes of its factors' entries
+// (0: every factor's entry is one)
+uint64_t dg_class(const Sched& S, const DRecipe& r, int j) {
+  uint64_t key = 0;
+  for (int f = 0; f < r.nfac; ++f) {
+    const DFactor& F = S.factors[r.goff + f];
+    const int b0 = (j >> F.s0) & 1;
+    const int idx = F.layout == OK_D1 ? b0 : b0 << 1 | ((j >> F.s1) & 1);
+    const int c = (F.cls >> 4 * idx) & 15;
+    if (c) key = (key ^ (uint64_t)(f * 16 + c)) * 0x9E3779B97F4A7C15ull + 1;
+  }
+  return key;
+}
+
+// The rz and rzz of a pass are used over their first entry, so that the
+// merged diagonals of one or two qubits leave half or a quarter of the
+// amplitudes alone; the pass's diagonal with the most other entries takes the
+// product of the first entries (scalars commute with everything).
+static void fold_scalars(Sched& S, const DPass& dp, const std::vector<DFactor>& scalars) {
+  DOp* best = nullptr;
+  DRecipe* rec = nullptr;
+  int most = -1;
+  for (int g = 0; g < dp.ngroups; ++g) {
+    const DGroup& dg = S.dgroup[dp.group0 + g];
+    for (int o = dg.op0; o < dg.op0 + dg.nops; ++o) {
+      if (S.dop[o].kind != OK_DG) continue;
+      DRecipe* r = nullptr;
+      for (DRecipe& q : S.recipes)
+        if (q.kind < 0 && q.out == S.dop[o].moff) r = &q;
+      int c = 0;
+      for (int j = 0; j < (1 << S.R); ++j) c += dg_class(S, *r, j) != 0;
+      if (c > most) {
+        most = c;
+        best = &S.dop[o];
+        rec = r;
+      }
+    }
+  }
+  const int g0 = (int)S.factors.size();
+  for (int f = 0; f < rec->nfac; ++f) S.factors.push_back(DFactor(S.factors[rec->goff + f]));
+  rec->goff = g0;
+  rec->extra = (int)scalars.size();
+  S.factors.insert(S.factors.end(), scalars.begin(), scalars.end());
+  best->flags |= OP_F_ALL;
 }
 
 static void tile_run(const Program& P, Sched& S, const std::vector<int>& items, uint64_t lmask, int cap) {
@@ -1284,6 +1366,7 @@ static void sched_fused(const Program& P, Sched& S, int k, int R, int Lwant, boo
       }
     dp.ngop = ngop;
     S.max_ngop_pass = std::max(S.max_ngop_pass, ngop);
+    std::vector<DFactor> scalars;
     for (const HGroup& hg : hp.groups) {
       DGroup dg{};
       std::memset(&dg, 0, sizeof dg);
@@ -1310,11 +1393,12 @@ static void sched_fused(const Program& P, Sched& S, int k, int R, int Lwant, boo
           dg.S[j] = (int32_t)swz_host(t);
         }
       }
-      build_group_ops(P, S, hg, local_of_bit, gloc_of_gop, dg);
+      build_group_ops(P, S, hg, local_of_bit, gloc_of_gop, dg, scalars);
       for (int o = dg.op0; o < dg.op0 + dg.nops; ++o)
         if (S.dop[o].kind == OK_U2 || (R == kTileSlots && S.dop[o].kind == OK_D2) || S.dop[o].gen == GN_M2) dp.full = 1;
       S.dgroup.push_back(dg);
     }
+    if (!scalars.empty()) fold_scalars(S, dp, scalars);
     if (R == kTileSlots) stage_pass(S, hp, dp, adj);
     S.dpass.push_back(dp);
   }

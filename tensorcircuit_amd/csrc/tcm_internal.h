@@ -68,7 +68,8 @@ struct DOp {
 // OP_F_SHEAR: an ry rotation whose table entry also holds the three-shear
 // form of its reduced angle (see k_prep): entries 4, 5, 6 = t, s, sigma
 // OP_F_RX: an rx rotation
-enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2, OP_F_RX = 4 };
+// OP_F_ALL: a merged diagonal with no entry that is known to be one
+enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2, OP_F_RX = 4, OP_F_ALL = 8 };
 
 // Gradient member of an OK_DG op (diagonal generator on slots of the group).
 struct DMember {
@@ -150,7 +151,9 @@ struct DRecipe {
   int32_t goff;    // EXP1 generator (constant table), or DG: first factor
   int32_t nfac;    // DG: number of factors
   int32_t R;       // DG: register slots
-  int32_t pad;
+  int32_t extra;   // RY, RZ, RZZ: also the entries that only compiled passes
+                   // read (kRySlot, kRzSlot, kRzzSlot); DG: scalar
+                   // factors (DFactor::layout DF_SCALAR) after the nfac others
   double theta, scale;
 };
 
@@ -166,13 +169,24 @@ struct DGopSum {
 // [-pi/2, pi/2] with R(phi) = sigma R(phi'), t = tan(phi' / 2), s' = sin phi'
 constexpr int kRySlot = 8;
 
+// Table entries of rz and rzz recipes of compiled programs: the exact
+// diagonal, then (from kRzOne, or kRzzOne) the diagonal over its first entry,
+// whose entries are 1 or e^{i angle}, the part of these that the working type
+// cuts off, and that of the first entry
+constexpr int kRzOne = 4, kRzLow = 8, kRzFirst = 12, kRzSlot = 16;
+constexpr int kRzzOne = 8, kRzzLow = 16, kRzzFirst = 24, kRzzSlot = 32;
+
 // Factor of a DG recipe: a diagonal (D1 or D2 layout, per-batch or constant)
 // evaluated on slots s0 (, s1) of the group index.
 struct DFactor {
   int32_t src;     // >= 0 per-batch offset; < 0 constant offset (-src-1)
-  int32_t layout;  // OK_D1, OK_D2, OK_CZ
+  int32_t layout;  // OK_D1, OK_D2, OK_CZ; DF_SCALAR: the complex number at src
   int32_t s0, s1;
+  int32_t low;     // 0, or the distance from src to the cut-off part
+  int32_t cls;     // entry r's class in bits 4r: 0 = exactly one, equal
+                   // classes = equal entries
 };
+constexpr int DF_SCALAR = 100;
 
 // ---------------------------------------------------------------------------
 // Host-side program
@@ -310,5 +324,7 @@ int set_error(int code, const char* fmt, ...);
 inline uint32_t swz_host(uint32_t t) {
   return t ^ (((t >> 4) ^ (t >> 8) ^ (t >> 12) ^ (t >> 16)) & 0xFu);
 }
+
+uint64_t dg_class(const Sched& S, const DRecipe& r, int j);
 
 }  // namespace tcm

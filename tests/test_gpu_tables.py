@@ -309,3 +309,55 @@ def test_gradient_sums(gpu, n, gates, batch, fuse):
         tol = 2 * (16 * gates + 2**n) * 2.0**-53 * np.abs(w).sum()
         assert abs(e[b] - ref_e) <= tol
         assert np.abs(g[b] - ref).max() <= tol
+
+
+# compiled passes: merged diagonals of one, two and more qubits (rz, rzz,
+# phase, T, CZ, alone and in runs) between rotations and CNOTs; widths of one
+# tile, one tile exactly and several, where a pass's diagonals are over
+# their first entries but for one
+@pytest.mark.parametrize("n,gates", [(10, 3), (10, 40), (11, 80), (13, 120), (14, 200), (20, 90)])
+def test_compiled_diagonals(gpu, n, gates):
+    from tensorcircuit_amd import _lib, engine
+
+    rng = np.random.default_rng(31 * n + gates)
+    t = np.diag([1.0, np.exp(0.25j * np.pi)])
+    cz, cx = np.diag([1.0, 1, 1, -1]).astype(np.complex128), np.eye(4)[[0, 1, 3, 2]].astype(np.complex128)
+    pick = ["ry", "rz", "rz", "rzz", "phase", "t", "cz", "cx", "rx"]
+    one = {"ry": _lib.G_RY, "rz": _lib.G_RZ, "phase": _lib.G_PHASE, "rx": _lib.G_RX}
+    specs, p = [engine.GateSpec(_lib.G_RZ, (n - 1,), 0, 0.0, 1.0, None)], 1
+    for _ in range(gates):
+        name = pick[rng.integers(len(pick))]
+        a, b = (int(x) for x in rng.choice(n, 2, replace=False))
+        if name in one:
+            specs.append(engine.GateSpec(one[name], (a,), p, 0.0, 1.0, None))
+            p += 1
+        elif name == "rzz":
+            specs.append(engine.GateSpec(_lib.G_RZZ, (a, b), p, 0.0, 1.0, None))
+            p += 1
+        else:
+            q = (a,) if name == "t" else (a, b)
+            specs.append(engine.GateSpec(_lib.G_MAT, q, -1, 0.0, 1.0, {"t": t, "cz": cz, "cx": cx}[name]))
+    codes, w = rng.integers(0, 4, size=(5, n)).astype(np.int8), rng.standard_normal(5)
+    ham = engine.PauliSum(n, codes, w, jit=0)
+    params = torch.as_tensor(rng.uniform(-4, 4, (2, p)))
+    # one kernel per gate
+    plain = engine.Program(n, specs, p, fuse=0)
+    ref, _ = plain.forward(params.cuda(), 2, "complex128")
+    re, rg = plain.energy_grad(params.cuda(), ham, 2, "complex128")
+    prog = engine.Program(n, specs, p, fuse=1, jit=1)
+    for dt, name in ((torch.complex64, "complex64"), (torch.complex128, "complex128")):
+        th = params.cuda().to(torch.float32 if dt == torch.complex64 else torch.float64)
+        if dt == torch.complex64:  # the angles as they were rounded
+            ref, _ = plain.forward(th.double(), 2, "complex128")
+            re, rg = plain.energy_grad(th.double(), ham, 2, "complex128")
+        else:
+            ref, _ = plain.forward(params.cuda(), 2, "complex128")
+            re, rg = plain.energy_grad(params.cuda(), ham, 2, "complex128")
+        psi, _ = prog.forward(th, 2, name)
+        e, g = prog.energy_grad(th, ham, 2, name)
+        # a gate moves a normalised state by a few units of rounding; there
+        # and back for state and adjoint, whose norm is at most sum |w|
+        tol = 4 * (4 + len(specs)) * UNIT[dt]
+        assert np.abs(np_of(psi) - np_of(ref)).max() <= tol
+        assert np.abs(np_of(e) - np_of(re)).max() <= 2 * tol * np.abs(w).sum()
+        assert np.abs(np_of(g) - np_of(rg)).max() <= 4 * tol * np.abs(w).sum()
