@@ -149,6 +149,21 @@ __device__ __forceinline__ void store_shears(float* o, double ph) {
     }
 }
 
+// The entries kRotShear.. of an rx or ry recipe: three shears (Paeth), the
+// rotation by phi' is x -= t y, y += s x, x -= t y with t = tan(phi' / 2),
+// s = sin phi'; phi' is phi reduced into [-pi/2, pi/2] (|t| <= 1) by
+// R(phi) = -R(phi - pi), the sign kept in sigma.
+template <typename T>
+__device__ __forceinline__ void put_rotation(T* o, double phi) {
+  double ph = remainder(phi, 2.0 * M_PI), sigma = 1.0;
+  if (fabs(ph) > 0.5 * M_PI) {
+    ph -= copysign(M_PI, ph);
+    sigma = -1.0;
+  }
+  store_shears(o + kRotShear, ph);
+  o[kRotSigma] = (T)sigma;
+}
+
 // ---------------------------------------------------------------------------
 // matrix preparation: a block evaluates every recipe of one batch item of one
 // schedule from its parameters.  A chain of a few loads and 64-bit sines, so
@@ -181,25 +196,13 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
         double c, s;
         sincos(0.5 * a, &s, &c);
         o[0] = (T)c; o[1] = 0; o[2] = 0; o[3] = (T)-s; o[4] = 0; o[5] = (T)-s; o[6] = (T)c; o[7] = 0;
+        if (r.extra) put_rotation(o, 0.5 * a);
       } break;
       case TCM_G_RY: {
         double c, s;
         sincos(0.5 * a, &s, &c);
         o[0] = (T)c; o[1] = (T)-s; o[2] = (T)s; o[3] = (T)c;
-        if (r.extra) {
-          // three-shear form (Paeth): the rotation by phi' is x -= t y,
-          // y += s' x, x -= t y with t = tan(phi' / 2), s' = sin phi'; phi' is
-          // phi = a / 2 reduced into [-pi/2, pi/2] (|t| <= 1) by
-          // R(phi) = -R(phi - pi), the sign kept in sigma
-          double ph = remainder(0.5 * a, 2.0 * M_PI);
-          double sg = 1.0;
-          if (fabs(ph) > 0.5 * M_PI) {
-            ph -= copysign(M_PI, ph);
-            sg = -1.0;
-          }
-          store_shears(o + 4, ph);
-          o[6] = (T)sg; o[7] = 0;
-        }
+        if (r.extra) put_rotation(o, 0.5 * a);
       } break;
       case TCM_G_RZ: {
         double c, s;

@@ -75,6 +75,19 @@ __device__ __forceinline__ unsigned swz(unsigned t) {
 // LDS element at a byte offset (addresses are kept in bytes so the XOR
 // swizzle needs no per-access shift)
 #define LDSB(arr, off) (*reinterpret_cast<cT*>(reinterpret_cast<char*>(arr) + (off)))
+// Real rotations of a pair, in the plane of its real and of its imaginary
+// parts (ry) or crosswise (rx), as three shears of each: three multiply-adds
+// where the matrix takes four (ry), or eight (rx as a complex matrix).
+__device__ __forceinline__ void shear_y(cT& x, cT& y, T t, T s) {
+  x.x -= t * y.x; x.y -= t * y.y;
+  y.x += s * x.x; y.y += s * x.y;
+  x.x -= t * y.x; x.y -= t * y.y;
+}
+__device__ __forceinline__ void shear_x(cT& x, cT& y, T t, T s) {
+  x.x += t * y.y; x.y -= t * y.x;
+  y.x += s * x.y; y.y -= s * x.x;
+  x.x += t * y.y; x.y -= t * y.x;
+}
 // sign bit of a table entry (1 for negative)
 __device__ __forceinline__ unsigned sgnb(float x) { return __float_as_uint(x) >> 31; }
 __device__ __forceinline__ unsigned sgnb(double x) { return (unsigned)((unsigned long long)__double_as_longlong(x) >> 63); }
@@ -204,19 +217,11 @@ struct Gen {
                pre.c_str()));
     }
   }
-  // real rotation as three shears per real 2-vector (x, y) of a pair:
-  // x -= t y; y += s x; x -= t y (three fused multiply-adds instead of two
-  // multiplies and two multiply-adds)
-  void op_shear(const char* a, int S0, const std::string& pre) {
-    const int m = 1 << S0;
-    const char* P = pre.c_str();
-    for (int j = 0; j < nreg; ++j) {
-      if (j & m) continue;
-      const std::string x = var(a, j), y = var(a, j | m);
-      line(fmt("%s.x -= %st * %s.x; %s.y -= %st * %s.y;", x.c_str(), P, y.c_str(), x.c_str(), P, y.c_str()));
-      line(fmt("%s.x += %ss * %s.x; %s.y += %ss * %s.y;", y.c_str(), P, x.c_str(), y.c_str(), P, x.c_str()));
-      line(fmt("%s.x -= %st * %s.x; %s.y -= %st * %s.y;", x.c_str(), P, y.c_str(), x.c_str(), P, y.c_str()));
-    }
+  // rx or ry on every pair (fn: shear_x or shear_y)
+  void op_rot(const char* a, const DOp& op, const std::string& fn, const std::string& args) {
+    for (int j = 0; j < nreg; ++j)
+      if (!(j >> op.s0 & 1))
+        line(fmt("%s(%s, %s, %s);", fn.c_str(), var(a, j).c_str(), var(a, j | 1 << op.s0).c_str(), args.c_str()));
   }
   // negate every register of the arrays when the product of the pass's
   // sigmas is -1 (sign bits XORed; block-uniform)
@@ -329,13 +334,9 @@ struct Gen {
                    mel(op.moff, 6).c_str(), P, mel(op.moff, 7).c_str()));
         break;
       case OK_R1:
-        if (op.flags & OP_F_SHEAR)  // R(phi')^dagger = R(-phi'): t and s' change sign
-          line(fmt("const T %st = %s%s, %ss = %s%s;", P, dag ? "-" : "", mel(op.moff, 4).c_str(), P, dag ? "-" : "",
-                   mel(op.moff, 5).c_str()));
-        else
-          line(fmt("const T %sa = %s, %sb = %s, %sc = %s, %sd = %s;", P, mel(op.moff, 0).c_str(), P,
-                   mel(op.moff, dag ? 2 : 1).c_str(), P, mel(op.moff, dag ? 1 : 2).c_str(), P,
-                   mel(op.moff, 3).c_str()));
+        line(fmt("const T %sa = %s, %sb = %s, %sc = %s, %sd = %s;", P, mel(op.moff, 0).c_str(), P,
+                 mel(op.moff, dag ? 2 : 1).c_str(), P, mel(op.moff, dag ? 1 : 2).c_str(), P,
+                 mel(op.moff, 3).c_str()));
         break;
       case OK_D1:
         line(fmt("const T %sd0r = %s, %sd0i = %s%s, %sd1r = %s, %sd1i = %s%s;", P, mel(op.moff, 0).c_str(), P,
@@ -370,17 +371,19 @@ struct Gen {
   // apply op to the arrays in `arrs` (one or two names)
   void apply(const DOp& op, const std::vector<const char*>& arrs, int id) {
     const std::string pre = fmt("c%d_", id);
+    if (op.flags & (OP_F_SHEAR | OP_F_RX)) {
+      const char* P = pre.c_str();
+      const std::string ax = op.flags & OP_F_RX ? "_x" : "_y", sg = dag ? "-" : "";
+      line(fmt("const T %st = %s%s, %ss = %s%s;", P, sg.c_str(), mel(op.moff, kRotShear).c_str(), P, sg.c_str(),
+               mel(op.moff, kRotShear + 1).c_str()));
+      for (auto a : arrs) op_rot(a, op, "shear" + ax, fmt("%st, %ss", P, P));
+      frame.push_back(mel(op.moff, kRotSigma));
+      return;
+    }
     coeffs(op, pre);
     switch (op.kind) {
       case OK_U1: for (auto a : arrs) op_u1(a, op.s0, pre); break;
-      case OK_R1:
-        if (op.flags & OP_F_SHEAR) {
-          for (auto a : arrs) op_shear(a, op.s0, pre);
-          frame.push_back(mel(op.moff, 6));
-        } else {
-          for (auto a : arrs) op_r1(a, op.s0, pre);
-        }
-        break;
+      case OK_R1: for (auto a : arrs) op_r1(a, op.s0, pre); break;
       case OK_D1: for (auto a : arrs) op_d1(a, op.s0, pre); break;
       case OK_D2: for (auto a : arrs) op_d2(a, op.s0, op.s1, pre); break;
       case OK_DG:

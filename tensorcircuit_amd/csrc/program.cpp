@@ -491,7 +491,7 @@ bool diag_kind(const LGate& g) {
 
 // table entries of a gate's recipe
 int recipe_slot(const Program& P, const LGate& g) {
-  if (g.src == TCM_G_RY) return kRySlot;
+  if (P.opts.jit && (g.src == TCM_G_RX || g.src == TCM_G_RY)) return kRotSlot;
   if (P.opts.jit && g.src == TCM_G_RZ) return kRzSlot;
   if (P.opts.jit && g.src == TCM_G_RZZ) return kRzzSlot;
   return layout_size(g.okind);
@@ -700,7 +700,7 @@ static void base_recipes(const Program& P, std::vector<DRecipe>& out, int* size)
     r.goff = g.goff;
     r.theta = g.theta;
     r.scale = g.scale;
-    r.extra = P.opts.jit && (g.src == TCM_G_RY || g.src == TCM_G_RZ || g.src == TCM_G_RZZ);
+    r.extra = P.opts.jit && (g.src == TCM_G_RX || g.src == TCM_G_RY || g.src == TCM_G_RZ || g.src == TCM_G_RZZ);
     out.push_back(r);
     sz = std::max(sz, g.mslot + recipe_slot(P, g));
   }

@@ -65,10 +65,9 @@ struct DOp {
 };
 
 // DOp flags
-// OP_F_SHEAR: an ry rotation whose table entry also holds the three-shear
-// form of its reduced angle (see k_prep): entries 4, 5, 6 = t, s, sigma
-// OP_F_RX: an rx rotation
-// OP_F_ALL: a merged diagonal with no entry that is known to be one
+// OP_F_SHEAR, OP_F_RX: ry, rx rotations (compiled passes: by three shears, the
+// entries kRotShear.. of the recipe)
+// OP_F_ALL: a merged diagonal that takes the pass's scalars
 enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2, OP_F_RX = 4, OP_F_ALL = 8 };
 
 // Gradient member of an OK_DG op (diagonal generator on slots of the group).
@@ -151,8 +150,8 @@ struct DRecipe {
   int32_t goff;    // EXP1 generator (constant table), or DG: first factor
   int32_t nfac;    // DG: number of factors
   int32_t R;       // DG: register slots
-  int32_t extra;   // RY, RZ, RZZ: also the entries that only compiled passes
-                   // read (kRySlot, kRzSlot, kRzzSlot); DG: scalar
+  int32_t extra;   // RX, RY, RZ, RZZ: also entries that only compiled passes
+                   // read (kRotSlot, kRzSlot, kRzzSlot); DG: scalar
                    // factors (DFactor::layout DF_SCALAR) after the nfac others
   double theta, scale;
 };
@@ -164,10 +163,11 @@ struct DGopSum {
   int32_t row, ngop, slots, pad;
 };
 
-// Table entries of an ry recipe: [c, -s, s, c] of the exact rotation by
-// phi = angle / 2, then [t, s', sigma, 0]: phi reduced to phi' in
-// [-pi/2, pi/2] with R(phi) = sigma R(phi'), t = tan(phi' / 2), s' = sin phi'
-constexpr int kRySlot = 8;
+// Table entries of rx and ry recipes of compiled programs: the exact matrix
+// (rx 8, ry 4 entries) by phi = angle / 2, then for three shears t =
+// tan(phi' / 2), s = sin phi' and sigma, phi reduced to phi' in [-pi/2, pi/2]
+// with R(phi) = sigma R(phi')
+constexpr int kRotShear = 8, kRotSigma = 10, kRotSlot = 12;
 
 // Table entries of rz and rzz recipes of compiled programs: the exact
 // diagonal, then (from kRzOne, or kRzzOne) the diagonal over its first entry,

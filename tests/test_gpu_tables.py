@@ -361,3 +361,35 @@ def test_compiled_diagonals(gpu, n, gates):
         assert np.abs(np_of(psi) - np_of(ref)).max() <= tol
         assert np.abs(np_of(e) - np_of(re)).max() <= 2 * tol * np.abs(w).sum()
         assert np.abs(np_of(g) - np_of(rg)).max() <= 4 * tol * np.abs(w).sum()
+
+
+# rx and ry of compiled passes as shears: small angles, angles near pi and
+# beyond, and middling ones, with and without diagonals
+@pytest.mark.parametrize("n,gates,diag", [(10, 30, True), (10, 30, False), (13, 120, True), (15, 200, True)])
+def test_compiled_rotations(gpu, n, gates, diag):
+    from tensorcircuit_amd import _lib, engine
+
+    rng = np.random.default_rng(5 * n + gates)
+    cx = np.eye(4)[[0, 1, 3, 2]].astype(np.complex128)
+    specs, p = [], 0
+    for _ in range(gates):
+        k = rng.integers(4 if diag else 3)
+        a, b = (int(x) for x in rng.choice(n, 2, replace=False))
+        if k == 2:
+            specs.append(engine.GateSpec(_lib.G_MAT, (a, b), -1, 0.0, 1.0, cx))
+            continue
+        specs.append(engine.GateSpec([_lib.G_RX, _lib.G_RY, None, _lib.G_RZ][k], (a,), p, 0.0, 1.0, None))
+        p += 1
+    th = rng.normal(0, 0.2, (3, p))
+    th[1, : p // 2] += 2 * np.pi  # cosines near -1
+    th[1, p // 3] = 3.1
+    th[2] = rng.uniform(1.2, 1.6, p)
+    th = torch.as_tensor(th).cuda()
+    ref, _ = engine.Program(n, specs, p, fuse=0).forward(th.float().double(), 3, "complex128")
+    exact, _ = engine.Program(n, specs, p, fuse=0).forward(th, 3, "complex128")
+    prog = engine.Program(n, specs, p, fuse=1, jit=1)
+    # each gate moves a normalised state by a few units of rounding
+    for name, x, want in (("complex64", th.float(), ref), ("complex128", th, exact)):
+        psi, _ = prog.forward(x, 3, name)
+        tol = 4 * (4 + len(specs)) * UNIT[psi.dtype]
+        assert np.abs(np_of(psi) - np_of(want)).max() <= tol
