@@ -267,14 +267,13 @@ class Circuit:
             return torch.zeros(0, dtype=rdt, device=dev)
         if all(not isinstance(t, torch.Tensor) for t in thetas):
             return torch.tensor([float(np.real(t)) for t in thetas], dtype=rdt, device=dev)
-        ts = []
-        for t in thetas:
-            if not isinstance(t, torch.Tensor):
-                t = torch.tensor(float(np.real(t)), dtype=rdt)
-            if t.is_complex():
-                t = torch.real(t)
-            ts.append(t.reshape(()).to(device=dev, dtype=rdt))
-        return torch.stack(ts)
+        ts = [t if isinstance(t, torch.Tensor) else torch.tensor(float(np.real(t)), dtype=rdt) for t in thetas]
+        ts = [t if t.dim() == 0 else t.reshape(()) for t in ts]
+        if any(t.dtype != ts[0].dtype or t.device != ts[0].device for t in ts):
+            ts = [(torch.real(t) if t.is_complex() else t).to(device=dev, dtype=rdt) for t in ts]
+        # one conversion of the stack, not one (and its backward) per angle
+        p = torch.stack(ts)
+        return (torch.real(p) if p.is_complex() else p).to(device=dev, dtype=rdt)
 
     def _program(self, specs: List[GateSpec], nparams: int) -> engine.Program:
         return engine.get_program(self._nstate, specs, nparams, fuse=1)

