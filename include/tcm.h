@@ -171,6 +171,13 @@ int tcm_forward(tcm_program* prog, int32_t dtype, const void* params,
                 int32_t init_zero, void* ckpts, void* workspace,
                 int64_t ws_bytes, void* stream);
 
+/* tcm_forward on the states `inputs` (batch x 2^n, left as they are), with the
+ * result in `state`; the two may not overlap. */
+int tcm_forward_from(tcm_program* prog, int32_t dtype, const void* params,
+                     int64_t param_stride, const void* inputs, void* state,
+                     int64_t batch, void* ckpts, void* workspace,
+                     int64_t ws_bytes, void* stream);
+
 /* ---- Pauli sums -----------------------------------------------------------
  * codes: host int8 [nterms][nqubits], 0=I 1=X 2=Y 3=Z (quantum.py:1025-1068);
  * coeffs: host real weights [nterms]. */

@@ -221,27 +221,29 @@ int64_t forward_ws(const Program& P, int dtype, int64_t batch) {
 }
 
 // one forward pass pi (tiled, matrix-core or plain); ckout: checkpoint copy
-// written by a tiled pass (nullable)
+// written by a tiled pass (nullable); src: the states a tiled or matrix-core
+// pass reads, default `state`
 template <typename T>
 int run_one_pass(Program& P, const Sched& S, const DeviceTables& D, int pi, const void* mtab, void* state,
-                 int64_t batch, void* ckout, hipStream_t st, bool zinit = false) {
+                 int64_t batch, void* ckout, hipStream_t st, bool zinit = false, const void* src = nullptr) {
   const int n = P.n;
+  if (!src) src = state;
   const bool mfma = S.k > 0 && S.dpass[pi].mfma;
   const bool tiled = S.k > 0 && S.dpass[pi].plain_op < 0 && !mfma;
   if (mfma) {
     if constexpr (std::is_same<T, float>::value) {
       if (!launch_mfma_tile(S.dpass[pi], (const DPass*)D.dpass, pi, (const DOp*)D.dop, (const int32_t*)D.ukbits,
-                            (const uint32_t*)D.runoff, D.ctab, state, n, batch, st))
+                            (const uint32_t*)D.runoff, D.ctab, src, state, n, batch, st))
         return set_error(TCM_E_UNSUPPORTED, "matrix-core tile pass %d: %d blocks on %d tile bits not supported", pi,
                          S.dpass[pi].nmop, S.dpass[pi].k);
     } else
       return set_error(TCM_E_UNSUPPORTED, "matrix-core passes are complex64 only");
   } else if (tiled) {
     if (!S.jit.empty() && S.jit[pi].kernel >= 0) {
-      if (int rc = jit_launch_fwd(S, D, pi, sizeof(T) == 8, mtab, D.ctab, state, batch, n, ckout, st, zinit ? 1 : 0))
+      if (int rc = jit_launch_fwd(S, D, pi, sizeof(T) == 8, mtab, D.ctab, src, state, batch, n, ckout, st, zinit ? 1 : 0))
         return rc;
     } else if (S.R == kTileSlots) {
-      launch_tile_fwd<T>(S, D, pi, mtab, D.ctab, state, state, batch, n, ckout, zinit, st);
+      launch_tile_fwd<T>(S, D, pi, mtab, D.ctab, src, state, batch, n, ckout, zinit, st);
     } else {
       return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", S.R);
     }
@@ -263,7 +265,8 @@ bool tile_first(const Sched& S) {
 // no tile pass or the initial state is a checkpoint
 template <typename T>
 int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const void* mtab, void* state,
-                       int64_t batch, void* ckpts, hipStream_t st, bool init_zero = false) {
+                       int64_t batch, void* ckpts, hipStream_t st, bool init_zero = false,
+                       const void* inputs = nullptr) {
   const int n = P.n;
   const int64_t N = 1ll << n;
   const int64_t ck_stride = batch * N;
@@ -273,6 +276,12 @@ int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const 
     for (int a : S.ckpt_after) ck0 = ck0 || a < 0;
   const bool zfirst = init_zero && !ck0 && tile_first(S);
   if (init_zero && !zfirst) launch_init_zero<T>(state, n, batch, st);
+  // a first pass over tiles reads the inputs itself (a 26-qubit state: 200 us
+  // of copying less); 16-byte loads
+  if (inputs && (ck0 || S.passes.empty() || S.k == 0 || S.dpass[0].plain_op >= 0 || ((uintptr_t)inputs & 15))) {
+    launch_copy<T>(state, inputs, ck_stride, st);
+    inputs = nullptr;
+  }
   // checkpoints of the initial state (before any pass)
   if (ckpts)
     for (size_t c = 0; c < S.ckpt_after.size(); ++c)
@@ -289,7 +298,8 @@ int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const 
           if (!ckout && tiled) ckout = ckpt_ptr(c);
           else extra.push_back(c);
         }
-    if (int rc = run_one_pass<T>(P, S, D, pi, mtab, state, batch, ckout, st, zfirst && pi == 0)) return rc;
+    if (int rc = run_one_pass<T>(P, S, D, pi, mtab, state, batch, ckout, st, zfirst && pi == 0, pi == 0 ? inputs : nullptr))
+      return rc;
     for (size_t c : extra) launch_copy<T>(ckpt_ptr(c), state, ck_stride, st);
   }
   return 0;
@@ -297,7 +307,8 @@ int run_forward_passes(Program& P, const Sched& S, const DeviceTables& D, const 
 
 template <typename T>
 int forward_impl(Program& P, int dtype, const void* params, int64_t pstride, void* state, int64_t batch,
-                 int init_zero, void* ckpts, void* ws, int64_t ws_bytes, hipStream_t st) {
+                 int init_zero, void* ckpts, void* ws, int64_t ws_bytes, hipStream_t st,
+                 const void* inputs = nullptr) {
   DeviceTables* D = nullptr;
   if (int rc = ensure_tables(P, dtype, 0, &D)) return rc;
   const Sched& S = P.sched[dtype][0];
@@ -307,7 +318,7 @@ int forward_impl(Program& P, int dtype, const void* params, int64_t pstride, voi
   PrepJobs J;
   add_prep<T>(J, S, *D, D->ctab, params, pstride, mtab, batch, st);
   launch_prep<T>(J, st);
-  if (int rc = run_forward_passes<T>(P, S, *D, mtab, state, batch, ckpts, st, init_zero != 0)) return rc;
+  if (int rc = run_forward_passes<T>(P, S, *D, mtab, state, batch, ckpts, st, init_zero != 0, inputs)) return rc;
   HIP_TRY(hipGetLastError(), "forward launch");
   return 0;
 }
@@ -771,8 +782,8 @@ int energy_grad_impl(Program& P, int dtype, const void* params, int64_t pstride,
   add_prep<T>(J, A, *DA, DA->ctab, params, pstride, w.mtab_a, batch, st);
   launch_prep<T>(J, st);
   // forward with checkpoints
-  if (inputs) launch_copy<T>(w.psi, inputs, batch * N, st);
-  if (int rc = run_forward_passes<T>(P, F, *DF, w.mtab_f, w.psi, batch, w.ckpt, st, inputs == nullptr)) return rc;
+  if (int rc = run_forward_passes<T>(P, F, *DF, w.mtab_f, w.psi, batch, w.ckpt, st, inputs == nullptr, inputs))
+    return rc;
   // energy and lambda = H psi
   if (int rc = pauli_energy_apply<T>(H, dtype, w.psi, w.lam, nullptr, batch, w.epart, true, true, st)) return rc;
   // reverse sweep, then energies and gradients from the partial sums
@@ -1139,6 +1150,20 @@ int tcm_forward(tcm_program* prog, int32_t dtype, const void* params, int64_t pa
   return dtype == TCM_C64
              ? forward_impl<float>(prog->p, dtype, params, param_stride, state, batch, init_zero, ckpts, workspace, ws_bytes, st)
              : forward_impl<double>(prog->p, dtype, params, param_stride, state, batch, init_zero, ckpts, workspace, ws_bytes, st);
+}
+
+int tcm_forward_from(tcm_program* prog, int32_t dtype, const void* params, int64_t param_stride, const void* inputs,
+                     void* state, int64_t batch, void* ckpts, void* workspace, int64_t ws_bytes, void* stream) {
+  if (!prog || !valid_dtype(dtype) || batch < 0 || (batch > 0 && (!state || !inputs)))
+    return set_error(TCM_E_ARG, "bad arguments to tcm_forward_from");
+  if (batch == 0) return 0;
+  if (prog->p.nparams > 0 && !params) return set_error(TCM_E_ARG, "params required");
+  if (param_stride < 0) return set_error(TCM_E_ARG, "param_stride < 0");
+  hipStream_t st = (hipStream_t)stream;
+  return dtype == TCM_C64 ? forward_impl<float>(prog->p, dtype, params, param_stride, state, batch, 0, ckpts, workspace,
+                                                ws_bytes, st, inputs)
+                          : forward_impl<double>(prog->p, dtype, params, param_stride, state, batch, 0, ckpts,
+                                                 workspace, ws_bytes, st, inputs);
 }
 
 int tcm_pauli_build(const int8_t* codes, const double* coeffs, int32_t nterms, int32_t nqubits, tcm_pauli** out) {

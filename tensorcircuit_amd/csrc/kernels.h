@@ -150,9 +150,9 @@ struct DeviceTables {
 
 // launch compiled pass kernels (jit.cpp)
 int jit_load(const Sched& S, DeviceTables& D);
-// zinit: the pass starts from |0..0> instead of reading `state`
+// zinit: the pass starts from |0..0> instead of reading `src` (`state` or others)
 int jit_launch_fwd(const Sched& S, const DeviceTables& D, int pi, int dt, const void* mtab, const void* ctab,
-                   void* state, int64_t batch, int n, void* ckout, hipStream_t st, int zinit = 0);
+                   const void* src, void* state, int64_t batch, int n, void* ckout, hipStream_t st, int zinit = 0);
 int jit_launch_adj(const Sched& S, const DeviceTables& D, int pi, int dt, const void* mtab, const void* ctab,
                    const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
                    double* part, int64_t pstride, hipStream_t st);
@@ -229,7 +229,7 @@ struct MeasureStep {
 // false if the pass does not fit the kernel (tile bits 10..13, at most
 // kMfmaTileMaxOps blocks)
 bool launch_mfma_tile(const DPass& P, const DPass* passes_dev, int pi, const DOp* dop_dev, const int32_t* ukbits_dev,
-                      const uint32_t* runoff_dev, const void* ctab, void* state, int n, int64_t batch,
+                      const uint32_t* runoff_dev, const void* ctab, const void* src, void* state, int n, int64_t batch,
                       hipStream_t st);
 template <typename T>
 void launch_probability(const void* psi, void* out, int64_t total, hipStream_t st);

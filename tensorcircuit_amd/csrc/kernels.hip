@@ -654,8 +654,9 @@ template <int K>
 __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ passes, int pi,
                                                    const DOp* __restrict__ dop, const int32_t* __restrict__ ukbits,
                                                    const uint32_t* __restrict__ runoff, const float* __restrict__ ct,
-                                                   float2* __restrict__ st, int64_t sstride, int64_t ntiles) {
-  // each thread moves PER2 pairs of adjacent amplitudes (16-byte accesses)
+                                                   const float2* src, float2* st, int64_t sstride, int64_t ntiles) {
+  // src: the states read, st itself or others (the first pass of a circuit on
+  // given inputs).  Each thread moves PER2 pairs of adjacent amplitudes (16-byte accesses)
   constexpr int NTHR = 512, PER2 = (1 << K) / (2 * NTHR), CHUNKS = 1 << (K - 10), NCOL = 1 << (K - 5);
   extern __shared__ __align__(16) unsigned char smem[];
   float2* tile = reinterpret_cast<float2*>(smem);
@@ -722,7 +723,7 @@ __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ pas
     return v;
   };
   // tile tt: batch item tt >> nbl; its block bits (ascending) hold the low nbl bits of tt
-  auto tile_ptr = [&](int64_t tt) {
+  auto tile_at = [&](int64_t tt) {
     const uint64_t blk = (uint64_t)tt & ((1ull << nbl) - 1);
     uint64_t m = bmask, base = 0;
     for (int i = 0; i < nbl; ++i) {
@@ -730,9 +731,10 @@ __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ pas
       if ((blk >> i) & 1) base |= low;
       m ^= low;
     }
-    return st + ((uint64_t)tt >> nbl) * sstride + base;
+    return (int64_t)(((uint64_t)tt >> nbl) * sstride + base);
   };
-  auto glb4 = [&](float2* sp, int it) -> tcm_v4f* { return reinterpret_cast<tcm_v4f*>(sp + roff[it] + dlo); };
+  auto in4 = [&](int64_t sp, int it) { return *reinterpret_cast<const tcm_v4f*>(src + sp + roff[it] + dlo); };
+  auto out4 = [&](int64_t sp, int it) -> tcm_v4f& { return *reinterpret_cast<tcm_v4f*>(st + sp + roff[it] + dlo); };
   const int lane = tid & 63, wave = tid >> 6;
   const int ai = lane & 31, ak = lane >> 5;
   // A operands of the pass's first two blocks (filled once staged)
@@ -778,9 +780,9 @@ __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ pas
     if (nmop > 1) block(1, [&](int q) { return a1[q]; });
     for (int o = 2; o < nmop; ++o) block(o, [&](int q) { return amat[o * 1024 + q * 64 + lane]; });
   };
-  float2* s = tile_ptr(t);
+  int64_t s = tile_at(t);
   tcm_v4f pre[PER2];
-  unrolled<PER2>([&](auto it) { pre[it] = *glb4(s, it); });
+  unrolled<PER2>([&](auto it) { pre[it] = in4(s, it); });
   unrolled<PER2>([&](auto it) { put4(it, pre[it]); });
   // the first two blocks' A operands stay in registers for every tile
   __syncthreads();
@@ -794,12 +796,12 @@ __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ pas
   for (;;) {
     const int64_t tn = t + gridDim.x;
     if (tn >= ntiles) break;
-    float2* sn = tile_ptr(tn);
-    unrolled<PER2>([&](auto it) { pre[it] = *glb4(sn, it); });
+    const int64_t sn = tile_at(tn);
+    unrolled<PER2>([&](auto it) { pre[it] = in4(sn, it); });
     __syncthreads();  // the tile (and, first time, the staged operands) in LDS
     blocks();
     unrolled<PER2>([&](auto it) {
-      *glb4(s, it) = get4(it);
+      out4(s, it) = get4(it);
       put4(it, pre[it]);
     });
     t = tn;
@@ -807,7 +809,7 @@ __global__ void __launch_bounds__(512) k_mfma_tile(const DPass* __restrict__ pas
   }
   __syncthreads();
   blocks();
-  unrolled<PER2>([&](auto it) { *glb4(s, it) = get4(it); });
+  unrolled<PER2>([&](auto it) { out4(s, it) = get4(it); });
 }
 
 // Blocks of `kern` (512 threads, `lds` bytes of LDS) resident on the whole
@@ -833,25 +835,25 @@ static void ensure_lds_attr(K kern, size_t bytes);
 
 template <int K>
 static void launch_mfma_tile_k(const DPass& P, const DPass* passes_dev, int pi, const DOp* dop_dev,
-                               const int32_t* ukbits_dev, const uint32_t* runoff_dev, const void* ctab, void* state,
-                               int n, int64_t batch, hipStream_t st) {
+                               const int32_t* ukbits_dev, const uint32_t* runoff_dev, const void* ctab, const void* src,
+                               void* state, int n, int64_t batch, hipStream_t st) {
   const size_t lds = ((size_t)8 << K) + (size_t)P.nmop * (8192 + 32 + (4 << (K - 5)));
   ensure_lds_attr(k_mfma_tile<K>, lds);
   const int64_t ntiles = batch << P.nblk_log;
   const int64_t grid = std::min<int64_t>(ntiles, resident_grid(k_mfma_tile<K>, lds));
   hipLaunchKernelGGL(k_mfma_tile<K>, dim3((unsigned)grid), dim3(512), lds, st, passes_dev, pi, dop_dev, ukbits_dev,
-                     runoff_dev, (const float*)ctab, (float2*)state, (int64_t)1 << n, ntiles);
+                     runoff_dev, (const float*)ctab, (const float2*)src, (float2*)state, (int64_t)1 << n, ntiles);
 }
 
 bool launch_mfma_tile(const DPass& P, const DPass* passes_dev, int pi, const DOp* dop_dev, const int32_t* ukbits_dev,
-                      const uint32_t* runoff_dev, const void* ctab, void* state, int n, int64_t batch,
+                      const uint32_t* runoff_dev, const void* ctab, const void* src, void* state, int n, int64_t batch,
                       hipStream_t st) {
   if (P.nmop < 1 || P.nmop > kMfmaTileMaxOps || P.nblk_log != n - P.k) return false;
   switch (P.k) {
-    case 10: launch_mfma_tile_k<10>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, state, n, batch, st); return true;
-    case 11: launch_mfma_tile_k<11>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, state, n, batch, st); return true;
-    case 12: launch_mfma_tile_k<12>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, state, n, batch, st); return true;
-    case 13: launch_mfma_tile_k<13>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, state, n, batch, st); return true;
+    case 10: launch_mfma_tile_k<10>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, src, state, n, batch, st); return true;
+    case 11: launch_mfma_tile_k<11>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, src, state, n, batch, st); return true;
+    case 12: launch_mfma_tile_k<12>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, src, state, n, batch, st); return true;
+    case 13: launch_mfma_tile_k<13>(P, passes_dev, pi, dop_dev, ukbits_dev, runoff_dev, ctab, src, state, n, batch, st); return true;
     default: return false;
   }
 }

@@ -813,7 +813,10 @@ std::string pass_body(const Program& P, const Sched& S, int pi, bool adj, int dt
   }
   // forward pass: one tile
   if (!multi) G.line(fmt("__shared__ cT tile[%d];", 1 << k));
-  G.line("cT* __restrict__ s = st + b * sstride + base;");
+  // si: the states read, st itself or others; a block reads all of its tile
+  // before it writes any
+  G.line(multi ? "cT* __restrict__ s = st + b * sstride + base;" : "cT* s = st + b * sstride + base;");
+  if (!multi) G.line("const cT* s0 = si + b * sstride + base;");
   if (multi) {
     for (int it = 0; it < nit; ++it) G.line(fmt("const cT r%d = s[dlo + %lluull];", it, hi(it)));
   } else {
@@ -824,7 +827,7 @@ std::string pass_body(const Program& P, const Sched& S, int pi, bool adj, int dt
     G.line("  r0 = cT{(base | (unsigned long long)dlo) == 0ull ? (T)1 : (T)0, (T)0};");
     for (int it = 1; it < nit; ++it) G.line(fmt("  r%d = cT{(T)0, (T)0};", it));
     G.line("} else {");
-    for (int it = 0; it < nit; ++it) G.line(fmt("  r%d = s[dlo + %lluull];", it, hi(it)));
+    for (int it = 0; it < nit; ++it) G.line(fmt("  r%d = s0[dlo + %lluull];", it, hi(it)));
     G.line("}");
   }
   for (int it = 0; it < nit; ++it) G.line(fmt("LDSB(tile, slo ^ %uu) = r%d;", swz_h((uint32_t)it << tl) * cb, it));
@@ -892,7 +895,7 @@ std::string gen_pass_source(const Program& P, const Sched& S, int dt, int mode, 
       // parameter lists: jit_launch_fwd / jit_launch_adj pass exactly these
       if (mode == 0)
         k = fmt("extern \"C\" __global__ void __launch_bounds__(%d) __attribute__((amdgpu_waves_per_eu(%d))) "
-                "tcm_fwd_k%d(cT* __restrict__ st, long long sstride, "
+                "tcm_fwd_k%d(const cT* si, cT* st, long long sstride, "
                 "const T* __restrict__ mtab, long long mstride, long long mbase, long long dbase, "
                 "const T* __restrict__ ct, cT* __restrict__ ck, long long total, int zinit) {\n",
                 NT, waves, id);

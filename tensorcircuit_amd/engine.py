@@ -155,11 +155,12 @@ class Program:
         dev = device()
         N = 1 << self.n
         code = _CODE[dtype]
+        src = None
         if out is None:
             if inputs is not None:
-                state = inputs.to(device=dev, dtype=_CDT[dtype]).reshape(batch, N).clone()
-            else:
-                state = torch.empty(batch, N, dtype=_CDT[dtype], device=dev)
+                src = inputs.to(device=dev, dtype=_CDT[dtype]).reshape(batch, N)
+                src = src.resolve_conj().resolve_neg().contiguous()
+            state = torch.empty(batch, N, dtype=_CDT[dtype], device=dev)
         else:
             state = out
             if inputs is not None:
@@ -172,9 +173,14 @@ class Program:
         nb = _i64()
         check(lib.tcm_forward_workspace_bytes(self.handle, code, batch, C.byref(nb)), "workspace")
         ws = _workspace(nb.value, dev)
-        check(lib.tcm_forward(self.handle, code, _ptr(p), pstride, state.data_ptr(), batch,
-                              1 if inputs is None else 0, _ptr(ck) if want_ckpts and self.nckpt else None,
-                              ws.data_ptr(), ws.numel(), _stream()), "tcm_forward")
+        ckp = _ptr(ck) if want_ckpts and self.nckpt else None
+        if src is not None:
+            check(lib.tcm_forward_from(self.handle, code, _ptr(p), pstride, src.data_ptr(), state.data_ptr(), batch,
+                                       ckp, ws.data_ptr(), ws.numel(), _stream()), "tcm_forward_from")
+        else:
+            check(lib.tcm_forward(self.handle, code, _ptr(p), pstride, state.data_ptr(), batch,
+                                  1 if inputs is None else 0, ckp, ws.data_ptr(), ws.numel(), _stream()),
+                  "tcm_forward")
         return state, ck
 
     # --- vector-Jacobian product ---------------------------------------------

@@ -434,3 +434,36 @@ def test_mixed_angles(gpu):
     h = torch.autograd.grad(layers(blocks.example_block, q.reshape(-1)), q)[0]
     assert h.shape == q.shape and torch.isfinite(h).all()
     assert g[:4, :4].abs().sum() > 0 and g[4:].abs().sum() == 0 and g[:, 4].abs().sum() == 0
+
+
+# the first pass reads given inputs itself: table-driven, compiled and
+# matrix-core passes, and the copy before per-gate kernels, circuits without
+# gates and inputs off a 16-byte boundary; against the same passes in place
+@pytest.mark.parametrize("n,opts", [(3, {}), (6, {}), (13, {}), (13, {"jit": 1}), (14, {"jit": 1, "ckpt_every": 1}),
+                                    (5, {"fuse": 0}), (12, {"mfma": 2}), (15, {"mfma": 2}), (4, {"empty": 1})])
+def test_forward_inputs(gpu, n, opts):
+    from tensorcircuit_amd import _lib, engine, fusion, workloads
+
+    rng = np.random.default_rng(n)
+    opts = {"fuse": 1, **opts}
+    if opts.get("mfma"):
+        prog, p = engine.Program(n, fusion.fuse(workloads.brickwork(n, 4, seed=2), n), 0, **opts), 0
+    else:
+        specs, p = [], 0
+        for i in range(0 if opts.pop("empty", 0) else 4 * n):
+            specs.append(engine.GateSpec((_lib.G_RX, _lib.G_RY, _lib.G_RZ)[i % 3], (i % n,), p, 0.0, 1.0, None))
+            p += 1
+            if i % n == n - 1:
+                specs.append(engine.barrier())
+        prog = engine.Program(n, specs, p, **opts)
+    for dt in DTYPES[:1] if opts.get("mfma") else DTYPES:
+        name = {torch.complex64: "complex64", torch.complex128: "complex128"}[dt]
+        th = torch.as_tensor(rng.normal(size=(3, p))).cuda() if p else None
+        flat = torch.as_tensor(rng.standard_normal(3 * 2**n + 1) + 1j * rng.standard_normal(3 * 2**n + 1)).to(dt).cuda()
+        for x in (flat[:-1], flat[1:], torch.conj(flat[:-1])):
+            x = x.reshape(3, 2**n)
+            before = x.clone()
+            want, wck = prog.forward(th, 3, name, inputs=x, want_ckpts=True, out=torch.empty_like(before))
+            got, ck = prog.forward(th, 3, name, inputs=x, want_ckpts=True)
+            assert torch.equal(got, want) and torch.equal(ck, wck) and torch.equal(x, before)
+            assert got.data_ptr() != x.data_ptr()
