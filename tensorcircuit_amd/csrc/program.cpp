@@ -1482,8 +1482,15 @@ int build_program(const tcm_gate* gates, int32_t ngates, int32_t n, int32_t npar
     // fewer passes at about the same per-pass bandwidth (24-qubit HEA: 44 +
     // 44 passes instead of 56 + 68)
     const int kd = (dt == 0 ? 12 : 11) + (o.jit ? 1 : 0);
+    // Table-driven complex128 adjoint passes take 64 KiB too from 18 qubits,
+    // where a state has tiles enough (18 qubits x 3, 6 layers: 771 -> 705 us
+    // qaoa, 502 -> 434 hea); below, a single state leaves more CUs idle than
+    // the passes save (17 qubits, hea: 341 -> 359).  Not the forward passes:
+    // programs run together share launches, whose LDS is the largest tile's
+    // (13 to 18 qubits x 21: 852 -> 1045 us).
+    const int kda = kd + (dt == 1 && !o.jit && n >= 18 ? 1 : 0);
     int kf = o.tile_bits > 0 ? o.tile_bits : kd;
-    int ka = o.adj_tile_bits > 0 ? o.adj_tile_bits : kd;
+    int ka = o.adj_tile_bits > 0 ? o.adj_tile_bits : kda;
     // a tile must fit one CU's 160 KiB of LDS with room for the adjoint's
     // partial sums: 2^14 complex64 or 2^13 complex128 amplitudes (128 KiB)
     const int kmax = dt == 0 ? 14 : 13;

@@ -74,7 +74,7 @@ def _long_runs(n):
 # states smaller than a wave of threads, one tile, a tile and more; few gates
 # and enough to fill several chunks of staged tables
 @pytest.mark.parametrize("n,gates", [(4, 12), (4, 0), (5, 30), (7, 60), (9, 25), (10, 0), (11, 90), (12, 400), (13, 0),
-                                     (14, 120)])
+                                     (14, 120), (18, 26)])
 def test_tile_pass(gpu, n, gates):
     import tensorcircuit_amd as tc
     from tensorcircuit_amd import engine
