@@ -66,6 +66,7 @@ struct PauliTileSched {
   std::vector<int> legacy;         // flip groups wider than a tile
   std::vector<int> legacy_slot0;
   int nslots = 0;                  // energy-partial slots of this dtype
+  int limit_slots = 0;  // what the batch limit of a fixed scratch counts per state
 };
 
 struct tcm_pauli {
@@ -564,9 +565,28 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
   int k = std::min(n, dt == 0 ? 12 : 11);
   const int Lw = std::min(dt == 0 ? 4 : 3, k);
   const uint64_t lmask = (1ull << Lw) - 1;
-  if (dt == 0 && n > k && (n <= 14 || n >= 20)) {
+  int64_t wide_slots = INT64_MAX;  // partial sums a state would have with 14-bit tiles
+  if (dt == 0 && n > k) {
     const int k14 = std::min(n, 14);
-    if (npasses(k14, lmask) < npasses(k, lmask)) k = k14;
+    int legacy12 = 0, legacy14 = 0;
+    int64_t slots14 = 0;  // of groups wider than a tile
+    for (const DPGroup& G : H->groups) {
+      const int w = __builtin_popcountll(G.flip | lmask);
+      legacy12 += w > k;
+      if (w > k14) {
+        ++legacy14;
+        slots14 += G.nblk;
+      }
+    }
+    const int np12 = npasses(k, lmask), np14 = npasses(k14, lmask);
+    // also where a 12-bit tile would leave a group to a launch of its own, or
+    // the passes are so many that their partial sums are
+    const bool narrow = n >= 15 && n <= 19 && legacy12 == legacy14 &&
+                        slots14 + ((int64_t)(np12 - legacy12) << (n - k)) <= 1 << 18;
+    if (np14 < np12) {
+      if (narrow) wide_slots = slots14 + ((int64_t)(np14 - legacy14) << (n - k14));
+      else k = k14;
+    }
   }
   std::vector<int> rem;
   for (int g = 0; g < (int)H->groups.size(); ++g) {
@@ -638,6 +658,7 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
     slot += H->groups[g].nblk;
   }
   S.nslots = slot;
+  S.limit_slots = (int)std::min<int64_t>(slot, wide_slots);
 }
 
 // ---- adjoint ---------------------------------------------------------------
@@ -997,7 +1018,11 @@ int pauli_expect_check(const tcm_pauli* ham, int32_t dtype, const void* state, i
                        int64_t scratch_bytes) {
   if (!ham || !valid_dtype(dtype) || batch < 0 || (batch > 0 && (!state || !out)))
     return set_error(TCM_E_ARG, "bad arguments to tcm_expect_pauli_sum_noalloc");
-  const int64_t need = pauli_ws(ham, dtype, batch);
+  // by the fewest partial sums of a state over the tilings that the schedule
+  // chooses from: where it takes another, the batch runs in parts
+  const PauliTileSched& S = ham->ts[dtype];
+  const int64_t slots = S.ok ? S.limit_slots : ham->nslots;
+  const int64_t need = align_up(batch * slots * 2 * (int64_t)sizeof(double)) + align_up(batch * 2 * (int64_t)sizeof(double));
   if (need > scratch_bytes)
     return set_error(TCM_E_WORKSPACE,
                      "tcm_expect_pauli_sum_noalloc: %lld states need %lld bytes of partial sums, the static scratch "
@@ -1032,11 +1057,17 @@ int pauli_expect_prepared(const tcm_pauli* ham, int32_t dtype, const void* state
   hipStream_t st = (hipStream_t)stream;
   // a single partial per state is the energy itself
   const int ns = pauli_slots(H, dtype);
-  double* epart = ns > 1 ? (double*)scratch : out;
-  int rc = dtype == TCM_C64 ? pauli_energy_apply<float>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st, pd)
-                            : pauli_energy_apply<double>(H, dtype, state, nullptr, nullptr, batch, epart, true, false, st, pd);
-  if (rc) return rc;
-  if (ns > 1) launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, out, batch, st);
+  const int64_t part = ns > 1 ? std::max<int64_t>(1, scratch_bytes / (ns * 2 * (int64_t)sizeof(double))) : batch;
+  for (int64_t b0 = 0; b0 < batch; b0 += part) {
+    const int64_t nb = std::min(part, batch - b0);
+    double* o = out + 2 * b0;
+    double* epart = ns > 1 ? (double*)scratch : o;
+    const void* s = (const char*)state + (b0 << H->n) * 2 * (int64_t)tsize(dtype);
+    const int rc = dtype == TCM_C64 ? pauli_energy_apply<float>(H, dtype, s, nullptr, nullptr, nb, epart, true, false, st, pd)
+                                    : pauli_energy_apply<double>(H, dtype, s, nullptr, nullptr, nb, epart, true, false, st, pd);
+    if (rc) return rc;
+    if (ns > 1) launch_sum_slots(epart, (int64_t)ns * 2, ns, 2, o, nb, st);
+  }
   HIP_TRY(hipGetLastError(), "expect launch");
   return 0;
 }

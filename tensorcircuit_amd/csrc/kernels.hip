@@ -81,13 +81,6 @@ __device__ __forceinline__ void block_sum2(double& a, double& b) {
   __syncthreads();
 }
 
-// the part of (re, im) that the working type cuts off
-template <typename T>
-__device__ __forceinline__ void put_low(T* o, double re, double im) {
-  o[0] = (T)(re - (double)(T)re);
-  o[1] = (T)(im - (double)(T)im);
-}
-
 // A diagonal entry in the working type.  For a phase in float, of the 9 pairs
 // around it the one with the least 16 (|z| - 1)^2 + (angle error)^2: an angle
 // error is a small unitary, which hardly moves the energy of a scrambled
@@ -116,6 +109,16 @@ __device__ __forceinline__ void store_diagonal(float* o, double re, double im) {
         o[1] = s;
       }
     }
+}
+
+// a phase rounded to u, or (sg = -1) its conjugate, and at o + low the part of
+// (re, sg im) that this cuts off
+template <typename T>
+__device__ __forceinline__ void put_phase(T* o, int low, const T* u, double re, double im, double sg) {
+  o[0] = u[0];
+  o[1] = (T)sg * u[1];
+  o[low] = (T)(re - (double)u[0]);
+  o[low + 1] = (T)(sg * (im - (double)u[1]));
 }
 
 // t = tan(ph / 2) and s = sin(ph) of the three shears.  In float, of the 9
@@ -195,44 +198,38 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
       case TCM_G_RX: {
         double c, s;
         sincos(0.5 * a, &s, &c);
-        o[0] = (T)c; o[1] = 0; o[2] = 0; o[3] = (T)-s; o[4] = 0; o[5] = (T)-s; o[6] = (T)c; o[7] = 0;
+        T u[2];
+        store_diagonal(u, c, s);
+        o[0] = u[0]; o[1] = 0; o[2] = 0; o[3] = -u[1]; o[4] = 0; o[5] = -u[1]; o[6] = u[0]; o[7] = 0;
         if (r.extra) put_rotation(o, 0.5 * a);
       } break;
       case TCM_G_RY: {
         double c, s;
         sincos(0.5 * a, &s, &c);
-        o[0] = (T)c; o[1] = (T)-s; o[2] = (T)s; o[3] = (T)c;
+        T u[2];
+        store_diagonal(u, c, s);
+        o[0] = u[0]; o[1] = -u[1]; o[2] = u[1]; o[3] = u[0];
         if (r.extra) put_rotation(o, 0.5 * a);
       } break;
-      case TCM_G_RZ: {
-        double c, s;
-        sincos(0.5 * a, &s, &c);
-        o[0] = (T)c; o[1] = (T)-s; o[2] = (T)c; o[3] = (T)s;
-        if (r.extra) {  // over the first entry: 1, e^{ia}
-          put_low(o + kRzFirst, c, -s);
-          sincos(a, &s, &c);
-          T* u = o + kRzOne;
-          u[0] = 1; u[1] = 0; u[2] = (T)c; u[3] = (T)s;
-          u = o + kRzLow;
-          u[0] = 0; u[1] = 0;
-          put_low(u + 2, c, s);
-        }
-      } break;
+      case TCM_G_RZ:
       case TCM_G_RZZ: {
+        // rz: entries by the bit; rzz: by the parity of the two bits
+        const bool rz = r.kind == TCM_G_RZ;
+        const int ne = rz ? 2 : 4, low = 2 * ne;
         double c, s;
+        T u[2];
         sincos(0.5 * a, &s, &c);
-        o[0] = (T)c; o[1] = (T)-s; o[2] = (T)c; o[3] = (T)s;
-        o[4] = (T)c; o[5] = (T)s; o[6] = (T)c; o[7] = (T)-s;
+        store_diagonal(u, c, s);
+        for (int e = 0; e < ne; ++e) put_phase(o + 2 * e, low, u, c, s, ((e >> 1) ^ e) & 1 ? 1.0 : -1.0);
         if (r.extra) {
-          put_low(o + kRzzFirst, c, -s);
+          const T one[2] = {1, 0};
           sincos(a, &s, &c);
-          T* u = o + kRzzOne;
-          u[0] = 1; u[1] = 0; u[2] = (T)c; u[3] = (T)s;
-          u[4] = (T)c; u[5] = (T)s; u[6] = 1; u[7] = 0;
-          u = o + kRzzLow;
-          u[0] = 0; u[1] = 0; u[6] = 0; u[7] = 0;
-          put_low(u + 2, c, s);
-          put_low(u + 4, c, s);
+          store_diagonal(u, c, s);
+          T* q = o + 2 * low;
+          for (int e = 0; e < ne; ++e) {
+            if (((e >> 1) ^ e) & 1) put_phase(q + 2 * e, low, u, c, s, 1.0);
+            else put_phase(q + 2 * e, low, one, 1.0, 0.0, 1.0);
+          }
         }
       } break;
       case TCM_G_RXX:

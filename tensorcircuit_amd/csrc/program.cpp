@@ -492,8 +492,8 @@ bool diag_kind(const LGate& g) {
 // table entries of a gate's recipe
 int recipe_slot(const Program& P, const LGate& g) {
   if (P.opts.jit && (g.src == TCM_G_RX || g.src == TCM_G_RY)) return kRotSlot;
-  if (P.opts.jit && g.src == TCM_G_RZ) return kRzSlot;
-  if (P.opts.jit && g.src == TCM_G_RZZ) return kRzzSlot;
+  if (g.src == TCM_G_RZ) return P.opts.jit ? kRzSlot : kRzOne;
+  if (g.src == TCM_G_RZZ) return P.opts.jit ? kRzzSlot : kRzzOne;
   return layout_size(g.okind);
 }
 
@@ -810,11 +810,14 @@ static void build_group_ops(const Program& P, Sched& S, const HGroup& hg,
         f.s0 = slot_of(g.bits[0]);
         f.s1 = g.nq > 1 ? slot_of(g.bits[1]) : -1;
         f.cls = factor_classes(P, g);
-        if (P.opts.jit && g.mslot >= 0 && (g.src == TCM_G_RZ || g.src == TCM_G_RZZ)) {
+        if (g.mslot >= 0 && (g.src == TCM_G_RZ || g.src == TCM_G_RZZ)) {
           const bool rz = g.src == TCM_G_RZ;
-          scalars.push_back(DFactor{f.src, DF_SCALAR, -1, -1, rz ? kRzFirst : kRzzFirst, 0});
-          f.src += rz ? kRzOne : kRzzOne;
-          f.low = rz ? kRzLow - kRzOne : kRzzLow - kRzzOne;
+          f.low = rz ? kRzLow : kRzzLow;
+          if (P.opts.jit) {
+            scalars.push_back(DFactor{f.src, DF_SCALAR, -1, -1, f.low, 0});
+            f.src += rz ? kRzOne : kRzzOne;
+            f.low = rz ? kRzOneLow - kRzOne : kRzzOneLow - kRzzOne;
+          }
         }
         S.factors.push_back(f);
         if (g.gop >= 0) {

@@ -169,12 +169,12 @@ struct DGopSum {
 // with R(phi) = sigma R(phi')
 constexpr int kRotShear = 8, kRotSigma = 10, kRotSlot = 12;
 
-// Table entries of rz and rzz recipes of compiled programs: the exact
-// diagonal, then (from kRzOne, or kRzzOne) the diagonal over its first entry,
-// whose entries are 1 or e^{i angle}, the part of these that the working type
-// cuts off, and that of the first entry
-constexpr int kRzOne = 4, kRzLow = 8, kRzFirst = 12, kRzSlot = 16;
-constexpr int kRzzOne = 8, kRzzLow = 16, kRzzFirst = 24, kRzzSlot = 32;
+// Table entries of rz and rzz recipes: the diagonal, then the part of it that
+// the working type cuts off (kRzLow, kRzzLow); of compiled programs also the
+// diagonal over its first entry (kRzOne, kRzzOne), whose entries are 1 or
+// e^{i angle}, and the part cut off of that
+constexpr int kRzLow = 4, kRzOne = 8, kRzOneLow = 12, kRzSlot = 16;
+constexpr int kRzzLow = 8, kRzzOne = 16, kRzzOneLow = 24, kRzzSlot = 32;
 
 // Factor of a DG recipe: a diagonal (D1 or D2 layout, per-batch or constant)
 // evaluated on slots s0 (, s1) of the group index.

@@ -467,3 +467,46 @@ def test_forward_inputs(gpu, n, opts):
             got, ck = prog.forward(th, 3, name, inputs=x, want_ckpts=True)
             assert torch.equal(got, want) and torch.equal(ck, wck) and torch.equal(x, before)
             assert got.data_ptr() != x.data_ptr()
+
+
+# Pauli sums whose 14-bit tiles would take fewer passes (XX on every pair of
+# qubits), at the qubit counts that keep 12-bit tiles, and with a string that
+# only a 14-bit tile holds; the entry point with a fixed scratch accepts the
+# batches that 14-bit tiles allow, in parts
+@pytest.mark.parametrize("n,wide", [(14, False), (15, False), (17, True), (15, True)])
+def test_pauli_tile_widths(gpu, n, wide):
+    import ctypes
+
+    from tensorcircuit_amd import _lib, engine
+
+    rng = np.random.default_rng(n + wide)
+    pairs = [(i, j) for i in range(n) for j in range(i)]
+    T = len(pairs) + 2
+    codes = np.zeros((T, n), dtype=np.int8)
+    for t, (i, j) in enumerate(pairs):
+        codes[t, i] = codes[t, j] = 1 + t % 2
+    codes[T - 2, 1:3] = 3
+    codes[T - 1, : 9 if wide else 1] = 1  # 9 flips above the 4 low bits, or 1
+    w = rng.standard_normal(T)
+    terms = [(float(w[t]), list(codes[t])) for t in range(T)]
+    ham = engine.PauliSum(n, codes, w, jit=0)
+    s = random_states(rng, 2, n)
+    for dt in DTYPES:
+        st = torch.as_tensor(s).to(dt).cuda()
+        sd = np_of(st).astype(np.complex128)
+        # T weights summed, then one product and sum per flip group (<= T)
+        tol = (2 * T + 8) * UNIT[dt] * np.abs(w).sum()
+        e, h = np_of(ham.expect(st)), np_of(ham.apply(st))
+        for b in range(2):
+            assert abs(e[b] - sv.pauli_sum_expectation(sd[b], n, terms)) <= tol
+            assert np.abs(h[b] - sv.pauli_sum_apply(sd[b], n, terms)).max() <= 2 * tol
+    if n == 15 and not wide:
+        nb = ctypes.c_int64()
+        _lib.lib.tcm_pauli_workspace_bytes(ham.handle, _lib.TCM_C64, 1000, ctypes.byref(nb))
+        batch = 3 * (8 << 20) // (2 * (nb.value // 1000))  # half as much again as the scratch holds
+        st = torch.as_tensor(s[:1]).to(torch.complex64).cuda().expand(batch, -1).contiguous()
+        out = torch.empty(batch, 2, dtype=torch.float64, device="cuda")
+        want = np_of(ham.expect(st[:1]))[0]
+        _lib.check(_lib.lib.tcm_expect_pauli_sum_noalloc(ham.handle, _lib.TCM_C64, st.data_ptr(), batch, out.data_ptr(),
+                                                         engine._stream()), "tcm_expect_pauli_sum_noalloc")
+        assert (np_of(out)[:, 0] == want.real).all()
