@@ -698,7 +698,7 @@ AdjWs carve_adj(const Program& P, const tcm_pauli* H, int dtype, int64_t batch, 
 
 template <typename T>
 int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, const void* lam_src, const void* ckpts,
-                  void* grad_input, int64_t batch, hipStream_t st) {
+                  void* grad_input, int64_t batch, hipStream_t st, int eslots = 0) {
   DeviceTables* D = nullptr;
   if (int rc = ensure_tables(P, dtype, 1, &D)) return rc;
   const Sched& A = P.sched[dtype][1];
@@ -760,7 +760,8 @@ int reverse_sweep(Program& P, int dtype, const AdjWs& w, const void* psi_src, co
                                     part_of(p), ps, st))
           return rc;
       } else if (A.R == kTileSlots) {
-        launch_tile_adj<T>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, part_of(p), ps, st);
+        launch_tile_adj<T>(A, *D, p, w.mtab_a, D->ctab, pin, pout, lin, lout, batch, n, part_of(p), ps, st,
+                           p == np - 1 && eslots > 0 ? w.epart : nullptr, eslots);
       } else {
         return set_error(TCM_E_UNSUPPORTED, "register slots R=%d not built", A.R);
       }
@@ -808,8 +809,12 @@ int energy_grad_impl(Program& P, int dtype, const void* params, int64_t pstride,
   // energy and lambda = H psi
   if (int rc = pauli_energy_apply<T>(H, dtype, w.psi, w.lam, nullptr, batch, w.epart, true, true, st)) return rc;
   // reverse sweep, then energies and gradients from the partial sums
-  if (int rc = reverse_sweep<T>(P, dtype, w, w.psi, w.lam, w.ckpt, nullptr, batch, st)) return rc;
-  finish_sweep(P, A, *DA, w, w.epart, pauli_slots(H, dtype), energy, 1.0, grad, batch, st);
+  // lambda less E psi, where the sum of a state's energy partials is cheap:
+  // only for states of norm one, whose E is no larger than H psi
+  const int ns = pauli_slots(H, dtype);
+  const int eslots = !inputs && P.unitary && ns <= kMaxShiftSlots ? ns : 0;
+  if (int rc = reverse_sweep<T>(P, dtype, w, w.psi, w.lam, w.ckpt, nullptr, batch, st, eslots)) return rc;
+  finish_sweep(P, A, *DA, w, w.epart, ns, energy, 1.0, grad, batch, st);
   HIP_TRY(hipGetLastError(), "adjoint launch");
   return 0;
 }
@@ -1094,6 +1099,7 @@ int tcm_program_build(const tcm_gate* gates, int32_t ngates, int32_t nqubits, in
   tp->p.gates = std::move(P->gates);
   tp->p.nlayers = P->nlayers;
   tp->p.ngop = P->ngop;
+  tp->p.unitary = P->unitary;
   tp->p.gop_gate = std::move(P->gop_gate);
   tp->p.p_ptr = std::move(P->p_ptr);
   tp->p.p_gops = std::move(P->p_gops);

@@ -189,10 +189,13 @@ TilePassArg tile_pass_arg(const DPass& P);
 template <typename T>
 void launch_tile_fwd(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
                      const void* in, void* out, int64_t batch, int n, void* ckout, bool zinit, hipStream_t st);
+// epart: energy partials [batch][eslots] (re, im), at most kMaxShiftSlots; the
+// pass then starts from lambda - E psi
+constexpr int kMaxShiftSlots = 1024;
 template <typename T>
 void launch_tile_adj(const Sched& S, const DeviceTables& D, int pi, const void* mtab, const void* ctab,
                      const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
-                     double* part, int64_t pstride, hipStream_t st);
+                     double* part, int64_t pstride, hipStream_t st, const double* epart, int eslots);
 // k: the largest tile of the jobs
 template <typename T>
 void launch_tile_fwd_multi(const MultiJobs& J, int64_t blocks, int threads, int k, hipStream_t st);

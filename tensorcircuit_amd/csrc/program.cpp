@@ -489,6 +489,20 @@ bool diag_kind(const LGate& g) {
          (g.gen == GN_NONE || g.gen == GN_Z || g.gen == GN_ZZ || g.gen == GN_P1);
 }
 
+bool is_unitary(const std::vector<double>& m, int d) {
+  for (int r = 0; r < d; ++r)
+    for (int c = 0; c <= r; ++c) {
+      double re = 0.0, im = 0.0;  // row r times row c conjugated
+      for (int k = 0; k < d; ++k) {
+        const double *a = &m[2 * (r * d + k)], *b = &m[2 * (c * d + k)];
+        re += a[0] * b[0] + a[1] * b[1];
+        im += a[1] * b[0] - a[0] * b[1];
+      }
+      if (std::fabs(re - (r == c)) > 1e-6 || std::fabs(im) > 1e-6) return false;
+    }
+  return true;
+}
+
 // table entries of a gate's recipe
 int recipe_slot(const Program& P, const LGate& g) {
   if (P.opts.jit && (g.src == TCM_G_RX || g.src == TCM_G_RY)) return kRotSlot;
@@ -549,6 +563,7 @@ static int lower(Program& P, const tcm_gate* gates, int32_t ngates) {
         if (!finite_all(g.mat, msz)) return set_error(TCM_E_NONFINITE, "gate %d: non-finite matrix", gi);
         L.mat.assign(g.mat, g.mat + msz);
         L.param = -1;
+        P.unitary = P.unitary && is_unitary(L.mat, 1 << g.nq);
         if (g.nq == 1) {
           if (equals(L.mat, kX, 8)) L.okind = OK_X1;
           else if (is_diag(L.mat, 2)) L.okind = OK_D1;
@@ -606,6 +621,7 @@ static int lower(Program& P, const tcm_gate* gates, int32_t ngates) {
         if (!g.mat) return set_error(TCM_E_ARG, "gate %d: EXP1 without generator", gi);
         if (!finite_all(g.mat, msz)) return set_error(TCM_E_NONFINITE, "gate %d: non-finite generator", gi);
         L.mat.assign(g.mat, g.mat + msz);
+        P.unitary = P.unitary && is_hermitian(L.mat, d);
         bool dg = is_diag(L.mat, d);
         L.okind = g.nq == 1 ? (dg ? OK_D1 : OK_U1) : (dg ? OK_D2 : OK_U2);
         if (g.nq == 1) {

@@ -281,6 +281,7 @@ struct Program {
   std::vector<LGate> gates;      // without barriers
   int32_t nlayers = 0;           // barriers seen
   int32_t ngop = 0;              // trainable gate count
+  bool unitary = true;           // every gate is, and every generator Hermitian
   std::vector<int32_t> gop_gate; // gop -> gate index
   // parameter -> gops (CSR) for the gradient reduction
   std::vector<int32_t> p_ptr, p_gops;

@@ -510,3 +510,51 @@ def test_pauli_tile_widths(gpu, n, wide):
         _lib.check(_lib.lib.tcm_expect_pauli_sum_noalloc(ham.handle, _lib.TCM_C64, st.data_ptr(), batch, out.data_ptr(),
                                                          engine._stream()), "tcm_expect_pauli_sum_noalloc")
         assert (np_of(out)[:, 0] == want.real).all()
+
+
+# lambda less E psi in the first reverse pass: one partial sum of the energy,
+# many, and more than the pass sums itself; gates that are not unitary and
+# given inputs keep lambda as it is.  A constant added to the Hamiltonian
+# (identity string) makes E large beside the gradients.
+@pytest.mark.parametrize("n,dtype,keep", [(6, "complex64", ""), (12, "complex64", ""), (15, "complex128", ""),
+                                          (18, "complex64", "inputs"), (8, "complex128", "gate"),
+                                          (19, "complex128", "")])
+def test_energy_shift(gpu, n, dtype, keep):
+    from tensorcircuit_amd import _lib, engine
+
+    rng = np.random.default_rng(n)
+    specs, p = [], 0
+    for i in range(2 * n):
+        specs.append(engine.GateSpec((_lib.G_RY, _lib.G_RZ, _lib.G_RX)[i % 3], (i % n,), p, 0.0, 1.0, None))
+        p += 1
+        if i % n == n - 1:
+            for q in range(n - 1):
+                specs.append(engine.GateSpec(_lib.G_MAT, (q, q + 1), -1, 0.0, 1.0,
+                                             np.eye(4)[[0, 1, 3, 2]].astype(np.complex128)))
+    if keep == "gate":
+        specs.insert(3, engine.GateSpec(_lib.G_MAT, (1,), -1, 0.0, 1.0, np.diag([1.0, 0.9]).astype(np.complex128)))
+    codes = np.zeros((n + 1, n), dtype=np.int8)
+    codes[np.arange(n), np.arange(n)] = 1 + np.arange(n) % 3
+    w = np.append(rng.standard_normal(n), 50.0)
+    th = torch.as_tensor(rng.normal(0, 0.3, (2, p))).cuda()
+    prog = engine.Program(n, specs, p, fuse=1, jit=0)
+    args = {}
+    if keep == "inputs":
+        args["inputs"] = torch.as_tensor(random_states(rng, 2, n)).cuda()
+    x = th if dtype == "complex128" else th.float()
+    with_one = engine.PauliSum(n, codes, w, jit=0)
+    without = engine.PauliSum(n, codes[:n], w[:n], jit=0)
+    kw = {k: v.to(torch.complex64 if dtype == "complex64" else torch.complex128) for k, v in args.items()}
+    e1, g1 = prog.energy_grad(x, with_one, 2, dtype, **kw)
+    # the gradient of the constant is zero: <psi|psi> does not depend on the
+    # angles of unitary gates; per-gate kernels in 64 bits as the reference
+    ref = engine.Program(n, specs, p, fuse=0)
+    h = without if keep != "gate" else with_one
+    e0, g0 = ref.energy_grad(x.double(), h, 2, "complex128",
+                             **{k: v.to(torch.complex128) for k, v in kw.items()})
+    u = 2.0**-24 if dtype == "complex64" else 2.0**-53
+    # roundings of each gate on psi and lambda (of norm <= sum |w|), there and back
+    tol = 4 * (len(specs) + 4) * u * np.abs(w).sum()
+    assert np.abs(np_of(g1) - np_of(g0)).max() <= tol
+    shift = 50.0 if keep != "gate" else 0.0
+    assert np.abs(np_of(e1) - np_of(e0) - shift).max() <= tol
