@@ -208,8 +208,9 @@ int tcm_expect_pauli_sum(const tcm_pauli* ham, int32_t dtype, const void* state,
  * cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  The partial sums live in a static
  * device array of 8 MiB per GPU (held until the process ends); a call whose
- * batch needs more (tcm_pauli_workspace_bytes > 8 MiB) returns
- * TCM_E_WORKSPACE.  `ham` must already be prepared on the current device
+ * batch needs more (tcm_pauli_workspace_bytes > 8 MiB; complex64 sums of 15
+ * to 19 qubits are counted with 14-bit tiles where those need less, and then
+ * run in parts) returns TCM_E_WORKSPACE.  `ham` must already be prepared on the current device
  * for `dtype` (one tcm_expect_pauli_sum call with it), else TCM_E_ARG.
  * Calls that overlap on one GPU share the array and race. */
 int tcm_expect_pauli_sum_noalloc(const tcm_pauli* ham, int32_t dtype,
