@@ -212,15 +212,14 @@ int jit_launch_fwd(const Sched& S, const DeviceTables& D, int pi, int dt, const 
   const JitPass& J = S.jit[pi];
   (void)dt;
   long long sstride = 1ll << n, mstride = S.mtab_size, mbase = J.mbase, dbase = J.dbase;
-  const void* a_si = src;
+  const void* a_si = zinit ? nullptr : src;
   void* a_st = state;
   const void* a_mt = mtab;
   const void* a_ct = ctab;
   void* a_ck = ckout;
   long long total = batch << P.nblk_log;
   // one entry per parameter of the generated signature, in its order
-  int a_z = zinit;
-  void* args[] = {&a_si, &a_st, &sstride, &a_mt, &mstride, &mbase, &dbase, &a_ct, &a_ck, &total, &a_z};
+  void* args[] = {&a_si, &a_st, &sstride, &a_mt, &mstride, &mbase, &dbase, &a_ct, &a_ck, &total};
   const unsigned blocks = (unsigned)total;
   const hipError_t e = hipModuleLaunchKernel((hipFunction_t)D.jit_fn[J.kernel], blocks, 1, 1,
                                              1u << P.tthreads_log, 1, 1, 0, st, args, nullptr);

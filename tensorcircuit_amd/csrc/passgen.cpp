@@ -813,20 +813,20 @@ std::string pass_body(const Program& P, const Sched& S, int pi, bool adj, int dt
   }
   // forward pass: one tile
   if (!multi) G.line(fmt("__shared__ cT tile[%d];", 1 << k));
-  // si: the states read, st itself or others; a block reads all of its tile
-  // before it writes any
+  // si: the states read, st itself, others or none; a block reads all of its
+  // tile before it writes any
   G.line(multi ? "cT* __restrict__ s = st + b * sstride + base;" : "cT* s = st + b * sstride + base;");
-  if (!multi) G.line("const cT* s0 = si + b * sstride + base;");
   if (multi) {
     for (int it = 0; it < nit; ++it) G.line(fmt("const cT r%d = s[dlo + %lluull];", it, hi(it)));
   } else {
-    // zinit: the pass starts from |0..0> instead of reading the state (the
+    // no si: the pass starts from |0..0> instead of reading states (the
     // element index base + dlo + hi(it) is 0 only for it = 0, hi(0) = 0)
     for (int it = 0; it < nit; ++it) G.line(fmt("cT r%d;", it));
-    G.line("if (zinit) {");
+    G.line("if (!si) {");
     G.line("  r0 = cT{(base | (unsigned long long)dlo) == 0ull ? (T)1 : (T)0, (T)0};");
     for (int it = 1; it < nit; ++it) G.line(fmt("  r%d = cT{(T)0, (T)0};", it));
     G.line("} else {");
+    G.line("  const cT* s0 = si + b * sstride + base;");
     for (int it = 0; it < nit; ++it) G.line(fmt("  r%d = s0[dlo + %lluull];", it, hi(it)));
     G.line("}");
   }
@@ -897,7 +897,7 @@ std::string gen_pass_source(const Program& P, const Sched& S, int dt, int mode, 
         k = fmt("extern \"C\" __global__ void __launch_bounds__(%d) __attribute__((amdgpu_waves_per_eu(%d))) "
                 "tcm_fwd_k%d(const cT* si, cT* st, long long sstride, "
                 "const T* __restrict__ mtab, long long mstride, long long mbase, long long dbase, "
-                "const T* __restrict__ ct, cT* __restrict__ ck, long long total, int zinit) {\n",
+                "const T* __restrict__ ct, cT* __restrict__ ck, long long total) {\n",
                 NT, waves, id);
       else
         k = fmt("extern \"C\" __global__ void __launch_bounds__(%d) __attribute__((amdgpu_waves_per_eu(%d))) "
