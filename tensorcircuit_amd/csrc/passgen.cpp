@@ -175,6 +175,9 @@ struct Gen {
   const DPass& dp;
   const HPass& hp;
   bool dag;       // adjoint: apply U^dagger, psi and lambda arrays
+  // rx and ry by shears: their tables hold the shears' entries (a plan of
+  // several programs may also hold some built without opts.jit)
+  bool shears;
   int R, nreg;
   int mbase, dbase;
   std::string out;
@@ -184,7 +187,8 @@ struct Gen {
   // multiplied by the product of their sigmas (frame_fix)
   std::vector<std::string> frame;
 
-  Gen(const Sched& s, const DPass& d, const HPass& h, bool adj) : S(s), dp(d), hp(h), dag(adj), R(s.R) {
+  Gen(const Program& P, const Sched& s, const DPass& d, const HPass& h, bool adj)
+      : S(s), dp(d), hp(h), dag(adj), shears(P.opts.jit != 0), R(s.R) {
     nreg = 1 << R;
     mbase = dbase = -1;
   }
@@ -371,7 +375,7 @@ struct Gen {
   // apply op to the arrays in `arrs` (one or two names)
   void apply(const DOp& op, const std::vector<const char*>& arrs, int id) {
     const std::string pre = fmt("c%d_", id);
-    if (op.flags & (OP_F_SHEAR | OP_F_RX)) {
+    if (shears && (op.flags & (OP_F_SHEAR | OP_F_RX))) {
       const char* P = pre.c_str();
       const std::string ax = op.flags & OP_F_RX ? "_x" : "_y", sg = dag ? "-" : "";
       line(fmt("const T %st = %s%s, %ss = %s%s;", P, sg.c_str(), mel(op.moff, kRotShear).c_str(), P, sg.c_str(),
@@ -557,7 +561,7 @@ std::string pass_body(const Program& P, const Sched& S, int pi, bool adj, int dt
                       bool multi = false) {
   const DPass& dp = S.dpass[pi];
   const HPass& hp = S.passes[pi];
-  Gen G(S, dp, hp, adj);
+  Gen G(P, S, dp, hp, adj);
   const int R = S.R, nreg = 1 << R;
   const int k = dp.k, tl = dp.tthreads_log, NT = 1 << tl, nbl = dp.nblk_log;
   const bool wide = P.n > 31;

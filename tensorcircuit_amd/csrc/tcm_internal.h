@@ -65,8 +65,8 @@ struct DOp {
 };
 
 // DOp flags
-// OP_F_SHEAR, OP_F_RX: ry, rx rotations (compiled passes: by three shears, the
-// entries kRotShear.. of the recipe)
+// OP_F_SHEAR, OP_F_RX: ry, rx rotations (compiled passes of opts.jit programs:
+// by three shears, the entries kRotShear.. of the recipe)
 // OP_F_ALL: a merged diagonal that takes the pass's scalars
 enum : int32_t { OP_F_MFMA = 1, OP_F_SHEAR = 2, OP_F_RX = 4, OP_F_ALL = 8 };
 

@@ -72,6 +72,58 @@ def test_multi_plan_matches_single_programs_and_oracle(gpu, dtype):
     np.testing.assert_allclose(np_of(st), np_of(s1), atol=tol)
 
 
+def _rotations(rng, n, depth):
+    """Every rotation kind on every qubit in turn, fixed angles among them:
+    (specs, oracle ops, number of parameters)."""
+    from tensorcircuit_amd import _lib, engine
+
+    kinds = [("ry", _lib.G_RY), ("rx", _lib.G_RX), ("rz", _lib.G_RZ), ("rzz", _lib.G_RZZ), ("rxx", _lib.G_RXX),
+             ("phase", _lib.G_PHASE)]
+    specs, ops, p = [], [], 0
+    for d in range(depth):
+        for q in range(n):
+            name, code = kinds[(q + d) % len(kinds)]
+            qs = (q, (q + 1) % n) if len(name) == 3 else (q,)
+            if q % 5 == 4:
+                th = float(rng.normal())
+                specs.append(engine.GateSpec(code, qs, -1, th, 1.0, None))
+                ops.append(sv.Op(name, qs, kw={"theta": th}))
+            else:
+                specs.append(engine.GateSpec(code, qs, p, 0.0, 1.0, None))
+                ops.append(sv.Op(name, qs, p))
+                p += 1
+    return specs, ops, p
+
+
+@pytest.mark.parametrize("jits", [(0, 0, 0), (0, 1, 0), (1, 0, 1)])
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+def test_multi_plan_of_programs_without_the_pass_compiler(gpu, dtype, jits):
+    """A plan compiles its programs' passes whether they were built with
+    jit = 0 (tables without the entries of the shear form) or jit = 1."""
+    from tensorcircuit_amd import engine, workloads
+
+    rng = np.random.default_rng(17)
+    rdt = torch.float32 if dtype == "complex64" else torch.float64
+    cdt = torch.complex64 if dtype == "complex64" else torch.complex128
+    items, refs = [], []
+    for n, jit in zip((10, 13, 15), jits):
+        specs, ops, p = _rotations(rng, n, 4)
+        prog = engine.Program(n, specs, p, fuse=1, jit=jit)
+        # angles beyond pi / 2 too, where the shear form changes its sign
+        pr = torch.as_tensor(2.0 * rng.normal(size=(3, p))).to(rdt).to(gpu)
+        items.append((prog, pr, torch.full((3, 1 << n), 7.0, dtype=cdt, device=gpu)))
+        refs.append(ops)
+    engine.MultiPlan([it[0] for it in items], dtype).forward(items)
+    torch.cuda.synchronize()
+    tol = 4e-6 if dtype == "complex64" else 1e-12
+    for (prog, pr, st), ops in zip(items, refs):
+        one, _ = prog.forward(pr, 3, dtype)
+        np.testing.assert_allclose(np_of(st), np_of(one), atol=tol, err_msg="n=%d" % prog.n)
+        for b in range(3):
+            ref = sv.run_ops(prog.n, ops, pr[b].double().cpu().numpy())
+            np.testing.assert_allclose(np_of(st)[b], ref, atol=tol, err_msg="n=%d b=%d" % (prog.n, b))
+
+
 def test_multi_plan_refuses_foreign_descriptors(gpu):
     from tensorcircuit_amd import engine
 

@@ -323,6 +323,27 @@ def test_compiled_pass_signatures(tmp_path, monkeypatch):
             assert len(s.split(",")) == nparams, (mode, s)
 
 
+@pytest.mark.parametrize("kind,entries", [("G_RX", 8), ("G_RY", 4), ("G_RZ", 8), ("G_RZZ", 16)])
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+def test_plan_source_reads_its_own_table(kind, entries, dtype, tmp_path, monkeypatch):
+    """The plan of a program without the pass compiler reads no matrix entry
+    behind those of its only rotation (rx: 8 numbers, ry: 4; rz and rzz become
+    a merged diagonal of 16 complex entries)."""
+    from tensorcircuit_amd import _lib, engine
+
+    monkeypatch.setenv("TCM_JIT_DUMP", str(tmp_path))
+    monkeypatch.setenv("TCM_CACHE_DIR", str(tmp_path / "cache"))
+    two = kind == "G_RZZ"
+    spec = engine.GateSpec(getattr(_lib, kind), (3, 5) if two else (3,), 0, 0.0, 1.0, None)
+    engine.MultiPlan([engine.Program(10, [spec], 1, fuse=1)], dtype)
+    (src,) = [p.read_text() for p in tmp_path.glob("tcm_passes_multi_*.hip")]
+    read = {int(i) for i in re.findall(r"\bmt\[(\d+)\]", src)}
+    merged = {int(i) for i in re.findall(r"\bmd\[(\d+)\]", src)}
+    assert read or merged
+    assert not read or max(read) < entries
+    assert not merged or max(merged) < 2 * 16
+
+
 def test_json_round_trip_and_qsim_parse(tmp_path):
     """to_json / from_json (abstractcircuit.py:932-1074, translation.py:587-702)
     and qsim text (abstractcircuit.py:953-1034) on the host: same gate
