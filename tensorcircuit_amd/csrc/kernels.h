@@ -157,8 +157,11 @@ int jit_launch_adj(const Sched& S, const DeviceTables& D, int pi, int dt, const 
                    const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
                    double* part, int64_t pstride, hipStream_t st);
 
-// matrix tables of up to kMaxPrepJobs schedules in one launch
+// matrix tables of up to kMaxPrepJobs schedules in one launch, and of at most
+// kMaxPrepBlocks batch items: a launch of 2^32 threads or more is cut short
+// without an error, and 2^23 blocks of 256 are half of that
 constexpr int kMaxPrepJobs = 16;
+constexpr int64_t kMaxPrepBlocks = 1 << 23;
 struct PrepJob {
   const void *rec, *fac, *params, *ctab;
   void* mtab;
@@ -170,7 +173,7 @@ struct PrepJobs {
   int64_t blocks = 0;
   PrepJob job[kMaxPrepJobs];
 };
-// adds a job; launches the jobs when they are kMaxPrepJobs
+// adds a job; launches the jobs at either limit
 template <typename T>
 void add_prep(PrepJobs& J, const Sched& S, const DeviceTables& D, const void* ctab, const void* params,
               int64_t pstride, void* mtab, int64_t batch, hipStream_t st);

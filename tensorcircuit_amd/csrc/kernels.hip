@@ -1082,11 +1082,16 @@ void add_prep(PrepJobs& J, const Sched& S, const DeviceTables& D, const void* ct
       if (first_dg == nrec) first_dg = i;
       dg_log = std::max(dg_log, (int)S.recipes[i].R);
     }
-  J.job[J.njobs++] = PrepJob{D.recipes, D.factors, params, ctab, mtab, pstride, (int64_t)S.mtab_size, J.blocks,
-                             nrec, first_dg, dg_log, 0};
-  J.blocks += batch;
-  J.widest = std::max({J.widest, first_dg, (nrec - first_dg) << dg_log});
-  if (J.njobs == kMaxPrepJobs) launch_prep<T>(J, st);
+  for (int64_t b0 = 0; b0 < batch;) {
+    const int64_t nb = std::min(batch - b0, kMaxPrepBlocks - J.blocks);
+    J.job[J.njobs++] = PrepJob{D.recipes, D.factors, params ? (const T*)params + b0 * pstride : nullptr, ctab,
+                               (T*)mtab + b0 * S.mtab_size, pstride, (int64_t)S.mtab_size, J.blocks,
+                               nrec, first_dg, dg_log, 0};
+    J.blocks += nb;
+    J.widest = std::max({J.widest, first_dg, (nrec - first_dg) << dg_log});
+    if (J.njobs == kMaxPrepJobs || J.blocks == kMaxPrepBlocks) launch_prep<T>(J, st);
+    b0 += nb;
+  }
 }
 
 template <typename T>
