@@ -894,22 +894,32 @@ int forward_multi_impl(const tcm_multi_desc* descs, int ndesc, int dtype, int in
       }
       if (S.dpass[r].mfma) return set_error(TCM_E_UNSUPPORTED, "matrix-core passes are not run in multi launches");
       const DPass& dp = S.dpass[r];
-      MultiJob& q = J.job[J.njobs++];
-      q.blob = D[i]->blob;
-      q.msrc = D[i]->msrc;
-      q.runoff = D[i]->runoff;
-      q.ctab = D[i]->ctab;
-      q.mtab = mtab[i];
-      q.state = descs[i].state;
-      q.mstride = S.mtab_size;
-      q.sstride = 1ll << P.n;
-      q.block0 = blocks;
-      q.pass = tile_pass_arg(dp);
-      q.zinit = r == 0 && init_zero;
-      blocks += descs[i].batch << dp.nblk_log;
-      threads = std::max(threads, 1 << dp.tthreads_log);
-      kmax = std::max(kmax, dp.k);
-      if (J.njobs == kMaxMultiJobs) flush();
+      for (int64_t b0 = 0; b0 < descs[i].batch;) {
+        // what fits the launch beside the jobs that it has (a single state does)
+        const int64_t room = kMaxLaunchThreads / std::max(threads, 1 << dp.tthreads_log) - blocks;
+        const int64_t nb = std::min(descs[i].batch - b0, room > 0 ? room >> dp.nblk_log : 0);
+        if (nb == 0) {
+          flush();
+          continue;
+        }
+        MultiJob& q = J.job[J.njobs++];
+        q.blob = D[i]->blob;
+        q.msrc = D[i]->msrc;
+        q.runoff = D[i]->runoff;
+        q.ctab = D[i]->ctab;
+        q.mtab = (T*)mtab[i] + b0 * S.mtab_size;
+        q.state = (V2<T>*)descs[i].state + (b0 << P.n);
+        q.mstride = S.mtab_size;
+        q.sstride = 1ll << P.n;
+        q.block0 = blocks;
+        q.pass = tile_pass_arg(dp);
+        q.zinit = r == 0 && init_zero;
+        blocks += nb << dp.nblk_log;
+        threads = std::max(threads, 1 << dp.tthreads_log);
+        kmax = std::max(kmax, dp.k);
+        b0 += nb;
+        if (J.njobs == kMaxMultiJobs) flush();
+      }
     }
     flush();
   }

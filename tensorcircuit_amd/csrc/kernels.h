@@ -157,11 +157,14 @@ int jit_launch_adj(const Sched& S, const DeviceTables& D, int pi, int dt, const 
                    const void* psi_in, void* psi_out, const void* lam_in, void* lam_out, int64_t batch, int n,
                    double* part, int64_t pstride, hipStream_t st);
 
+// most threads of a launch whose blocks are one per tile or parameter set: one
+// of 2^32 or more is cut short without an error
+constexpr int64_t kMaxLaunchThreads = 1ll << 31;
+
 // matrix tables of up to kMaxPrepJobs schedules in one launch, and of at most
-// kMaxPrepBlocks batch items: a launch of 2^32 threads or more is cut short
-// without an error, and 2^23 blocks of 256 are half of that
+// kMaxPrepBlocks batch items (blocks of 256 threads)
 constexpr int kMaxPrepJobs = 16;
-constexpr int64_t kMaxPrepBlocks = 1 << 23;
+constexpr int64_t kMaxPrepBlocks = kMaxLaunchThreads / 256;
 struct PrepJob {
   const void *rec, *fac, *params, *ctab;
   void* mtab;

@@ -227,15 +227,21 @@ static void allow_lds(const void* kern, size_t bytes) {
 
 template <typename T, int LE, bool ENERGY, bool APPLY>
 static void launch_le(const PauliTileArgs& A, int np, const PauliTileTables& D, const void* psi, const void* lam_in,
-                      void* lam_out, int n, const double* alpha, double* epart, int64_t estride, int64_t blocks,
+                      void* lam_out, int n, const double* alpha, double* epart, int64_t estride, int64_t batch,
                       hipStream_t st) {
   const size_t lds = (sizeof(V2<T>) << A.k) + kPauliChunk * (sizeof(Rec<T>) + sizeof(DPGroupS));
   allow_lds((const void*)k_pauli_tile<T, LE, ENERGY, APPLY>, lds);
   const unsigned threads = std::max(64u, 1u << (A.k - LE));
-  hipLaunchKernelGGL((k_pauli_tile<T, LE, ENERGY, APPLY>), dim3((unsigned)blocks, (unsigned)np), dim3(threads), lds,
-                     st, A, (const DPChunk*)D.chunks, (const DPGroupS*)D.groups, (const DPTermS*)D.terms,
-                     (const uint32_t*)D.runoff, (const V2<T>*)psi, (const V2<T>*)lam_in, (V2<T>*)lam_out,
-                     (int64_t)1 << n, alpha, epart, estride);
+  // all states at once unless they are too many threads
+  const int64_t part = std::max<int64_t>(1, (kMaxLaunchThreads / threads) >> A.nblk_log);
+  for (int64_t b0 = 0; b0 < batch; b0 += part) {
+    const int64_t nb = std::min(part, batch - b0), o = b0 << n;
+    hipLaunchKernelGGL((k_pauli_tile<T, LE, ENERGY, APPLY>), dim3((unsigned)(nb << A.nblk_log), (unsigned)np),
+                       dim3(threads), lds, st, A, (const DPChunk*)D.chunks, (const DPGroupS*)D.groups,
+                       (const DPTermS*)D.terms, (const uint32_t*)D.runoff, (const V2<T>*)psi + o,
+                       lam_in ? (const V2<T>*)lam_in + o : nullptr, lam_out ? (V2<T>*)lam_out + o : nullptr,
+                       (int64_t)1 << n, alpha ? alpha + b0 : nullptr, epart ? epart + b0 * estride : nullptr, estride);
+  }
 }
 
 template <typename T>
@@ -254,7 +260,6 @@ void launch_pauli_tile(const DPPass* P, int np, const PauliTileTables& D, const 
     a.nc = P[q].nc;
     for (int i = 0; i < P[q].nblk_log; ++i) a.bmask |= 1ull << P[q].blk_bits[i];
   }
-  const int64_t blocks = batch << A.nblk_log;
   // 8 amplitudes per thread; 4 where the tile would not fill a wave, 16 for
   // the complex64 tiles of 2^14.  4, 8 and 16 run alike in complex64 (1049,
   // 1032, 1036 us for a step over 10 to 18 qubits); in complex128 16 spill
@@ -263,11 +268,11 @@ void launch_pauli_tile(const DPPass* P, int np, const PauliTileTables& D, const 
 #define TCM_PT(LE)                                                                                                  \
   do {                                                                                                              \
     if (energy && apply)                                                                                            \
-      launch_le<T, LE, true, true>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, blocks, st);           \
+      launch_le<T, LE, true, true>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, batch, st);            \
     else if (energy)                                                                                                \
-      launch_le<T, LE, true, false>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, blocks, st);          \
+      launch_le<T, LE, true, false>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, batch, st);           \
     else                                                                                                            \
-      launch_le<T, LE, false, true>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, blocks, st);          \
+      launch_le<T, LE, false, true>(A, np, D, psi, lam_in, lam_out, n, alpha, epart, estride, batch, st);           \
   } while (0)
   if (le == 2) TCM_PT(2);
   else if (le == 3) TCM_PT(3);

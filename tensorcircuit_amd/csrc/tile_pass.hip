@@ -822,6 +822,14 @@ size_t lds_adj(int k, int nw) {
 
 unsigned threads_of(const DPass& P) { return std::max(64u, 1u << (P.k - kR)); }
 
+// launch(b0, nb) for batch items b0 .. b0 + nb - 1, all at once unless they
+// are too many threads
+template <typename F>
+void batch_parts(const DPass& P, int64_t batch, F launch) {
+  const int64_t part = std::max<int64_t>(1, (kMaxLaunchThreads / threads_of(P)) >> P.nblk_log);
+  for (int64_t b0 = 0; b0 < batch; b0 += part) launch(b0, std::min(part, batch - b0));
+}
+
 }  // namespace
 
 TilePassArg tile_pass_arg(const DPass& P) {
@@ -844,10 +852,14 @@ void launch_tile_fwd(const Sched& S, const DeviceTables& D, int pi, const void* 
   const size_t lds = lds_fwd<T>(P.k);
   auto go = [&](auto kern) {
     allow_lds((const void*)kern, lds);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(batch << P.nblk_log)), dim3(threads_of(P)), lds, st, tile_pass_arg(P),
-                       (const uint32_t*)D.blob, (const int32_t*)D.msrc, (const uint32_t*)D.runoff, (const T*)mtab,
-                       (int64_t)S.mtab_size, (const T*)ctab, (const A2<T>*)in, (A2<T>*)out, (int64_t)1 << n,
-                       (A2<T>*)ckout, zinit ? 1 : 0);
+    batch_parts(P, batch, [&](int64_t b0, int64_t nb) {
+      const int64_t o = b0 << n;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(nb << P.nblk_log)), dim3(threads_of(P)), lds, st, tile_pass_arg(P),
+                         (const uint32_t*)D.blob, (const int32_t*)D.msrc, (const uint32_t*)D.runoff,
+                         (const T*)mtab + b0 * S.mtab_size, (int64_t)S.mtab_size, (const T*)ctab,
+                         zinit ? nullptr : (const A2<T>*)in + o, (A2<T>*)out + o, (int64_t)1 << n,
+                         ckout ? (A2<T>*)ckout + o : nullptr, zinit ? 1 : 0);
+    });
   };
   if (P.full) go(k_tile_fwd<T, true>);
   else go(k_tile_fwd<T, false>);
@@ -869,10 +881,15 @@ void launch_tile_adj(const Sched& S, const DeviceTables& D, int pi, const void* 
   const size_t lds = lds_adj<T>(P.k, (int)(thr / 64));
   auto go = [&](auto kern) {
     allow_lds((const void*)kern, lds);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(batch << P.nblk_log)), dim3(thr), lds, st, tile_pass_arg(P),
-                       (const uint32_t*)D.blob, (const int32_t*)D.msrc, (const uint32_t*)D.runoff, (const T*)mtab,
-                       (int64_t)S.mtab_size, (const T*)ctab, (const A2<T>*)psi_in, (A2<T>*)psi_out,
-                       (const A2<T>*)lam_in, (A2<T>*)lam_out, (int64_t)1 << n, part, pstride, epart, eslots);
+    batch_parts(P, batch, [&](int64_t b0, int64_t nb) {
+      const int64_t o = b0 << n;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(nb << P.nblk_log)), dim3(thr), lds, st, tile_pass_arg(P),
+                         (const uint32_t*)D.blob, (const int32_t*)D.msrc, (const uint32_t*)D.runoff,
+                         (const T*)mtab + b0 * S.mtab_size, (int64_t)S.mtab_size, (const T*)ctab,
+                         (const A2<T>*)psi_in + o, psi_out ? (A2<T>*)psi_out + o : nullptr, (const A2<T>*)lam_in + o,
+                         lam_out ? (A2<T>*)lam_out + o : nullptr, (int64_t)1 << n, part + b0 * pstride, pstride,
+                         epart ? epart + 2 * b0 * eslots : nullptr, eslots);
+    });
   };
   if (P.full) go(k_tile_adj<T, true>);
   else go(k_tile_adj<T, false>);

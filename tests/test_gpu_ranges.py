@@ -27,3 +27,41 @@ def test_tables_of_many_parameter_sets(gpu):
     for (_, _, st), one in zip(items, (torch.complex(0 * s, -s), torch.complex(s, 0 * s))):
         ref = torch.cat([torch.complex(c, 0 * c), one], dim=1)
         assert float((st - ref).abs().max()) <= 4 * 2.0**-24
+
+
+def test_launches_of_many_small_states(gpu):
+    """2^26 states of four qubits: a wave each is 2^32 threads."""
+    from tensorcircuit_amd import _lib, engine
+
+    n, B = 4, (1 << 26) + 5
+    x = np.array([[0, 1], [1, 0]])
+    prog = engine.Program(n, [engine.GateSpec(_lib.G_MAT, (q,), -1, 0.0, 1.0, x) for q in (0, 3)], 0, fuse=1)
+    st = torch.zeros(B, 16, dtype=torch.complex64, device=gpu)
+    prog.forward(None, B, "complex64", out=st)
+    ref = torch.zeros(16, dtype=torch.complex64, device=gpu)
+    ref[0b1001] = 1.0
+    for part in st.split(1 << 22):
+        assert bool((part == ref).all())
+    codes = [[1, 0, 0, 0], [0, 0, 0, 3]]
+    hs = engine.PauliSum(n, codes, [2.0, 1.0], jit=0).apply(st)
+    ref = torch.zeros(16, dtype=torch.complex64, device=gpu)
+    ref[0b0001], ref[0b1001] = 2.0, -1.0
+    for part in hs.split(1 << 22):
+        assert bool((part == ref).all())
+
+
+def test_multi_program_launch_of_many_states(gpu):
+    """Programs whose tiles come to 2^32 threads when they share a launch."""
+    from tensorcircuit_amd import _lib, engine
+
+    x = np.array([[0, 1], [1, 0]])
+    items = []
+    for n, B in ((4, 9_000_000), (12, 3), (5, 9_000_000)):
+        prog = engine.Program(n, [engine.GateSpec(_lib.G_MAT, (0,), -1, 0.0, 1.0, x)], 0, fuse=1)
+        items.append((prog, None, torch.zeros(B, 1 << n, dtype=torch.complex64, device=gpu)))
+    engine.forward_multi(items, "complex64")
+    for prog, _, st in items:
+        ref = torch.zeros(st.shape[1], dtype=torch.complex64, device=gpu)
+        ref[st.shape[1] // 2] = 1.0
+        for part in st.split(1 << 22):
+            assert bool((part == ref).all())
