@@ -180,16 +180,17 @@ __global__ void __launch_bounds__(512) k_pauli_terms(const DPChunk* __restrict__
 }
 
 // out[b][t] = the sum of the nblk partials of (b, t) and a zero imaginary part
-// (NaN where the sum is not finite); one wave per (b, t)
-__global__ void __launch_bounds__(64) k_pauli_terms_sum(const double* __restrict__ part, int nblk,
+// (NaN where the sum is not finite); one wave per (b, t) in turn
+__global__ void __launch_bounds__(64) k_pauli_terms_sum(const double* __restrict__ part, int nblk, int64_t total,
                                                         double* __restrict__ out) {
-  const int64_t bt = blockIdx.x;
-  double a = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += 64) a += part[bt * nblk + i];
-  for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
-  if (threadIdx.x == 0) {
-    out[2 * bt] = a;
-    out[2 * bt + 1] = a - a;
+  for (int64_t bt = blockIdx.x; bt < total; bt += gridDim.x) {
+    double a = 0.0;
+    for (int i = threadIdx.x; i < nblk; i += 64) a += part[bt * nblk + i];
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+    if (threadIdx.x == 0) {
+      out[2 * bt] = a;
+      out[2 * bt + 1] = a - a;
+    }
   }
 }
 
@@ -323,8 +324,9 @@ void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n
   };
   if (k >= 9) go(k_pauli_terms<T, 3>, 3);
   else go(k_pauli_terms<T, 0>, 0);
-  hipLaunchKernelGGL(k_pauli_terms_sum, dim3((unsigned)(batch * nterms)), dim3(64), 0, st, (const double*)part, nblk,
-                     out);
+  const int64_t total = batch * nterms;
+  hipLaunchKernelGGL(k_pauli_terms_sum, dim3((unsigned)std::min(total, kMaxLaunchThreads / 64)), dim3(64), 0, st,
+                     (const double*)part, nblk, total, out);
 }
 
 template <typename T>

@@ -65,3 +65,15 @@ def test_multi_program_launch_of_many_states(gpu):
         ref[st.shape[1] // 2] = 1.0
         for part in st.split(1 << 22):
             assert bool((part == ref).all())
+
+
+def test_terms_of_many_states(gpu):
+    """65535 states x 1100 strings: 2^26 sums, a wave each."""
+    from tensorcircuit_amd import engine
+
+    T, B = 1100, 65535
+    ham = engine.PauliSum(1, [[3]] * T, np.ones(T))
+    st = torch.zeros(B, 2, dtype=torch.complex64, device=gpu)
+    st[:, 1] = 1.0
+    e = ham.expect_terms(st)
+    assert bool((e.real == -1.0).all()) and bool((e.imag == 0.0).all())
