@@ -131,7 +131,13 @@ __global__ void __launch_bounds__(1024) k_sample_scan(double* __restrict__ cum, 
 // weights of a stretch, 4 per lane -- about 4 + 1 + 1 dependent reads and 0.7
 // KiB a draw.  (A wave per draw, a binary search and a running scan of the
 // chunk: 14 + 16 dependent reads and up to 8 KiB; 187 us for 100000 draws
-// from 24 qubits, this 23 us.)  grid (ceil(shots / 16), batch)
+// from 24 qubits, this 23 us.)
+// Tree scans round in another order at every lane, so that a running sum can
+// grow by a unit over entries of zero weight, and r fall in between (the
+// total, for u = 0, did in one of five distributions that end in zeros).  An
+// index of probability zero is not drawn then: an empty chunk or stretch is
+// left for the last one of nonzero weight before it, and only indices of
+// nonzero weight are taken (r = 0 takes index 0).  grid (ceil(shots / 16), batch)
 template <typename T, bool PROB>
 __global__ void __launch_bounds__(256) k_sample_draw(const void* __restrict__ src, int64_t sstride, int cl, int sl,
                                                      int64_t nchunks, const double* __restrict__ cum,
@@ -153,41 +159,61 @@ __global__ void __launch_bounds__(256) k_sample_draw(const void* __restrict__ sr
     rem = step;
   }
   const int nsub = 1 << (cl - sl);
+  double sp = l < nsub ? sub[(b * nchunks + lo) * nsub + l] : 0.0;
+  if (r > 0.0 && !mask16(sp != 0.0)) {
+    // the last chunk of nonzero weight before
+    uint32_t some = 0;
+    for (int64_t e = lo; e > 0 && !some; e -= 16) {
+      some = mask16(e > l && sub[(b * nchunks + (e > l ? e - 1 - l : 0)) * nsub + nsub - 1] != 0.0);
+      if (some) lo = e - __ffs(some);
+    }
+    if (l < nsub) sp = sub[(b * nchunks + lo) * nsub + l];
+  }
   const double c0 = c[lo];
-  const double sp = l < nsub ? sub[(b * nchunks + lo) * nsub + l] : 0.0;
   const double before = __shfl_up(sp, 1, 16);
   uint32_t m = mask16(l < nsub && c0 + sp >= r);
   // rounding left r just above the chunk's last sum: its last stretch of
   // nonzero weight (and, below, the last index of it)
   const uint32_t grows = mask16(l < nsub && sp > (l ? before : 0.0));
-  const int k = m ? __ffs(m) - 1 : grows ? 31 - __clz(grows) : 0;
-  const double prefix = __shfl(sp, k > 0 ? k - 1 : 0, 16);
-  const double run = c0 + (k > 0 ? prefix : 0.0);
-  const int64_t first = (lo << cl) + ((int64_t)k << sl);
+  int k = m ? __ffs(m) - 1 : grows ? 31 - __clz(grows) : 0;
   // 2^sl weights, `per` consecutive ones per lane
   const int len = 1 << sl, per = len >= 16 ? len >> 4 : 1;
-  double p[4], acc = 0.0;
-  int lastnz = -1;
+  double p[4], acc;
+  uint32_t some, nz;  // which of a lane's, which lane's are not zero
+  auto sum_before = [&](int q) {
+    const double prefix = __shfl(sp, q > 0 ? q - 1 : 0, 16);
+    return c0 + (q > 0 ? prefix : 0.0);
+  };
+  double run = sum_before(k);
+  for (;;) {
+    const int64_t first = b * sstride + (lo << cl) + ((int64_t)k << sl);
+    acc = 0.0;
+    some = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int i = l * per + j;
-    const double x = j < per && i < len ? weight_at<T, PROB>(src, b * sstride + first + i) : 0.0;
-    acc += x;
-    p[j] = acc;
-    if (x > 0.0) lastnz = i;
+    for (int j = 0; j < 4; ++j) {
+      const int i = l * per + j;
+      const double x = j < per && i < len ? weight_at<T, PROB>(src, first + i) : 0.0;
+      acc += x;
+      p[j] = acc;
+      some |= x > 0.0 ? 1u << j : 0u;
+    }
+    nz = mask16(some != 0);
+    if (nz || k == 0 || !(r > 0.0)) break;
+    run = sum_before(--k);
   }
+  const uint32_t take = r > 0.0 ? some : 0xfu;
   const double excl = scan16(acc, l) - acc;
   int hit = -1;
 #pragma unroll
   for (int j = 3; j >= 0; --j) {
     const int i = l * per + j;
-    if (j < per && i < len && run + (excl + p[j]) >= r) hit = i;
+    if (j < per && i < len && run + (excl + p[j]) >= r && (take >> j & 1u)) hit = i;
   }
   m = mask16(hit >= 0);
-  const uint32_t nz = mask16(lastnz >= 0);
+  const int lastnz = l * per + 31 - __clz(some);
   const int from = m ? __ffs(m) - 1 : nz ? 31 - __clz(nz) : 0;
   const int found = __shfl(m ? hit : nz ? lastnz : 0, from, 16);
-  if (live && l == 0) out[b * shots + s] = first + found;
+  if (live && l == 0) out[b * shots + s] = (lo << cl) + ((int64_t)k << sl) + found;
 }
 
 // chunks of up to 2^10 indices, stretches of up to 2^6; cum: batch x

@@ -77,3 +77,39 @@ def test_terms_of_many_states(gpu):
     st[:, 1] = 1.0
     e = ham.expect_terms(st)
     assert bool((e.real == -1.0).all()) and bool((e.imag == 0.0).all())
+
+
+def draws(p, u):
+    from tensorcircuit_amd import engine
+
+    n = p.shape[1].bit_length() - 1
+    return engine.sample_prob_indices(p.cuda(), n, torch.as_tensor(u)).cpu().numpy()
+
+
+# one stretch of 64 indices, one chunk of 1024, several chunks, more than 256
+# and more than 4096 of them: the running sums over indices without weight
+# (behind, before and between those with weight) stay what they are, so that
+# no such index is drawn, least of all for u = 0
+@pytest.mark.parametrize("n", [2, 6, 9, 10, 12, 18, 19, 20, 23])
+def test_draws_have_weight(gpu, n):
+    N = 1 << n
+    reps = 2 if n > 20 else 10 if n > 12 else 40
+    for dt in (torch.float32, torch.float64):
+        for seed in range(reps):
+            rng = np.random.default_rng(1000 * n + seed)
+            w = rng.random((3, N))
+            cut = int(rng.integers(1, N))
+            w[0, cut:] = 0.0
+            w[1, N // 2:] = 0.0
+            w[2] *= np.repeat(rng.random(max(N // 32, 1)) < 0.3, min(N, 32))  # 32 at a time
+            w[2, rng.integers(0, N)] = 1.0
+            p = torch.as_tensor(w).to(dt)
+            u = np.concatenate([np.zeros((3, 1)), rng.random((3, 200))], axis=1)
+            # r on the running sums themselves
+            cdf = np.cumsum(p.double().numpy(), axis=1)
+            at = rng.integers(0, N, (3, 50))
+            u = np.concatenate([u, np.maximum(0.0, 1.0 - np.take_along_axis(cdf, at, 1) / cdf[:, -1:])], axis=1)
+            u = np.where(u < 1.0, u, 0.5)
+            got = draws(p, u)
+            drawn = np.take_along_axis(p.numpy(), got, 1)
+            assert (drawn > 0).all(), (dt, seed, np.argwhere(~(drawn > 0))[:5])
