@@ -113,3 +113,13 @@ def test_draws_have_weight(gpu, n):
             got = draws(p, u)
             drawn = np.take_along_axis(p.numpy(), got, 1)
             assert (drawn > 0).all(), (dt, seed, np.argwhere(~(drawn > 0))[:5])
+
+
+@pytest.mark.parametrize("shots", [1, 70])
+def test_draws_from_one_qubit(gpu, shots):
+    rng = np.random.default_rng(shots)
+    p = torch.as_tensor([[0.25, 0.75], [1.0, 0.0], [0.0, 2.0], [3.0, 1.0]])
+    u = rng.random((4, shots))
+    r = p.numpy().sum(axis=1, keepdims=True) * (1.0 - u)
+    for dt in (torch.float32, torch.float64):
+        assert (draws(p.to(dt), u) == (r > p.numpy()[:, :1])).all()
