@@ -65,33 +65,37 @@ __global__ void __launch_bounds__(256) k_sample_sums(const void* __restrict__ sr
     const double s = scan16(tot[threadIdx.x], threadIdx.x);
     if ((int)threadIdx.x < nsub) sub[(b * nchunks + c) * nsub + threadIdx.x] = s;
     if ((int)threadIdx.x == nsub - 1) cum[b * (nchunks + 1) + c + 1] = s;
+    if (c == 0 && threadIdx.x == 0) cum[b * (nchunks + 1)] = 0.0;
   }
 }
 
-// In-place inclusive prefix sums of cum[b][1 .. nchunks], cum[b][0] = 0; one
-// 1024-thread block per batch item, 4096 sums at a time through LDS so that
-// memory is read and written in order (a contiguous range per thread: 32 us
-// for 16384 sums; this: 11 us).
-__global__ void __launch_bounds__(1024) k_sample_scan(double* __restrict__ cum, int64_t nchunks) {
-  __shared__ double buf[4096 + 1024];
-  __shared__ double wt[16];
+// In-place inclusive prefix sums of cum[b][1 .. nchunks]; one block per batch
+// item, 4 NT sums at a time through LDS so that memory is read and written in
+// order (a contiguous range per thread: 32 us for 16384 sums; this: 11 us).
+// A wave where a batch item has up to 256 sums (one draw from each of 4096
+// vectors of 14 qubits: 123 us with 1024 threads, 100 us), none where it has one
+// (of 6 qubits: 41 us with the scan, 17.5 us).
+template <int NT>
+__global__ void __launch_bounds__(NT) k_sample_scan(double* __restrict__ cum, int64_t nchunks) {
+  __shared__ double buf[4 * NT + NT];
+  __shared__ double wt[NT / 64];
   __shared__ double last;
   double* c = cum + blockIdx.x * (nchunks + 1) + 1;
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   auto at = [](int i) { return i + (i >> 2); };
   double carry = 0.0, nx[4];
-  auto fetch = [&](int64_t base) {  // the next 4096, while these are summed
+  auto fetch = [&](int64_t base) {  // the next ones, while these are summed
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int64_t i = base + q * 1024 + t;
+      const int64_t i = base + q * NT + t;
       nx[q] = i < nchunks ? c[i] : 0.0;
     }
   };
   fetch(0);
-  for (int64_t base = 0; base < nchunks; base += 4096) {
+  for (int64_t base = 0; base < nchunks; base += 4 * NT) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) buf[at(q * 1024 + t)] = nx[q];
-    fetch(base + 4096);
+    for (int q = 0; q < 4; ++q) buf[at(q * NT + t)] = nx[q];
+    fetch(base + 4 * NT);
     __syncthreads();
     double v[4];
 #pragma unroll
@@ -112,17 +116,16 @@ __global__ void __launch_bounds__(1024) k_sample_scan(double* __restrict__ cum, 
       run += v[q];
       buf[at(4 * t + q)] = run;
     }
-    if (t == 1023) last = run;
+    if (t == NT - 1) last = run;
     __syncthreads();
     carry = last;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int i = q * 1024 + t;
+      const int i = q * NT + t;
       if (base + i < nchunks) c[base + i] = buf[at(i)];
     }
     __syncthreads();
   }
-  if (t == 0) c[-1] = 0.0;
 }
 
 // 16 lanes per draw: r = total (1 - u); the drawn index is the smallest i
@@ -228,7 +231,8 @@ void launch_sample(const void* src, bool prob, int n, int64_t batch, const doubl
   const dim3 gc((unsigned)nchunks, (unsigned)batch), gd((unsigned)((shots + 15) / 16), (unsigned)batch);
   if (prob) hipLaunchKernelGGL((k_sample_sums<T, true>), gc, dim3(256), 0, st, src, sstride, cl, sl, nchunks, cum, sub);
   else hipLaunchKernelGGL((k_sample_sums<T, false>), gc, dim3(256), 0, st, src, sstride, cl, sl, nchunks, cum, sub);
-  hipLaunchKernelGGL(k_sample_scan, dim3((unsigned)batch), dim3(1024), 0, st, cum, nchunks);
+  if (nchunks > 256) hipLaunchKernelGGL(k_sample_scan<1024>, dim3((unsigned)batch), dim3(1024), 0, st, cum, nchunks);
+  else if (nchunks > 1) hipLaunchKernelGGL(k_sample_scan<64>, dim3((unsigned)batch), dim3(64), 0, st, cum, nchunks);
   if (prob)
     hipLaunchKernelGGL((k_sample_draw<T, true>), gd, dim3(256), 0, st, src, sstride, cl, sl, nchunks,
                        (const double*)cum, (const double*)sub, u, shots, out);
