@@ -121,18 +121,16 @@ __device__ __forceinline__ void put_phase(T* o, int low, const T* u, double re, 
   o[low + 1] = (T)(sg * (im - (double)u[1]));
 }
 
-// t = tan(ph / 2) and s = sin(ph) of the three shears.  In float, of the 9
-// pairs around them the one whose matrix M = [[1 - ts, -t (2 - ts)], [s, 1 - ts]]
-// has the least 16 |symmetric part|^2 + |angle error|^2 of M R(ph)^T - 1
-// (see store_diagonal; cs, sn: cos ph, sin ph).
-__device__ __forceinline__ void store_shears(double* o, double ph) {
-  o[0] = tan(0.5 * ph);
-  o[1] = sin(ph);
+// t = tan(ph / 2) and s = sin(ph) of the three shears, from cs = cos ph >= 0
+// and sn = sin ph.  In float, of the 9 pairs around them the one whose matrix
+// M = [[1 - ts, -t (2 - ts)], [s, 1 - ts]] has the least 16 |symmetric part|^2
+// + |angle error|^2 of M R(ph)^T - 1 (see store_diagonal).
+__device__ __forceinline__ void store_shears(double* o, double cs, double sn) {
+  o[0] = sn / (1.0 + cs);
+  o[1] = sn;
 }
-__device__ __forceinline__ void store_shears(float* o, double ph) {
-  double cs, sn;
-  sincos(ph, &sn, &cs);
-  const float t0 = (float)tan(0.5 * ph), s0 = (float)sn;
+__device__ __forceinline__ void store_shears(float* o, double cs, double sn) {
+  const float t0 = (float)(sn / (1.0 + cs)), s0 = (float)sn;
   o[0] = t0;
   o[1] = s0;
   if (t0 == 0.0f || s0 == 0.0f) return;
@@ -152,18 +150,16 @@ __device__ __forceinline__ void store_shears(float* o, double ph) {
     }
 }
 
-// The entries kRotShear.. of an rx or ry recipe: three shears (Paeth), the
-// rotation by phi' is x -= t y, y += s x, x -= t y with t = tan(phi' / 2),
-// s = sin phi'; phi' is phi reduced into [-pi/2, pi/2] (|t| <= 1) by
-// R(phi) = -R(phi - pi), the sign kept in sigma.
+// The entries kRotShear.. of an rx or ry recipe from c = cos phi, s = sin phi:
+// three shears (Paeth), the rotation by phi' is x -= t y, y += s' x, x -= t y
+// with t = tan(phi' / 2), s' = sin phi'; phi' is phi brought into [-pi/2, pi/2]
+// (|t| <= 1) by R(phi) = -R(phi - pi), the sign kept in sigma.  All from c and
+// s, whose reduction of the angle is exact: by the remainder of phi, a unit of
+// pi was lost with every turn (1e-8 after 10^8).
 template <typename T>
-__device__ __forceinline__ void put_rotation(T* o, double phi) {
-  double ph = remainder(phi, 2.0 * M_PI), sigma = 1.0;
-  if (fabs(ph) > 0.5 * M_PI) {
-    ph -= copysign(M_PI, ph);
-    sigma = -1.0;
-  }
-  store_shears(o + kRotShear, ph);
+__device__ __forceinline__ void put_rotation(T* o, double c, double s) {
+  const double sigma = c < 0.0 ? -1.0 : 1.0;
+  store_shears(o + kRotShear, sigma * c, sigma * s);
   o[kRotSigma] = (T)sigma;
 }
 
@@ -201,7 +197,7 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
         T u[2];
         store_diagonal(u, c, s);
         o[0] = u[0]; o[1] = 0; o[2] = 0; o[3] = -u[1]; o[4] = 0; o[5] = -u[1]; o[6] = u[0]; o[7] = 0;
-        if (r.extra) put_rotation(o, 0.5 * a);
+        if (r.extra) put_rotation(o, c, s);
       } break;
       case TCM_G_RY: {
         double c, s;
@@ -209,7 +205,7 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
         T u[2];
         store_diagonal(u, c, s);
         o[0] = u[0]; o[1] = -u[1]; o[2] = u[1]; o[3] = u[0];
-        if (r.extra) put_rotation(o, 0.5 * a);
+        if (r.extra) put_rotation(o, c, s);
       } break;
       case TCM_G_RZ:
       case TCM_G_RZZ: {

@@ -123,3 +123,22 @@ def test_draws_from_one_qubit(gpu, shots):
     r = p.numpy().sum(axis=1, keepdims=True) * (1.0 - u)
     for dt in (torch.float32, torch.float64):
         assert (draws(p.to(dt), u) == (r > p.numpy()[:, :1])).all()
+
+
+@pytest.mark.parametrize("kind", ["rx", "ry"])
+@pytest.mark.parametrize("jit", [0, 1])
+def test_angles_of_many_turns(gpu, kind, jit):
+    """Rotations by angles of up to 10^9, reduced to one turn without loss."""
+    from tensorcircuit_amd import _lib, engine
+
+    n = 10
+    th = np.array([0.3, -2.0, 3.0, 4.0, 9.5, 1e3, -1e5, 1e7, 12345678.9, -1e9])
+    code = {"rx": _lib.G_RX, "ry": _lib.G_RY}[kind]
+    prog = engine.Program(n, [engine.GateSpec(code, (q,), q, 0.0, 1.0, None) for q in range(n)], n, fuse=1, jit=jit)
+    got = np_of(prog.forward(torch.as_tensor(th)[None].to(gpu), 1, "complex128")[0])[0]
+    ref = np.ones(1)
+    for t in th:
+        c, s = np.cos(0.5 * t), np.sin(0.5 * t)
+        ref = np.kron(ref, [c, -1j * s if kind == "rx" else s])
+    # ten rotations, each of up to three shears with two rounded constants
+    assert np.abs(got - ref).max() <= 10 * 3 * 4 * 2.0**-53
