@@ -101,8 +101,10 @@ __global__ void __launch_bounds__(256) k_csr(const int64_t* __restrict__ rowptr,
         hr = a + ((double)gb.x * dr - (double)gb.y * di);
         hi = c + ((double)gb.x * di + (double)gb.y * dr);
       } else {
-        hr *= 2.0 * (double)gb.x;
-        hi *= 2.0 * (double)gb.x;
+        // the imaginary parts cancel; one that is not finite leaves NaN
+        const double a = 2.0 * (double)gb.x + ((double)gb.y - (double)gb.y);
+        hr *= a;
+        hi *= a;
       }
     }
     if constexpr (MODE != CSR_EXPECT) {

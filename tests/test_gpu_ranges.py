@@ -142,3 +142,23 @@ def test_angles_of_many_turns(gpu, kind, jit):
         ref = np.kron(ref, [c, -1j * s if kind == "rx" else s])
     # ten rotations, each of up to three shears with two rounded constants
     assert np.abs(got - ref).max() <= 10 * 3 * 4 * 2.0**-53
+
+
+@pytest.mark.parametrize("hermitian", [True, False])
+def test_sparse_cotangent_that_is_not_finite(gpu, hermitian):
+    """A cotangent with a NaN part shows in the gradient, also where only its
+    real part counts (A = A^dagger)."""
+    from tensorcircuit_amd import engine
+
+    N = 64
+    rng = np.random.default_rng(5)
+    m = rng.standard_normal((N, N)) + 1j * rng.standard_normal((N, N))
+    if hermitian:
+        m = m + m.conj().T
+    x = torch.as_tensor(rng.standard_normal((2, N)) + 0j).to(gpu)
+    a = engine.CsrMatrix(torch.as_tensor(m).to(gpu).to_sparse_csr(), 6, torch.complex128)
+    assert a.hermitian == hermitian
+    for bad in (complex(1.0, float("nan")), complex(float("nan"), 1.0), complex(0.0, float("inf"))):
+        y = a.vjp(x, torch.tensor([bad, 1.0 + 0j], device=gpu))
+        assert not torch.isfinite(torch.view_as_real(y[0])).any()
+        assert torch.isfinite(torch.view_as_real(y[1])).all()
