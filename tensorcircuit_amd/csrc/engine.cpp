@@ -1478,11 +1478,10 @@ int tcm_csr_expect(int32_t n, int32_t dtype, const int64_t* rowptr, const int64_
     return set_error(TCM_E_ARG, "bad arguments to tcm_csr_expect");
   if (ws_bytes < 2 * kCsrBlocks * (int64_t)sizeof(double)) return set_error(TCM_E_WORKSPACE, "workspace too small");
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nrows = (int64_t)1 << n;
   if (dtype == TCM_C64)
-    launch_csr_expect<float>(rowptr, cols, vals, state, nrows, (double*)workspace, out, st);
+    launch_csr_expect<float>(rowptr, cols, vals, state, n, (double*)workspace, out, st);
   else
-    launch_csr_expect<double>(rowptr, cols, vals, state, nrows, (double*)workspace, out, st);
+    launch_csr_expect<double>(rowptr, cols, vals, state, n, (double*)workspace, out, st);
   HIP_TRY(hipGetLastError(), "csr_expect launch");
   return 0;
 }
@@ -1566,11 +1565,10 @@ int tcm_csr_matvec(int32_t n, int32_t dtype, const int64_t* rowptr, const int64_
     return set_error(TCM_E_ARG, "bad arguments to tcm_csr_matvec");
   if (batch == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nrows = (int64_t)1 << n;
   if (dtype == TCM_C64)
-    launch_csr_matvec<float>(rowptr, cols, vals, x, y, nrows, batch, st);
+    launch_csr_matvec<float>(rowptr, cols, vals, x, y, n, batch, st);
   else
-    launch_csr_matvec<double>(rowptr, cols, vals, x, y, nrows, batch, st);
+    launch_csr_matvec<double>(rowptr, cols, vals, x, y, n, batch, st);
   HIP_TRY(hipGetLastError(), "csr_matvec launch");
   return 0;
 }
@@ -1584,11 +1582,10 @@ int tcm_csr_expect_vjp(int32_t n, int32_t dtype, const int64_t* rowptr, const in
     return set_error(TCM_E_ARG, "bad arguments to tcm_csr_expect_vjp");
   if (batch == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nrows = (int64_t)1 << n;
   if (dtype == TCM_C64)
-    launch_csr_vjp<float>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, nrows, batch, st);
+    launch_csr_vjp<float>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, n, batch, st);
   else
-    launch_csr_vjp<double>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, nrows, batch, st);
+    launch_csr_vjp<double>(rowptr, cols, vals, dag_rowptr, dag_cols, dag_vals, x, g, y, n, batch, st);
   HIP_TRY(hipGetLastError(), "csr_expect_vjp launch");
   return 0;
 }

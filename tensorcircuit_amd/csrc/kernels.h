@@ -258,13 +258,13 @@ void launch_pauli_terms_apply(const PauliTermTables& D, int nchunks, int nterms,
 constexpr int kCsrBlocks = 2048;  // most blocks, and partial sums, of a launch
 template <typename T>
 void launch_csr_matvec(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* x, void* y,
-                       int64_t nrows, int64_t batch, hipStream_t st);
+                       int n, int64_t batch, hipStream_t st);
 template <typename T>
 void launch_csr_vjp(const int64_t* rowptr, const int64_t* cols, const void* vals, const int64_t* drowptr,
-                    const int64_t* dcols, const void* dvals, const void* x, const void* g, void* y, int64_t nrows,
+                    const int64_t* dcols, const void* dvals, const void* x, const void* g, void* y, int n,
                     int64_t batch, hipStream_t st);
 template <typename T>
-void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* psi, int64_t nrows,
+void launch_csr_expect(const int64_t* rowptr, const int64_t* cols, const void* vals, const void* psi, int n,
                        double* part, double* out, hipStream_t st);
 // src: states [batch][2^n] (prob false) or probability vectors (prob true);
 // cum: scratch of sample_ws (sample.hip)
