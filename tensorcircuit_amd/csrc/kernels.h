@@ -162,18 +162,18 @@ int jit_launch_adj(const Sched& S, const DeviceTables& D, int pi, int dt, const 
 constexpr int64_t kMaxLaunchThreads = 1ll << 31;
 
 // matrix tables of up to kMaxPrepJobs schedules in one launch, and of at most
-// kMaxPrepBlocks batch items (blocks of 256 threads)
+// kMaxPrepItems batch items (of at most 256 threads each)
 constexpr int kMaxPrepJobs = 16;
-constexpr int64_t kMaxPrepBlocks = kMaxLaunchThreads / 256;
+constexpr int64_t kMaxPrepItems = kMaxLaunchThreads / 256;
 struct PrepJob {
   const void *rec, *fac, *params, *ctab;
   void* mtab;
-  int64_t pstride, mstride, block0;
-  int32_t nrec, first_dg, dg_log, pad;
+  int64_t pstride, mstride, block0, batch;
+  int32_t nrec, first_dg, dg_log, wlog;
 };
 struct PrepJobs {
   int32_t njobs = 0, widest = 0;
-  int64_t blocks = 0;
+  int64_t items = 0;
   PrepJob job[kMaxPrepJobs];
 };
 // adds a job; launches the jobs at either limit

@@ -164,14 +164,16 @@ __device__ __forceinline__ void put_rotation(T* o, double c, double s) {
 }
 
 // ---------------------------------------------------------------------------
-// matrix preparation: a block evaluates every recipe of one batch item of one
-// schedule from its parameters.  A chain of a few loads and 64-bit sines, so
+// matrix preparation: 2^wlog threads evaluate every recipe of one batch item of
+// one schedule from its parameters.  A chain of a few loads and 64-bit sines, so
 // the schedules of a call (forward and reverse, or the programs of an uneven
 // batch) share a launch: 2 of 5 us became one of 6 us at 12 qubits x 4
 // layers, 9 of 9 us one of 9 us for 9 programs.  Blocks are 1024 threads
 // where a batch item has more than 512 entries
 // and its block would be alone on its CU (2 of 63 us with 256 threads,
 // one of 27 us, for 1420 gates and 4 parameter sets), else 256.
+// Items of few entries share a block (2^20 parameter sets of one rotation,
+// complex64, forward on 2 qubits: 1.62 ms with a block each, 0.05 ms).
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
@@ -181,11 +183,13 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
   const DFactor* __restrict__ fac = (const DFactor*)J.job[q].fac;
   const T* __restrict__ ct = (const T*)J.job[q].ctab;
   const int nrec = J.job[q].nrec, first_dg = J.job[q].first_dg, dg_log = J.job[q].dg_log;
-  const int64_t b = blockIdx.x - J.job[q].block0;
+  const int wlog = J.job[q].wlog, W = 1 << wlog, lane = threadIdx.x & (W - 1);
+  const int64_t b = (((int64_t)blockIdx.x - J.job[q].block0) * blockDim.x + threadIdx.x) >> wlog;
+  const bool have = b < J.job[q].batch;
   T* mt = (T*)J.job[q].mtab + b * J.job[q].mstride;
   const T* __restrict__ pr = (const T*)J.job[q].params;
   if (pr) pr += b * J.job[q].pstride;
-  for (int i = threadIdx.x; i < first_dg; i += blockDim.x) {
+  for (int i = lane; i < first_dg && have; i += W) {
     const DRecipe r = rec[i];
     if (r.kind < 0) continue;
     double a = r.param >= 0 ? r.scale * (double)pr[r.param] : r.theta;
@@ -298,10 +302,10 @@ __global__ void __launch_bounds__(1024) k_prep(PrepJobs J) {
   }
   __syncthreads();
   // fused diagonals (recipes first_dg..nrec-1): products of member diagonals
-  // over the group index j; thread t takes recipe first_dg + (t >> dg_log)
+  // over the group index j; lane t takes recipe first_dg + (t >> dg_log)
   // and entry t & (2^dg_log - 1), so all recipes are built side by side
   const int ndg = nrec - first_dg;
-  for (int t = threadIdx.x; t < (ndg << dg_log); t += blockDim.x) {
+  for (int t = lane; t < (ndg << dg_log) && have; t += W) {
     const DRecipe r = rec[first_dg + (t >> dg_log)];
     const int j = t & ((1 << dg_log) - 1);
     if (r.kind >= 0 || j >= (1 << r.R)) continue;
@@ -1079,22 +1083,29 @@ void add_prep(PrepJobs& J, const Sched& S, const DeviceTables& D, const void* ct
       dg_log = std::max(dg_log, (int)S.recipes[i].R);
     }
   for (int64_t b0 = 0; b0 < batch;) {
-    const int64_t nb = std::min(batch - b0, kMaxPrepBlocks - J.blocks);
+    const int64_t nb = std::min(batch - b0, kMaxPrepItems - J.items);
     J.job[J.njobs++] = PrepJob{D.recipes, D.factors, params ? (const T*)params + b0 * pstride : nullptr, ctab,
-                               (T*)mtab + b0 * S.mtab_size, pstride, (int64_t)S.mtab_size, J.blocks,
+                               (T*)mtab + b0 * S.mtab_size, pstride, (int64_t)S.mtab_size, 0, nb,
                                nrec, first_dg, dg_log, 0};
-    J.blocks += nb;
+    J.items += nb;
     J.widest = std::max({J.widest, first_dg, (nrec - first_dg) << dg_log});
-    if (J.njobs == kMaxPrepJobs || J.blocks == kMaxPrepBlocks) launch_prep<T>(J, st);
+    if (J.njobs == kMaxPrepJobs || J.items == kMaxPrepItems) launch_prep<T>(J, st);
     b0 += nb;
   }
 }
 
 template <typename T>
 void launch_prep(PrepJobs& J, hipStream_t st) {
-  if (J.njobs)
-    hipLaunchKernelGGL(k_prep<T>, dim3((unsigned)J.blocks), dim3(J.widest > 512 && J.blocks <= 1024 ? 1024 : 256), 0,
-                       st, J);
+  const int threads = J.widest > 512 && J.items <= 1024 ? 1024 : 256;
+  int64_t blocks = 0;
+  for (int q = 0; q < J.njobs; ++q) {
+    PrepJob& p = J.job[q];
+    const int wide = std::max(p.first_dg, (p.nrec - p.first_dg) << p.dg_log);
+    while ((1 << p.wlog) < std::min(wide, threads)) ++p.wlog;
+    p.block0 = blocks;
+    blocks += ((p.batch << p.wlog) + threads - 1) / threads;
+  }
+  if (blocks) hipLaunchKernelGGL(k_prep<T>, dim3((unsigned)blocks), dim3(threads), 0, st, J);
   J = PrepJobs();
 }
 

@@ -162,3 +162,20 @@ def test_sparse_cotangent_that_is_not_finite(gpu, hermitian):
         y = a.vjp(x, torch.tensor([bad, 1.0 + 0j], device=gpu))
         assert not torch.isfinite(torch.view_as_real(y[0])).any()
         assert torch.isfinite(torch.view_as_real(y[1])).all()
+
+
+# tables of 1, 2, 5, 24, 60 and 300 entries: up to 256 parameter sets to a
+# block, one set and part of one; batches that leave the last block part empty
+@pytest.mark.parametrize("n,gates", [(1, 1), (2, 2), (3, 5), (4, 3), (6, 24), (8, 60), (10, 300)])
+@pytest.mark.parametrize("batch", [2, 5, 129, 257])
+def test_tables_sharing_blocks(gpu, n, gates, batch):
+    from tensorcircuit_amd import _lib, engine
+
+    kinds = (_lib.G_RX, _lib.G_RZ, _lib.G_RY, _lib.G_PHASE)
+    specs = [engine.GateSpec(kinds[g % 4], (g % n,), g, 0.0, 1.0, None) for g in range(gates)]
+    prog = engine.Program(n, specs, gates, fuse=1)
+    for dt, rdt in (("complex64", torch.float32), ("complex128", torch.float64)):
+        p = torch.randn(batch, gates, dtype=rdt, device=gpu)
+        st, _ = prog.forward(p, batch, dt)
+        for b in sorted({0, 1, batch // 2, batch - 2, batch - 1}):
+            assert torch.equal(st[b], prog.forward(p[b:b + 1], 1, dt)[0][0])
