@@ -516,6 +516,8 @@ void pauli_sort_strings(tcm_pauli* H, std::map<uint64_t, std::vector<std::pair<i
       DPGroupX g{(uint32_t)kv.first, 0};
       for (; i < ts.size() && ch.nt < kTermsChunk; ++i, ++ch.nt) {
         g.cnt += ts[i].first ? 0x10000u : 1u;
+        ts[i].second.flip = g.flip;
+        ts[i].second.odd = (uint32_t)ts[i].first;
         H->xterms.push_back(ts[i].second);
       }
       H->xgroups.push_back(g);

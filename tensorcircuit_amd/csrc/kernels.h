@@ -54,6 +54,7 @@ struct DPPass {
 struct DPTermX {
   double w;
   uint32_t yz, idx;
+  uint32_t flip, odd;  // its group's
 };
 struct DPGroupX {
   uint32_t flip, cnt;

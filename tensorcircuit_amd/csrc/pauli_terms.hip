@@ -10,15 +10,16 @@
 //   (P psi)[a] = (-i)^ny (-1)^popcount(a & yz) psi[a ^ flip].
 // State layout: [batch][2^n] complex, qubit 0 = most significant index bit.
 //
-// Both walk tiles of 2^k consecutive amplitudes held in LDS, 2^LE per thread
-// at positions it << tl | tid, with the strings sorted by flip mask (DPGroupX,
+// Two ways for each, chosen by the number of strings and amplitudes (each_term,
+// each_term_apply): straight from memory, a string or 16 bytes at a time, or
+// by tiles of 2^k consecutive amplitudes held in LDS, 2^LE per thread at
+// positions it << tl | tid, with the strings sorted by flip mask (DPGroupX,
 // DPTermX): a partner whose flip stays inside the tile is an LDS read, one
 // outside it a coalesced read of another tile; conj(psi) psi' is formed once
 // per flip mask, and the sign of a string splits into block, thread and
-// element parts.  One launch per string that read both amplitudes from memory
-// took 67 us (59 strings of a 20-qubit complex64 state), and a thread per
-// amplitude over all strings 76 us for the application; these take 25 and 30 us,
-// bound by their issue of 64-bit operations and LDS reads at two waves per SIMD.
+// element parts.  59 strings of a 20-qubit complex64 state: 67 us from memory
+// (8 bytes at a time), 25 us by tiles; applied, 76 and 30 us, bound by their
+// issue of 64-bit operations and LDS reads at two waves per SIMD.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -303,9 +304,116 @@ __global__ void __launch_bounds__(512) k_pauli_terms_apply(const DPChunk* __rest
 }
 
 namespace {
+// 16 bytes of a state: one complex128 amplitude, or two of complex64, those
+// at the positions of a flipped within the 16 bytes as well
+template <typename T>
+constexpr int kQuad = 16 / sizeof(V2<T>);
+__device__ __forceinline__ void load_quad(V2<double>* q, const V2<double>* s, uint32_t a) { q[0] = s[a]; }
+__device__ __forceinline__ void load_quad(V2<float>* q, const V2<float>* s, uint32_t a) {
+  const float4 v = *reinterpret_cast<const float4*>(s + (a & ~1u));
+  const bool odd = a & 1u;
+  q[0].x = odd ? v.z : v.x;
+  q[0].y = odd ? v.w : v.y;
+  q[1].x = odd ? v.x : v.z;
+  q[1].y = odd ? v.y : v.w;
+}
+__device__ __forceinline__ void store_quad(V2<double>* s, const double* re, const double* im) {
+  *s = double2{re[0], im[0]};
+}
+__device__ __forceinline__ void store_quad(V2<float>* s, const double* re, const double* im) {
+  *reinterpret_cast<float4*>(s) = float4{(float)re[0], (float)im[0], (float)re[1], (float)im[1]};
+}
+}  // namespace
+
+// part as k_pauli_terms, blocks of one string each and no tiles: both
+// amplitudes from memory.  grid (nblk, nterms, batch)
+template <typename T>
+__global__ void __launch_bounds__(256) k_pauli_terms_each(const DPTermX* __restrict__ terms, int n, int nterms,
+                                                          const V2<T>* __restrict__ psi, double* __restrict__ part) {
+  constexpr int E = kQuad<T>;
+  __shared__ double red[4];
+  const DPTermX tm = terms[blockIdx.y];
+  const int64_t b = blockIdx.z;
+  const V2<T>* s = psi + (b << n);
+  const uint64_t N = 1ull << n;
+  double x = 0.0;
+  for (uint64_t i = (blockIdx.x * 256ull + threadIdx.x) * E; i < N; i += gridDim.x * 256ull * E) {
+    const uint32_t a = (uint32_t)i;
+    V2<T> p[E], q[E];
+    load_quad(p, s, a);
+    load_quad(q, s, a ^ tm.flip);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const double c = tm.odd ? (double)p[e].y * q[e].x - (double)p[e].x * q[e].y
+                              : (double)p[e].x * q[e].x + (double)p[e].y * q[e].y;
+      x += with_sign(c, __popc((a + e) & tm.yz) & 1u);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    part[(b * nterms + tm.idx) * gridDim.x + blockIdx.x] = tm.w * ((red[0] + red[1]) + (red[2] + red[3]));
+}
+
+// out as k_pauli_terms_apply, 16 bytes per thread over all strings
+template <typename T>
+__global__ void __launch_bounds__(256) k_pauli_terms_apply_each(const DPTermX* __restrict__ terms, int n, int nterms,
+                                                                const V2<T>* __restrict__ psi,
+                                                                V2<T>* __restrict__ out,
+                                                                const double* __restrict__ wts, int64_t total) {
+  constexpr int E = kQuad<T>;
+  for (int64_t i = (blockIdx.x * 256ll + threadIdx.x) * E; i < total; i += gridDim.x * 256ll * E) {
+    const int64_t b = i >> n;
+    const uint32_t a = (uint32_t)(i & (((int64_t)1 << n) - 1));
+    const V2<T>* s = psi + (b << n);
+    const double* wb = wts + b * nterms;
+    double hr[E], hi[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) hr[e] = hi[e] = 0.0;
+    for (int t = 0; t < nterms; ++t) {
+      const DPTermX tm = terms[t];
+      const double w = tm.w * wb[tm.idx];
+      if (w == 0.0) continue;
+      V2<T> q[E];
+      load_quad(q, s, a ^ tm.flip);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const double c = with_sign(w, __popc((a + e) & tm.yz) & 1u);
+        hr[e] += tm.odd ? -c * (double)q[e].y : c * (double)q[e].x;
+        hi[e] += tm.odd ? c * (double)q[e].x : c * (double)q[e].y;
+      }
+    }
+    store_quad(out + i, hr, hi);
+  }
+}
+
+namespace {
 // 32 KiB tiles; 8 amplitudes per thread, 1 where that would not fill a wave
 template <typename T>
 int tile_bits(int n) { return std::min(n, sizeof(T) == 4 ? 12 : 11); }
+
+bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Without tiles, from 9 qubits (below, a tile is a wave with one amplitude per
+// thread and as fast) and for states that can be read 16 bytes at a time:
+//  - one or two strings, which leave little to share (expectation of one on
+//    8 x 2^22 amplitudes, complex64: 45 us, 83 by tiles; of four, 98 and 63 us
+//    on 2^24); applied in complex128 up to six (one and four on 8 x 2^22: 179
+//    and 369 us, 329 and 548 by tiles; eight on 64 x 2^20: 1083 and 897 us);
+//  - few amplitudes times strings, where tiles are a chain of LDS reads on few
+//    CUs (60 strings on 2^18 amplitudes, complex64: 17 us, 22 by tiles; on 64 x
+//    2^14, 48 and 34 us), or, applied, up to 4 MiB of states (60 strings on 2^10:
+//    18 and 28 us, on 8 x 2^16 28 and 38, on 64 x 2^14 50 and 39 us).
+template <typename T>
+bool each_term(int n, int nterms, int64_t batch, const void* psi) {
+  return n >= 9 && aligned16(psi) && (nterms <= 2 || (batch << n) * nterms * (int64_t)sizeof(V2<T>) <= 128 << 20);
+}
+template <typename T>
+bool each_term_apply(int n, int nterms, int64_t batch, const void* psi, const void* out) {
+  return n >= 9 && aligned16(psi) && aligned16(out) &&
+         (nterms <= (sizeof(T) == 4 ? 2 : 6) || (batch << n) * (int64_t)sizeof(V2<T>) <= 4 << 20);
+}
 }  // namespace
 
 int pauli_terms_blocks(int n, bool c64) { return 1 << std::min(n - (c64 ? tile_bits<float>(n) : tile_bits<double>(n)), 10); }
@@ -322,7 +430,10 @@ void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n
                        (const DPChunk*)D.chunks, (const DPGroupX*)D.groups, (const DPTermX*)D.terms, n, k, nterms,
                        (const V2<T>*)psi, part);
   };
-  if (k >= 9) go(k_pauli_terms<T, 3>, 3);
+  if (each_term<T>(n, nterms, batch, psi))
+    hipLaunchKernelGGL(k_pauli_terms_each<T>, dim3((unsigned)nblk, (unsigned)nterms, (unsigned)batch), dim3(256), 0, st,
+                       (const DPTermX*)D.terms, n, nterms, (const V2<T>*)psi, part);
+  else if (k >= 9) go(k_pauli_terms<T, 3>, 3);
   else go(k_pauli_terms<T, 0>, 0);
   const int64_t total = batch * nterms;
   hipLaunchKernelGGL(k_pauli_terms_sum, dim3((unsigned)std::min(total, kMaxLaunchThreads / 64)), dim3(64), 0, st,
@@ -340,8 +451,16 @@ void launch_pauli_terms_apply(const PauliTermTables& D, int nchunks, int nterms,
                        lds, st, (const DPChunk*)D.chunks, nchunks, (const DPGroupX*)D.groups, (const DPTermX*)D.terms,
                        n, k, nterms, (const V2<T>*)psi, (V2<T>*)out, weights, ntiles);
   };
-  if (k >= 9) go(k_pauli_terms_apply<T, 3>, 3);
-  else go(k_pauli_terms_apply<T, 0>, 0);
+  const int64_t total = batch << n;
+  if (each_term_apply<T>(n, nterms, batch, psi, out)) {
+    const int64_t blocks = std::min<int64_t>(std::max<int64_t>(total / (256 * kQuad<T>), 1), 65536);
+    hipLaunchKernelGGL(k_pauli_terms_apply_each<T>, dim3((unsigned)blocks), dim3(256), 0, st, (const DPTermX*)D.terms, n,
+                       nterms, (const V2<T>*)psi, (V2<T>*)out, weights, total);
+  } else if (k >= 9) {
+    go(k_pauli_terms_apply<T, 3>, 3);
+  } else {
+    go(k_pauli_terms_apply<T, 0>, 0);
+  }
 }
 
 #define TCM_TERMS_INST(T)                                                                                           \

@@ -179,3 +179,36 @@ def test_tables_sharing_blocks(gpu, n, gates, batch):
         st, _ = prog.forward(p, batch, dt)
         for b in sorted({0, 1, batch // 2, batch - 2, batch - 1}):
             assert torch.equal(st[b], prog.forward(p[b:b + 1], 1, dt)[0][0])
+
+
+# many states run by tiles, one state straight from memory: one tile, several,
+# flips that leave it; 33 strings (a second chunk), Z only, and one to seven
+# strings (the lines between the two ways)
+@pytest.mark.parametrize("n,T,batch", [(9, 33, 1100), (10, 40, 700), (11, 33, 300), (12, 90, 150), (13, 64, 60),
+                                       (12, 1, 150), (12, 2, 150), (12, 3, 1500), (11, 7, 1300)])
+@pytest.mark.parametrize("letters", [(0, 1, 2, 3), (0, 3), (0, 0, 0, 1, 3)])
+def test_pauli_strings_by_tiles_and_without(gpu, n, T, batch, letters):
+    from tensorcircuit_amd import engine
+
+    rng = np.random.default_rng(100 * n + T)
+    codes = rng.choice(letters, size=(T, n)).astype(np.int8)
+    w = rng.standard_normal(T)
+    ham = engine.PauliSum(n, codes, w)
+    a = torch.as_tensor(rng.standard_normal((batch, T))).to(gpu)
+    for dt, unit in ((torch.complex64, 2.0**-24), (torch.complex128, 2.0**-53)):
+        st = torch.randn(batch, 1 << n, dtype=dt, device=gpu)
+        st /= torch.linalg.vector_norm(st, dim=1, keepdim=True)
+        e, y = ham.expect_terms(st), ham.apply_terms(st, a)
+        for b in (0, 1, batch // 2, batch - 1):
+            # sums of 2^n products of total size one in 64 bits
+            assert float((e[b] - ham.expect_terms(st[b])[0]).abs().max()) <= np.abs(w).max() * n * 2.0**-50
+            # sums of T in 64 bits, rounded once
+            size = float((a[b].abs() * torch.as_tensor(np.abs(w)).to(gpu)).sum() * st[b].abs().max())
+            assert float((y[b] - ham.apply_terms(st[b], a[b:b + 1])[0]).abs().max()) <= 4 * (unit + T * 2.0**-53) * size
+        # a state that starts between 16-byte boundaries
+        buf = torch.empty((1 << n) + 1, dtype=dt, device=gpu)
+        buf[1:] = st[0]
+        assert float((e[0] - ham.expect_terms(buf[1:])[0]).abs().max()) <= np.abs(w).max() * n * 2.0**-50
+        y0 = ham.apply_terms(buf[1:], a[:1])[0]
+        assert float((y[0] - y0).abs().max()) <= 4 * (unit + T * 2.0**-53) * float(
+            (a[0].abs() * torch.as_tensor(np.abs(w)).to(gpu)).sum() * st[0].abs().max())
