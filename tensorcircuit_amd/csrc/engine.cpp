@@ -561,9 +561,14 @@ void pauli_tile_sched(tcm_pauli* H, int dt) {
   // complex64 tiles of 12 bits (32 KiB of LDS, several blocks per CU), or of
   // 14 bits (128 KiB, one block of 1024 threads per CU) where that saves a
   // pass: a 24-qubit sum of single X terms then takes 2 passes instead of 3.
-  // Not for 15 to 19 qubits, where 14-bit tiles are 2 to 32 blocks a state
-  // and leave most CUs idle (200 strings on 4 x 2^18 amplitudes, H psi: 4
-  // passes of 25 us with 14-bit tiles, 6 of 13 us with 12-bit ones).
+  // Not for 15 to 19 qubits, where 14-bit tiles are 2 to 32 blocks a state and
+  // leave most CUs idle.  What counts is the blocks of a call, but the tiles are
+  // chosen before its batch is known: the line serves one to 21 states.  Time
+  // with 14-bit tiles over that with 12-bit ones, H psi of 30, 100 and 200
+  // random strings: one state of 15 to 19 qubits 1.00, 1.33, 1.53 to 1.47, 1.19,
+  // 1.35; 4 states 0.92 to 1.63, 21 states 0.86 to 1.36.  64 states: 1.15 to
+  // 0.76, and 0.61 to 1.01 with 8 strings, where 12-bit tiles are one launch
+  // more.  20 and 21 qubits: one state 1.32 to 1.04, 4 states 0.98 to 0.87.
   int k = std::min(n, dt == 0 ? 12 : 11);
   const int Lw = std::min(dt == 0 ? 4 : 3, k);
   const uint64_t lmask = (1ull << Lw) - 1;

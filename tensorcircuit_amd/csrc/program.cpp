@@ -1501,10 +1501,14 @@ int build_program(const tcm_gate* gates, int32_t ngates, int32_t n, int32_t npar
     // fewer passes at about the same per-pass bandwidth (24-qubit HEA: 44 +
     // 44 passes instead of 56 + 68)
     const int kd = (dt == 0 ? 12 : 11) + (o.jit ? 1 : 0);
-    // Table-driven complex128 adjoint passes take 64 KiB too from 18 qubits,
-    // where a state has tiles enough (18 qubits x 3, 6 layers: 771 -> 705 us
-    // qaoa, 502 -> 434 hea); below, a single state leaves more CUs idle than
-    // the passes save (17 qubits, hea: 341 -> 359).  Not the forward passes:
+    // Table-driven complex128 adjoint passes take 64 KiB too from 18 qubits.
+    // Fewer passes, but of half as many blocks: what counts is the blocks of a
+    // call, and the tiles are chosen before its batch is known, so the line lies
+    // where one state loses little.  Energy and gradient, time with 32 KiB over
+    // that with 64, 6 layers of hea, qaoa: 17 qubits 0.95, 0.98 for one state
+    // (0.96, 0.99 for 3, 1.13, 1.08 for 8, 0.98, 0.99 for 33); 18 qubits 0.98,
+    // 0.99 for one, 1.02, 1.01 for 2, 1.16, 1.10 for 3, 1.04, 1.04 for 8; 19
+    // qubits 1.00, 1.02 for one; 20 qubits 1.17, 1.10.  Not the forward passes:
     // programs run together share launches, whose LDS is the largest tile's
     // (13 to 18 qubits x 21: 852 -> 1045 us).
     const int kda = kd + (dt == 1 && !o.jit && n >= 18 ? 1 : 0);

@@ -97,7 +97,7 @@ constexpr int kMfmaTileMaxOps = 8;
 // Staged tables of the table-driven tile passes (tile_pass.hip): a pass's
 // segments in processing order (reversed for the adjoint), cut into chunks of
 // a fixed size that one block copies into LDS at a time.
-//   blob words per chunk: [segments, 2 words each][ops, 2 words each]
+//   blob words per chunk: [segments, 2 words each][ops, 4 words each, 3 used]
 //     [members][gradient indices][segment count, gradient count]
 //   segment: tile bit of slot s at bits 4s, the same four ascending at bits
 //     16 + 4i; then its number of ops, at bits 8 + 4s the slots that register
