@@ -229,16 +229,6 @@ __device__ __forceinline__ void ap_swap(A2<T>* v) {
   }
 }
 
-template <typename T, int R, bool DAG>
-__device__ __forceinline__ void ap_dg(A2<T>* v, const T* d) {
-#pragma unroll
-  for (int j = 0; j < (1 << R); ++j) {
-    T dr = d[2 * j], di = DAG ? -d[2 * j + 1] : d[2 * j + 1];
-    A2<T> x = v[j];
-    v[j] = ma<T>(dr * x.x - di * x.y, dr * x.y + di * x.x);
-  }
-}
-
 // apply one op (kinds with a register form) on v
 template <typename T, int R, bool DAG>
 __device__ __forceinline__ void apply_op(A2<T>* v, const DOp& op, const T* mt, const T* ct) {
