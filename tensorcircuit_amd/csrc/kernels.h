@@ -149,6 +149,9 @@ struct DeviceTables {
   std::vector<void*> jit_fn;
 };
 
+// kernels that need more than 64 KiB of dynamic LDS opt in once per device
+void allow_lds(const void* kern, size_t bytes);
+
 // launch compiled pass kernels (jit.cpp)
 int jit_load(const Sched& S, DeviceTables& D);
 // zinit: the pass starts from |0..0> instead of reading `src` (`state` or others)

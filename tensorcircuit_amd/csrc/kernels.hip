@@ -827,15 +827,13 @@ static int64_t resident_grid(Kern kern, size_t lds) {
   return cache[key] = (int64_t)per_cu * ncu;
 }
 
-template <typename K>
-static void ensure_lds_attr(K kern, size_t bytes);
 
 template <int K>
 static void launch_mfma_tile_k(const DPass& P, const DPass* passes_dev, int pi, const DOp* dop_dev,
                                const int32_t* ukbits_dev, const uint32_t* runoff_dev, const void* ctab, const void* src,
                                void* state, int n, int64_t batch, hipStream_t st) {
   const size_t lds = ((size_t)8 << K) + (size_t)P.nmop * (8192 + 32 + (4 << (K - 5)));
-  ensure_lds_attr(k_mfma_tile<K>, lds);
+  allow_lds((const void*)k_mfma_tile<K>, lds);
   const int64_t ntiles = batch << P.nblk_log;
   const int64_t grid = std::min<int64_t>(ntiles, resident_grid(k_mfma_tile<K>, lds));
   hipLaunchKernelGGL(k_mfma_tile<K>, dim3((unsigned)grid), dim3(512), lds, st, passes_dev, pi, dop_dev, ukbits_dev,
@@ -1158,16 +1156,16 @@ void launch_plain_gate(const DOp& op, const int32_t* ukbits_dev, const void* mta
   }
 }
 
-// kernels that need more than 64 KiB of dynamic LDS must opt in once
-template <typename K>
-static void ensure_lds_attr(K kern, size_t bytes) {
+void allow_lds(const void* kern, size_t bytes) {
   if (bytes <= 65536) return;
   static std::mutex mu;
-  static std::map<const void*, size_t> done;
+  static std::map<std::pair<int, const void*>, size_t> done;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return;
   std::lock_guard<std::mutex> lk(mu);
-  size_t& d = done[(const void*)kern];
+  size_t& d = done[{dev, kern}];
   if (bytes <= d) return;
-  (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   d = bytes;
 }
 

@@ -9,8 +9,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 
 #include "kernels.h"
 
@@ -209,20 +207,6 @@ __global__ void __launch_bounds__(1024) k_pauli_tile(PauliTileArgs S, const DPCh
       epart[b * estride + 2 * (A.slot0 + blk) + 1] = ei;
     }
   }
-}
-
-// kernels that need more than 64 KiB of dynamic LDS opt in once
-static void allow_lds(const void* kern, size_t bytes) {
-  if (bytes <= 65536) return;
-  static std::mutex mu;
-  static std::map<std::pair<int, const void*>, size_t> done;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
-  std::lock_guard<std::mutex> lk(mu);
-  size_t& d = done[{dev, kern}];
-  if (bytes <= d) return;
-  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  d = bytes;
 }
 
 template <typename T, int LE, bool ENERGY, bool APPLY>

@@ -9,8 +9,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <type_traits>
 
 #include "kernels.h"
@@ -798,20 +796,6 @@ __global__ void __launch_bounds__(sizeof(T) == 4 ? 1024 : 512) k_tile_adj(
 // host launchers
 // ---------------------------------------------------------------------------
 namespace {
-
-// kernels that need more than 64 KiB of dynamic LDS opt in once per device
-void allow_lds(const void* kern, size_t bytes) {
-  if (bytes <= 65536) return;
-  static std::mutex mu;
-  static std::map<std::pair<int, const void*>, size_t> done;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
-  std::lock_guard<std::mutex> lk(mu);
-  size_t& d = done[{dev, kern}];
-  if (bytes <= d) return;
-  (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  d = bytes;
-}
 
 template <typename T>
 size_t lds_fwd(int k) { return (sizeof(A2<T>) << k) + kStageMat * sizeof(T) + kStageBlob * 4; }
