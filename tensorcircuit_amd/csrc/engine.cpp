@@ -75,6 +75,7 @@ struct tcm_pauli {
   std::vector<DPTerm> terms;
   std::vector<DPTermX> xterms;     // the strings kept apart (pauli_terms.hip)
   std::vector<DPGroupX> xgroups;
+  int xfar[2] = {0, 0};            // their flip masks that leave a tile, per dtype
   std::vector<DPChunk> xchunks;
   int nslots = 0;                  // slots of the per-group kernels
   PauliTileSched ts[2];
@@ -504,6 +505,7 @@ void pauli_sort_strings(tcm_pauli* H, std::map<uint64_t, std::vector<std::pair<i
   };
   for (auto& kv : by_flip) {
     auto& ts = kv.second;
+    for (int dt = 0; dt < 2; ++dt) H->xfar[dt] += pauli_terms_far((uint32_t)kv.first, H->n, dt == TCM_C64);
     std::stable_sort(ts.begin(), ts.end(), [](const std::pair<int, DPTermX>& a, const std::pair<int, DPTermX>& b) {
       if (a.first != b.first) return a.first < b.first;
       // the tile's bits first: strings that differ only outside it share an
@@ -1538,9 +1540,9 @@ int tcm_expect_pauli_terms(const tcm_pauli* ham, int32_t dtype, const void* stat
   const PauliTermTables D{pd->xchunks, pd->xgroups, pd->xterms};
   const int nch = (int)H->xchunks.size();
   if (dtype == TCM_C64)
-    launch_pauli_terms<float>(D, nch, (int)nt, H->n, state, batch, (double*)workspace, out, st);
+    launch_pauli_terms<float>(D, nch, (int)nt, H->xfar, H->n, state, batch, (double*)workspace, out, st);
   else
-    launch_pauli_terms<double>(D, nch, (int)nt, H->n, state, batch, (double*)workspace, out, st);
+    launch_pauli_terms<double>(D, nch, (int)nt, H->xfar, H->n, state, batch, (double*)workspace, out, st);
   HIP_TRY(hipGetLastError(), "pauli_terms launch");
   return 0;
 }

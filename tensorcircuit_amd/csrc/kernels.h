@@ -250,11 +250,13 @@ template <typename T>
 void launch_pauli_coo(const DPGroup* groups, int ngroups, const DPTerm* terms, int n, int64_t nterms, int64_t* rows,
                       int64_t* cols, void* vals, hipStream_t st);
 // per-term Pauli expectations and weighted applications (pauli_terms.hip);
-// part: pauli_terms_blocks partial sums per (state, string)
+// part: pauli_terms_blocks partial sums per (state, string); far: flip masks
+// that leave the tile, complex64 and complex128
 int pauli_terms_blocks(int n, bool c64);
+int pauli_terms_far(uint32_t flip, int n, bool c64);  // 1 where the flip leaves the tile
 template <typename T>
-void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n, const void* psi, int64_t batch,
-                        double* part, double* out, hipStream_t st);
+void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, const int* far, int n, const void* psi,
+                        int64_t batch, double* part, double* out, hipStream_t st);
 template <typename T>
 void launch_pauli_terms_apply(const PauliTermTables& D, int nchunks, int nterms, int n, const void* psi, void* out,
                               const double* weights, int64_t batch, hipStream_t st);

@@ -303,6 +303,30 @@ __global__ void __launch_bounds__(512) k_pauli_terms_apply(const DPChunk* __rest
   }
 }
 
+// part as k_pauli_terms, blocks of one string each and no tiles: both
+// amplitudes from memory.  grid (nblk, nterms, batch)
+template <typename T>
+__global__ void __launch_bounds__(256) k_pauli_terms_each(const DPTermX* __restrict__ terms, int n, int nterms,
+                                                          const V2<T>* __restrict__ psi, double* __restrict__ part) {
+  __shared__ double red[4];
+  const DPTermX tm = terms[blockIdx.y];
+  const int64_t b = blockIdx.z;
+  const V2<T>* s = psi + (b << n);
+  const uint64_t N = 1ull << n;
+  double x = 0.0;
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < N; i += gridDim.x * 256ull) {
+    const uint32_t a = (uint32_t)i;
+    const V2<T> p = s[a], q = s[a ^ tm.flip];
+    const double c = tm.odd ? (double)p.y * q.x - (double)p.x * q.y : (double)p.x * q.x + (double)p.y * q.y;
+    x += with_sign(c, __popc(a & tm.yz) & 1u);
+  }
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    part[(b * nterms + tm.idx) * gridDim.x + blockIdx.x] = tm.w * ((red[0] + red[1]) + (red[2] + red[3]));
+}
+
 namespace {
 // 16 bytes of a state: one complex128 amplitude, or two of complex64, those
 // at the positions of a flipped within the 16 bytes as well
@@ -324,37 +348,6 @@ __device__ __forceinline__ void store_quad(V2<float>* s, const double* re, const
   *reinterpret_cast<float4*>(s) = float4{(float)re[0], (float)im[0], (float)re[1], (float)im[1]};
 }
 }  // namespace
-
-// part as k_pauli_terms, blocks of one string each and no tiles: both
-// amplitudes from memory.  grid (nblk, nterms, batch)
-template <typename T>
-__global__ void __launch_bounds__(256) k_pauli_terms_each(const DPTermX* __restrict__ terms, int n, int nterms,
-                                                          const V2<T>* __restrict__ psi, double* __restrict__ part) {
-  constexpr int E = kQuad<T>;
-  __shared__ double red[4];
-  const DPTermX tm = terms[blockIdx.y];
-  const int64_t b = blockIdx.z;
-  const V2<T>* s = psi + (b << n);
-  const uint64_t N = 1ull << n;
-  double x = 0.0;
-  for (uint64_t i = (blockIdx.x * 256ull + threadIdx.x) * E; i < N; i += gridDim.x * 256ull * E) {
-    const uint32_t a = (uint32_t)i;
-    V2<T> p[E], q[E];
-    load_quad(p, s, a);
-    load_quad(q, s, a ^ tm.flip);
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const double c = tm.odd ? (double)p[e].y * q[e].x - (double)p[e].x * q[e].y
-                              : (double)p[e].x * q[e].x + (double)p[e].y * q[e].y;
-      x += with_sign(c, __popc((a + e) & tm.yz) & 1u);
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    part[(b * nterms + tm.idx) * gridDim.x + blockIdx.x] = tm.w * ((red[0] + red[1]) + (red[2] + red[3]));
-}
 
 // out as k_pauli_terms_apply, 16 bytes per thread over all strings
 template <typename T>
@@ -393,34 +386,44 @@ namespace {
 template <typename T>
 int tile_bits(int n) { return std::min(n, sizeof(T) == 4 ? 12 : 11); }
 
-bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
 // Without tiles, from 9 qubits (below, a tile is a wave with one amplitude per
-// thread and as fast) and for states that can be read 16 bytes at a time:
-//  - one or two strings, which leave little to share (expectation of one on
-//    8 x 2^22 amplitudes, complex64: 45 us, 83 by tiles; of four, 98 and 63 us
-//    on 2^24); applied in complex128 up to six (one and four on 8 x 2^22: 179
-//    and 369 us, 329 and 548 by tiles; eight on 64 x 2^20: 1083 and 897 us);
-//  - few amplitudes times strings, where tiles are a chain of LDS reads on few
-//    CUs (60 strings on 2^18 amplitudes, complex64: 17 us, 22 by tiles; on 64 x
-//    2^14, 48 and 34 us), or, applied, up to 4 MiB of states (60 strings on 2^10:
-//    18 and 28 us, on 8 x 2^16 28 and 38, on 64 x 2^14 50 and 39 us).
+// thread and as fast):
+//  - few amplitudes and strings, where tiles are a chain of LDS reads on few CUs
+//    (expectations of 60 and of 200 strings on 2^16 amplitudes, complex64: 17 and
+//    17 us, 21 and 24 by tiles; of 200 on 2^18, 50 and 32 us; of 16 on 64 x 2^14,
+//    22 and 17 us);
+//  - one or two strings, which leave little to share (one on 8 x 2^22
+//    amplitudes, complex64: 54 us, 83 by tiles; on 64 x 2^20 in complex128 176
+//    and 207), four where most flips leave the tile and a state stays in cache
+//    (four of four on 8 x 2^20, complex128: 52 and 80 us; two of four on 64 x
+//    2^18, 111 and 59 us).
+// far: flip masks that leave the tile
 template <typename T>
-bool each_term(int n, int nterms, int64_t batch, const void* psi) {
-  return n >= 9 && aligned16(psi) && (nterms <= 2 || (batch << n) * nterms * (int64_t)sizeof(V2<T>) <= 128 << 20);
+bool each_term(int n, int nterms, int far, int64_t batch) {
+  if (n < 9) return false;
+  if (nterms <= 2 || (batch << n <= 1 << 18 && (batch << n) * nterms <= 1 << 24)) return true;
+  return nterms <= 4 && 2 * far > nterms && (int64_t)sizeof(V2<T>) << n <= 16 << 20;
 }
+// Applied, for states that can be read 16 bytes at a time:
+//  - up to 2^19 amplitudes (60 strings on 2^10, complex64: 18 us, 28 by tiles; on
+//    8 x 2^16 28 and 38, on 64 x 2^14 50 and 39 us);
+//  - one or two strings, in complex128 up to eight (two on 8 x 2^20, complex64:
+//    24 and 39 us, four on 2^24 94 and 73; eight on 8 x 2^22 in complex128 537
+//    and 619 us, sixteen on 2^24 542 and 540).
 template <typename T>
 bool each_term_apply(int n, int nterms, int64_t batch, const void* psi, const void* out) {
-  return n >= 9 && aligned16(psi) && aligned16(out) &&
-         (nterms <= (sizeof(T) == 4 ? 2 : 6) || (batch << n) * (int64_t)sizeof(V2<T>) <= 4 << 20);
+  if (n < 9 || (((uintptr_t)psi | (uintptr_t)out) & 15)) return false;
+  return nterms <= (sizeof(T) == 4 ? 2 : 8) || batch << n <= 1 << 19;
 }
 }  // namespace
+
+int pauli_terms_far(uint32_t flip, int n, bool c64) { return flip >> (c64 ? tile_bits<float>(n) : tile_bits<double>(n)) ? 1 : 0; }
 
 int pauli_terms_blocks(int n, bool c64) { return 1 << std::min(n - (c64 ? tile_bits<float>(n) : tile_bits<double>(n)), 10); }
 
 template <typename T>
-void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n, const void* psi, int64_t batch,
-                        double* part, double* out, hipStream_t st) {
+void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, const int* far, int n, const void* psi,
+                        int64_t batch, double* part, double* out, hipStream_t st) {
   const int k = tile_bits<T>(n), nblk = pauli_terms_blocks(n, sizeof(T) == 4);
   auto go = [&](auto kern, int le) {
     const unsigned threads = std::max(64u, 1u << (k - le)), nw = threads / 64;
@@ -430,7 +433,7 @@ void launch_pauli_terms(const PauliTermTables& D, int nchunks, int nterms, int n
                        (const DPChunk*)D.chunks, (const DPGroupX*)D.groups, (const DPTermX*)D.terms, n, k, nterms,
                        (const V2<T>*)psi, part);
   };
-  if (each_term<T>(n, nterms, batch, psi))
+  if (each_term<T>(n, nterms, far[sizeof(T) == 8], batch))
     hipLaunchKernelGGL(k_pauli_terms_each<T>, dim3((unsigned)nblk, (unsigned)nterms, (unsigned)batch), dim3(256), 0, st,
                        (const DPTermX*)D.terms, n, nterms, (const V2<T>*)psi, part);
   else if (k >= 9) go(k_pauli_terms<T, 3>, 3);
@@ -464,8 +467,8 @@ void launch_pauli_terms_apply(const PauliTermTables& D, int nchunks, int nterms,
 }
 
 #define TCM_TERMS_INST(T)                                                                                           \
-  template void launch_pauli_terms<T>(const PauliTermTables&, int, int, int, const void*, int64_t, double*,         \
-                                      double*, hipStream_t);                                                        \
+  template void launch_pauli_terms<T>(const PauliTermTables&, int, int, const int*, int, const void*, int64_t,     \
+                                      double*, double*, hipStream_t);                                               \
   template void launch_pauli_terms_apply<T>(const PauliTermTables&, int, int, int, const void*, void*,              \
                                             const double*, int64_t, hipStream_t);
 TCM_TERMS_INST(float)
