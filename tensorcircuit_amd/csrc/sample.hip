@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(NT) k_sample_scan(double* __restrict__ cum, in
 // weights of a stretch, 4 per lane -- about 4 + 1 + 1 dependent reads and 0.7
 // KiB a draw.  (A wave per draw, a binary search and a running scan of the
 // chunk: 14 + 16 dependent reads and up to 8 KiB; 187 us for 100000 draws
-// from 24 qubits, this 23 us.)
+// from 24 qubits, this 20 us.)
 // Tree scans round in another order at every lane, so that a running sum can
 // grow by a unit over entries of zero weight, and r fall in between (the
 // total, for u = 0, did in one of five distributions that end in zeros).  An
@@ -162,58 +162,65 @@ __global__ void __launch_bounds__(256) k_sample_draw(const void* __restrict__ sr
     rem = step;
   }
   const int nsub = 1 << (cl - sl);
-  double sp = l < nsub ? sub[(b * nchunks + lo) * nsub + l] : 0.0;
-  if (r > 0.0 && !mask16(sp != 0.0)) {
-    // the last chunk of nonzero weight before
-    uint32_t some = 0;
+  double c0, sp;
+  uint32_t m, grows;
+  auto read_sums = [&] {
+    c0 = c[lo];
+    sp = l < nsub ? sub[(b * nchunks + lo) * nsub + l] : 0.0;
+    const double before = __shfl_up(sp, 1, 16);
+    m = mask16(l < nsub && c0 + sp >= r);
+    // rounding left r just above the chunk's last sum: its last stretch of
+    // nonzero weight (and, below, the last index of it)
+    grows = mask16(l < nsub && sp > (l ? before : 0.0));
+  };
+  read_sums();
+  // the rare steps back are left to branches of the whole wave
+  if (__any(!m && !grows)) {  // an empty chunk: the last one of nonzero weight before
+    uint32_t some = m | grows;
     for (int64_t e = lo; e > 0 && !some; e -= 16) {
-      some = mask16(e > l && sub[(b * nchunks + (e > l ? e - 1 - l : 0)) * nsub + nsub - 1] != 0.0);
+      some = mask16(e > l && sub[(b * nchunks + (e > l ? e - 1 - l : 0)) * nsub + nsub - 1] > 0.0);
       if (some) lo = e - __ffs(some);
     }
-    if (l < nsub) sp = sub[(b * nchunks + lo) * nsub + l];
+    read_sums();
   }
-  const double c0 = c[lo];
-  const double before = __shfl_up(sp, 1, 16);
-  uint32_t m = mask16(l < nsub && c0 + sp >= r);
-  // rounding left r just above the chunk's last sum: its last stretch of
-  // nonzero weight (and, below, the last index of it)
-  const uint32_t grows = mask16(l < nsub && sp > (l ? before : 0.0));
   int k = m ? __ffs(m) - 1 : grows ? 31 - __clz(grows) : 0;
   // 2^sl weights, `per` consecutive ones per lane
   const int len = 1 << sl, per = len >= 16 ? len >> 4 : 1;
-  double p[4], acc;
-  uint32_t some, nz;  // which of a lane's, which lane's are not zero
-  auto sum_before = [&](int q) {
-    const double prefix = __shfl(sp, q > 0 ? q - 1 : 0, 16);
-    return c0 + (q > 0 ? prefix : 0.0);
-  };
-  double run = sum_before(k);
-  for (;;) {
+  double p[4], acc, run;
+  bool some[4];  // which of them are not zero
+  uint32_t nz;   // in which lanes
+  auto read_weights = [&] {
+    const double prefix = __shfl(sp, k > 0 ? k - 1 : 0, 16);
+    run = c0 + (k > 0 ? prefix : 0.0);
     const int64_t first = b * sstride + (lo << cl) + ((int64_t)k << sl);
+    double x[4];  // all four loads in flight
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = weight_at<T, PROB>(src, first + (j < per && l * per + j < len ? l * per + j : 0));
     acc = 0.0;
-    some = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int i = l * per + j;
-      const double x = j < per && i < len ? weight_at<T, PROB>(src, first + i) : 0.0;
-      acc += x;
+      if (j >= per || l * per + j >= len) x[j] = 0.0;
+      acc += x[j];
       p[j] = acc;
-      some |= x > 0.0 ? 1u << j : 0u;
+      some[j] = x[j] > 0.0;
     }
-    nz = mask16(some != 0);
-    if (nz || k == 0 || !(r > 0.0)) break;
-    run = sum_before(--k);
+    nz = mask16(some[0] || some[1] || some[2] || some[3]);
+  };
+  read_weights();
+  while (__any(!nz && k > 0 && r > 0.0)) {  // an empty stretch: the one before
+    if (!nz && k > 0 && r > 0.0) --k;
+    read_weights();
   }
-  const uint32_t take = r > 0.0 ? some : 0xfu;
+  const bool all = !(r > 0.0);
   const double excl = scan16(acc, l) - acc;
   int hit = -1;
 #pragma unroll
   for (int j = 3; j >= 0; --j) {
     const int i = l * per + j;
-    if (j < per && i < len && run + (excl + p[j]) >= r && (take >> j & 1u)) hit = i;
+    if (j < per && i < len && (some[j] || all) && run + (excl + p[j]) >= r) hit = i;
   }
   m = mask16(hit >= 0);
-  const int lastnz = l * per + 31 - __clz(some);
+  const int lastnz = l * per + (some[3] ? 3 : some[2] ? 2 : some[1] ? 1 : 0);
   const int from = m ? __ffs(m) - 1 : nz ? 31 - __clz(nz) : 0;
   const int found = __shfl(m ? hit : nz ? lastnz : 0, from, 16);
   if (live && l == 0) out[b * shots + s] = (lo << cl) + ((int64_t)k << sl) + found;
