@@ -499,7 +499,7 @@ __device__ __forceinline__ void fwd_tile(const TilePassArg& A, const uint32_t* _
 // and 160 -> 76 us adjoint (one wave per SIMD: bound by the issue of one
 // wave's instructions, about 8 per gate's multiply-add); 33 x 17 qubits, 8
 // layers 492 -> 259 us forward (5 passes) and 1484 -> 590 us adjoint (8 -> 5
-// passes), 2.2 TB/s and VALU-bound.
+// passes), 0.50 and 0.70 of VALU issue, 1.1 TB/s.
 template <typename T, bool FULL>
 __global__ void __launch_bounds__(sizeof(T) == 4 ? 1024 : 512) k_tile_fwd(
     TilePassArg A, const uint32_t* __restrict__ blob, const int32_t* __restrict__ msrc,
