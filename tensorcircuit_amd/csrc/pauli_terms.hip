@@ -25,6 +25,7 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "regops.h"
 
 namespace tcm {
 
@@ -33,13 +34,6 @@ namespace {
 __device__ __forceinline__ uint32_t first_lane(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ double with_sign(double x, uint32_t odd) {
   return __hiloint2double(__double2hiint(x) ^ (int)(odd << 31), __double2loint(x));
-}
-
-template <int CTRL>
-__device__ __forceinline__ double row_shr(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
 }
 
 constexpr int kRow = 66;  // a string's 64 lane values, padded off its banks
@@ -57,10 +51,10 @@ struct TermSink {
     const double* r = buf + q * kRow + (lane & 15) * 4;
     double x = (r[0] + r[1]) + (r[2] + r[3]);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    x += row_shr<0x111>(x);
-    x += row_shr<0x112>(x);
-    x += row_shr<0x114>(x);
-    x += row_shr<0x118>(x);
+    x += dpp_shr<0x111>(x);
+    x += dpp_shr<0x112>(x);
+    x += dpp_shr<0x114>(x);
+    x += dpp_shr<0x118>(x);
     if ((lane & 15) == 15 && first + q < cnt) acc[(first + q) * nw + wv] += x;
   }
   __device__ __forceinline__ void push(double x) {

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "kernels.h"
+#include "regops.h"
 
 namespace tcm {
 
@@ -29,12 +30,6 @@ __device__ __forceinline__ float flip_sign(float x, uint32_t odd) {
 }
 __device__ __forceinline__ double flip_sign(double x, uint32_t odd) {
   return __hiloint2double(__double2hiint(x) ^ (int)(odd << 31), __double2loint(x));
-}
-
-// tile position x -> state offset from the block base (the L low tile bits
-// are contiguous; linear over disjoint bit sets)
-__device__ __forceinline__ uint32_t run_dep(const uint32_t* __restrict__ ro, int L, uint32_t x) {
-  return ro[x >> L] + (x & ((1u << L) - 1));
 }
 
 // (a, b) summed over the block in fp64, valid in thread 0

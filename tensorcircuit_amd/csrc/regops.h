@@ -1,6 +1,7 @@
 // Gates and gradient generators on 2^R amplitudes held in registers, shared by
 // the per-gate kernels (kernels.hip) and the table-driven tile passes
-// (tile_pass.hip).
+// (tile_pass.hip), and the tile offsets and row sums that the Pauli kernels use
+// as well.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -27,6 +28,12 @@ __device__ __forceinline__ T recj(A2<T> a, A2<T> b) { return a.x * b.x + a.y * b
 template <typename T>
 __device__ __forceinline__ const T* mptr(int moff, const T* mt, const T* ct) {
   return moff >= 0 ? mt + moff : ct + (-moff - 1);
+}
+
+// state offset of tile position x from its block's base: the L low tile bits
+// are contiguous, the others' runs are at ro (linear over disjoint bit sets)
+__device__ __forceinline__ uint32_t run_dep(const uint32_t* __restrict__ ro, int L, uint32_t x) {
+  return ro[x >> L] + (x & ((1u << L) - 1));
 }
 
 // one DPP row-shift of a double (lanes without a source read 0)

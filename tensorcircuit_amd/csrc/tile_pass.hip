@@ -32,12 +32,6 @@ constexpr uint32_t kPermNone = 0x08421u;
 
 __device__ __forceinline__ uint32_t uni(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// state offset of tile position x from the block base (linear over disjoint
-// bit sets)
-__device__ __forceinline__ uint32_t run_dep(const uint32_t* ro, int L, uint32_t x) {
-  return ro[x >> L] + (x & ((1u << L) - 1));
-}
-
 // block index -> the index bits outside the tile
 __device__ __forceinline__ uint64_t deposit(uint64_t blk, uint64_t m, int nbl) {
   uint64_t base = 0;
