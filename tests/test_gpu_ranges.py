@@ -212,3 +212,21 @@ def test_pauli_strings_by_tiles_and_without(gpu, n, T, batch, letters):
         y0 = ham.apply_terms(buf[1:], a[:1])[0]
         assert float((y[0] - y0).abs().max()) <= 4 * (unit + T * 2.0**-53) * float(
             (a[0].abs() * torch.as_tensor(np.abs(w)).to(gpu)).sum() * st[0].abs().max())
+
+
+@pytest.mark.parametrize("n", [13, 14, 16])
+@pytest.mark.parametrize("dtype,bits", [("complex64", 14), ("complex128", 13)])
+def test_widest_adjoint_tiles(gpu, n, dtype, bits):
+    """128 KiB tiles, the widest that a CU's LDS holds, against 32 KiB ones."""
+    from tensorcircuit_amd import _lib, engine
+
+    kinds = (_lib.G_RX, _lib.G_RZ, _lib.G_RY, _lib.G_RZZ)
+    specs = [engine.GateSpec(kinds[g % 4], (g % n, (g + 3) % n)[: 2 if g % 4 == 3 else 1], g, 0.0, 1.0, None)
+             for g in range(6 * n)]
+    ham = engine.PauliSum(n, [[3, 3] + [0] * (n - 2), [0] * (n - 1) + [1]], [0.7, 1.1])
+    p = torch.randn(2, len(specs), dtype=torch.float32 if dtype == "complex64" else torch.float64, device=gpu)
+    (e, g), (e2, g2) = (engine.Program(n, specs, len(specs), fuse=1, adj_tile_bits=b).energy_grad(p, ham, 2, dtype)
+                        for b in (bits, 11))
+    # 6 n gates on states of norm one, each rounded a few times per amplitude
+    unit = 2.0**-24 if dtype == "complex64" else 2.0**-53
+    assert float((e - e2).abs().max()) <= 16 * len(specs) * unit and float((g - g2).abs().max()) <= 16 * len(specs) * unit
