@@ -870,20 +870,21 @@ __device__ __forceinline__ double strided_sum(const double* __restrict__ part, i
   return (a0 + a1) + (a2 + a3);
 }
 
-// out[b * ncomp + c] = sum_s part[b * bstride + s * ncomp + c]; one block per
-// b, bound by the loads that it keeps in flight (49k pairs: 86 us with 256
+// out[b * ncomp + c] = sum_s part[b * bstride + s * ncomp + c]; a block per b
+// (several in turn for very many), bound by the loads that it keeps in flight (49k pairs: 86 us with 256
 // threads and one load each, 20 us with 1024 and four), or by the blocks where
 // there are few per b (60000 states of 2 qubits and 3 pairs, with the launches
 // that make them: 155 us with 256 threads each, 131 us with 64)
 __global__ void __launch_bounds__(1024) k_sum_slots(const double* __restrict__ part, int64_t bstride, int64_t nslots,
-                                                    int ncomp, double* __restrict__ out) {
-  const int64_t b = blockIdx.x;
-  double a = strided_sum(part + b * bstride, nslots, ncomp, threadIdx.x, blockDim.x), c = 0.0;
-  if (ncomp > 1) c = strided_sum(part + b * bstride + 1, nslots, ncomp, threadIdx.x, blockDim.x);
-  block_sum2(a, c);
-  if (threadIdx.x == 0) {
-    out[b * ncomp] = a;
-    if (ncomp > 1) out[b * ncomp + 1] = c;
+                                                    int ncomp, double* __restrict__ out, int64_t batch) {
+  for (int64_t b = blockIdx.x; b < batch; b += gridDim.x) {
+    double a = strided_sum(part + b * bstride, nslots, ncomp, threadIdx.x, blockDim.x), c = 0.0;
+    if (ncomp > 1) c = strided_sum(part + b * bstride + 1, nslots, ncomp, threadIdx.x, blockDim.x);
+    block_sum2(a, c);
+    if (threadIdx.x == 0) {
+      out[b * ncomp] = a;
+      if (ncomp > 1) out[b * ncomp + 1] = c;
+    }
   }
 }
 
@@ -1217,7 +1218,9 @@ void launch_inner(const void* a, const void* c, int n, int64_t batch, int nblk, 
 
 void launch_sum_slots(const double* part, int64_t bstride, int64_t nslots, int ncomp, double* out, int64_t batch,
                       hipStream_t st) {
-  hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)batch), dim3(nslots > 1024 ? 1024 : nslots > 64 ? 256 : 64), 0, st, part, bstride, nslots, ncomp, out);
+  const int threads = nslots > 1024 ? 1024 : nslots > 64 ? 256 : 64;
+  hipLaunchKernelGGL(k_sum_slots, dim3((unsigned)std::min(batch, kMaxLaunchThreads / threads)), dim3(threads), 0, st,
+                     part, bstride, nslots, ncomp, out, batch);
 }
 
 void launch_reduce_gop(const double* part, int64_t pstride, int64_t nslots, const int32_t* gop_list, int gop_single,

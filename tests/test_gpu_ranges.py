@@ -230,3 +230,18 @@ def test_widest_adjoint_tiles(gpu, n, dtype, bits):
     # 6 n gates on states of norm one, each rounded a few times per amplitude
     unit = 2.0**-24 if dtype == "complex64" else 2.0**-53
     assert float((e - e2).abs().max()) <= 16 * len(specs) * unit and float((g - g2).abs().max()) <= 16 * len(specs) * unit
+
+
+def test_sums_of_many_states(gpu):
+    """2^26 inner products and energies of one-qubit states: a wave each."""
+    from tensorcircuit_amd import engine
+
+    B = (1 << 26) + 3
+    st = torch.zeros(B, 2, dtype=torch.complex64, device=gpu)
+    st[:, 1] = 1.0
+    st[-1, 1] = 3.0
+    got = engine.inner(st, st, 1).real
+    assert bool((got[:-1] == 1.0).all()) and float(got[-1]) == 9.0
+    del got
+    e = engine.PauliSum(1, [[3], [1]], [2.0, 1.0], jit=0).expect(st).real
+    assert bool((e[:-1] == -2.0).all()) and float(e[-1]) == -18.0
